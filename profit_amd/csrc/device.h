@@ -124,19 +124,20 @@ struct WorkQueue {
 	// written by the forward walk of a gradient evaluation (null otherwise)
 	float *ljac, *hjac;
 	// the light entries whose root node has a cell to refine (indices into
-	// the family's light list, in the same segments): the root pass, one lane
-	// per entry, hands these to the wavefront walker
+	// the family's light list, in the same segments), which the root pass
+	// hands to the tree walk: small trees from a segment's front, big ones
+	// (kBigTree) from its back
 	int *deep;
 };
 constexpr int kJacStride = 12;
-// count[1]: length of the heavy list; then a (heavy, deep) pair of hand-out
-// counters per walker launch (one per profile family); the length of each
-// family's light list; the root pass's hand-out counter per family; the
-// length of each family's deep list (count[0] is not used)
+// count[0]: trees that overflowed the tree walk's stack; count[1]: length of
+// the heavy list; then a (heavy, deep) pair of hand-out counters per mask walk
+// (one per profile family); the length of each family's light list, of its big
+// trees' list and of its other deep entries' list
 constexpr int kQueueCounters = 32;
 __host__ __device__ constexpr int fwd_counter(int type) { return 2 + 2 * type; }
 __host__ __device__ constexpr int light_count(int type) { return 14 + type; }
-__host__ __device__ constexpr int root_counter(int type) { return 20 + type; }
+__host__ __device__ constexpr int big_count(int type) { return 20 + type; }
 __host__ __device__ constexpr int deep_count(int type) { return 26 + type; }
 
 

@@ -743,13 +743,24 @@ WorkQueue Engine::work_queue()
 	return q;
 }
 
-// whether the last evaluation's work lists fitted
+// whether the last evaluation's trees fitted the tree walk's stack
+bool Engine::trees_ok() const { return h_qcount_.as<int>()[0] == 0; }
+
+// whether the last evaluation's work lists and trees fitted
 bool Engine::queue_ok() const
 {
 	const int *q = h_qcount_.as<int>();
+	if (!trees_ok()) return false;
 	for (int f = 0; f < kFamilies; ++f)
 		if (q[light_count(f)] > lcap_[f]) return false;
 	return q[1] <= hcap_;
+}
+
+// prepares a second run of an evaluation whose work lists or trees did not fit
+void Engine::retry_evaluation()
+{
+	if (!trees_ok()) mask_walk_ = true;
+	grow_queue();
 }
 
 // grows the work lists to what the last evaluation needed (drops the graphs)
@@ -1124,7 +1135,7 @@ void Engine::launch_walkers_fwd(int split, bool jac, hipStream_t st)
 	for (int t = 0; t < 6; ++t)
 		if ((radial_types_ >> t) & 1u)
 			hip_check(launch_subsample_fwd(t, subsample_blocks_, d_gals_.as<GalaxyDev>(), d_insts_.as<InstDev>(),
-			                               d_comps_.as<Comp>(), work_queue(), split, jac, st),
+			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, st),
 			          "subsample");
 }
 
@@ -1132,9 +1143,10 @@ void Engine::run(bool grad, bool use_graph)
 {
 	hip_check(hipSetDevice(device_), "hipSetDevice");
 	if (timing_) use_graph = false;  // events between kernels need the eager sequence
+	mask_walk_ = false;
 	for (int attempt = 0; attempt < 4; ++attempt) {
 		const int gi = grad ? 1 : 0;
-		if (use_graph) {
+		if (use_graph && !mask_walk_) {
 			if (!graph_exec_[gi]) {
 				// first call runs eagerly (sets kernel attributes), later calls replay a graph
 				record(grad);
@@ -1186,7 +1198,7 @@ void Engine::run(bool grad, bool use_graph)
 			stats_.evaluations += 1;
 			return;
 		}
-		grow_queue();  // drops the graphs; run again
+		retry_evaluation();
 	}
 	throw std::runtime_error("sub-pixel work queue kept overflowing");
 }
@@ -1278,6 +1290,7 @@ void Engine::model_images(const ProfileParams *params, float *out)
 	hipStream_t st = stream_;
 	const GalaxyDev *gals = d_gals_.as<GalaxyDev>();
 	const InstDev *insts = d_insts_.as<InstDev>();
+	mask_walk_ = false;
 	for (int attempt = 0; attempt < 4; ++attempt) {
 		hip_check(hipMemcpyAsync(d_params_.as<ProfileParams>(), h_params_.as<ProfileParams>(), nc * sizeof(ProfileParams),
 		                         hipMemcpyHostToDevice, st),
@@ -1297,7 +1310,7 @@ void Engine::model_images(const ProfileParams *params, float *out)
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
 		if (queue_ok()) break;
-		grow_queue();
+		retry_evaluation();
 	}
 	size_t off = 0;
 	for (int i = 0; i < n; ++i) {
@@ -1323,6 +1336,7 @@ void Engine::model_canvas(const ProfileParams *params, float *out, float *out_di
 	const InstDev *insts = d_insts_.as<InstDev>();
 	const GalaxyDev &g = gal_host_[inst_galaxy_[0]];
 	const bool conv = g.has_psf != 0;
+	mask_walk_ = false;
 	for (int attempt = 0; attempt < 4; ++attempt) {
 		hip_check(hipMemcpyAsync(d_params_.as<ProfileParams>(), h_params_.as<ProfileParams>(), nc * sizeof(ProfileParams),
 		                         hipMemcpyHostToDevice, st),
@@ -1347,7 +1361,7 @@ void Engine::model_canvas(const ProfileParams *params, float *out, float *out_di
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
 		if (queue_ok()) break;
-		grow_queue();
+		retry_evaluation();
 	}
 	const size_t nd = (size_t)g.DW * g.DH;
 	if (out_direct) {

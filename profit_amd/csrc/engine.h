@@ -29,9 +29,10 @@ int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *tile_o
 // the forward walker and the adjoint render, one launch per radial family
 // (and per sum precision in the adjoint render: 1 = FP64 per-thread sums,
 // steep cores only).  jac: the forward walk also writes each entry's Jacobian
-// (wq.ljac, wq.hjac), which launch_adj_queue weighs by G(q).
+// (wq.ljac, wq.hjac), which launch_adj_queue weighs by G(q).  mask: the trees
+// by the mask walk (after a tree overflowed the tree walk's stack).
 int launch_subsample_fwd(int type, int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
-                         WorkQueue wq, int split, bool jac, hipStream_t st);
+                         WorkQueue wq, int split, bool jac, bool mask, hipStream_t st);
 int launch_adj_queue(int type, int nblocks, const InstDev *insts, const Comp *comps, WorkQueue wq, double *grad_acc,
                      hipStream_t st);
 int launch_subsample_nodes(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
@@ -305,6 +306,11 @@ class Engine {
 	// radial families present (bit t) and the adjoint's (family, precision)
 	// keys present (bit 2t + prec), which decide the walker launches
 	unsigned radial_types_ = 0, grad_keys_ = 0;
+	// trees by the mask walk: set while an evaluation runs again because a
+	// tree overflowed the tree walk's stack
+	bool mask_walk_ = false;
+	bool trees_ok() const;
+	void retry_evaluation();
 	void launch_walkers_fwd(int split, bool jac, hipStream_t st);
 	bool sync_aux_flags(bool enable);
 	std::vector<int> ct_off_, at_off_, ag_off_;

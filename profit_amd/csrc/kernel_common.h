@@ -394,9 +394,11 @@ __device__ __forceinline__ void walk_pixel(const Comp &c, WalkLevel *L, int lane
 	}
 }
 
-// One wavefront per queued pixel of a TYPE component: adds flux_scale * value
-// to the canvas (or the aux canvas, or the FP64 canvas) and, with kJac, writes
-// the entry's Jacobian and value to wq.ljac / hjac for k_adj_queue.
+// One wavefront per queued pixel of a TYPE component (the walk of last resort,
+// for evaluations with a tree that overflows k_subsample_tree's stack: its
+// memory is one mask per level): adds flux_scale * value to the canvas (or the
+// aux canvas, or the FP64 canvas) and, with kJac, writes the entry's Jacobian
+// and value to wq.ljac / hjac for k_adj_queue.
 // `counter`: the pair of hand-out counters of this launch (heavy, light).
 // Held to the registers of four waves per SIMD (three for the Sersic, Moffat
 // and broken-exponential walks with kJac, whose code needs more).
@@ -524,83 +526,335 @@ __global__ __launch_bounds__(256, kJac && (TYPE == SERSIC || TYPE == MOFFAT || T
 	}
 }
 
-// The root pass of the sub-sampled pixels, one lane per light entry of a
-// TYPE family: the lane evaluates its pixel's root cells one after another
-// with the walker's cell step and, when none is to be refined (most pixels:
-// 98% on a 400x400 bulge+disk), adds the value to the canvas and, with kJac,
-// writes the entry's Jacobian and value itself, with no exchange between
-// lanes.  An entry with a cell to refine goes to the family's deep list,
-// whose trees the wavefront walker (k_subsample) walks from the root.
-// entries from which the root pass works a lane per entry: 2^17, two
-// wavefronts of 64 entries for each SIMD of the chip
-constexpr int kRootMinEntries = 1 << 17;
+// The root pass of the sub-sampled pixels, one group of 2^k lanes per light
+// entry of a TYPE family: the lanes share the pixel's root cells, and when none
+// is to be refined (most pixels: 98% on a 400x400 bulge+disk) the group adds
+// the value to the canvas and, with kJac, writes the entry's Jacobian and
+// value.  An entry with a cell to refine goes to the family's deep list: to its
+// front, or, with `split_big` and from kBigTree refined cells on, to its back;
+// k_subsample_tree walks those trees from the root.
+//
+// Bound by VALU issue on long lists and by latency on short ones, so the group
+// is as wide as the list leaves room for in kRootLanes lanes (four wavefronts
+// per SIMD): one lane per entry from 131,073 entries (no exchange, 0.63 ms for
+// the 1.3 M of a batch of 1024 bulge+disk images), a whole wavefront below
+// 4,097.  Entries are dealt out by index: asking a counter cost 11.6 ns per
+// wavefront (95 us for 8,192 of them, also with nothing to do).
+constexpr int kRootLanes = 1 << 18;
+constexpr int kBigTree = 8;
 
 template <int TYPE, bool kJac>
 __global__ __launch_bounds__(256) void k_subsample_root(const GalaxyDev *__restrict__ gals,
                                                          const InstDev *__restrict__ insts,
-                                                         const Comp *__restrict__ comps, WorkQueue wq, int split)
+                                                         const Comp *__restrict__ comps, WorkQueue wq, int split,
+                                                         int split_big)
 {
+	constexpr int kSlots = G_S0 + n_shape(TYPE);
 	const int lane = threadIdx.x & 63;
-	const int lb = wq.lbase[TYPE];
-	const int nl = min(wq.count[light_count(TYPE)], wq.lbase[TYPE + 1] - lb);
-	// a lane per entry pays off when the entries fill the GPU; a shorter list
-	// (a single image, say) goes whole to the walker, whose wavefronts share
-	// each pixel's cells and so finish sooner
-	const bool lanes = nl >= kRootMinEntries;
-	for (;;) {
-		int base = 0;
-		if (lane == 0) base = atomicAdd(&wq.count[root_counter(TYPE)], 64);
-		base = __shfl(base, 0);
-		if (base >= nl) break;
-		const int e = base + lane;
-		bool deep = false;
+	const int lb = wq.lbase[TYPE], cap = wq.lbase[TYPE + 1] - lb;
+	const int nl = min(wq.count[light_count(TYPE)], cap);
+	int lg = 0;
+	while (lg < 6 && ((long)nl << (lg + 1)) <= kRootLanes) ++lg;
+	const int grp = 1 << lg, sub = lane & (grp - 1);
+	const long gtid = (long)blockIdx.x * blockDim.x + threadIdx.x, sweep = (long)gridDim.x * blockDim.x;
+	// the loop's bound is the wavefront's first entry: uniform
+	for (long t = gtid; ((t - lane) >> lg) < nl; t += sweep) {
+		const int e = (int)min(t >> lg, (long)nl);
+		int nref = 0;
+		double sum = 0;
+		float gj[NGRAD];
+#pragma unroll
+		for (int s = 0; s < NGRAD; ++s) gj[s] = 0.f;
+		QEntry q{-1, 0};
+		bool mine = false;
 		if (e < nl) {
-			const QEntry q = wq.light[lb + e];
+			q = wq.light[lb + e];
 			const Comp &c = comps[q.comp];
-			const InstDev &I = insts[c.instance];
-			const GalaxyDev &g = gals[I.galaxy];
+			const GalaxyDev &g = gals[insts[c.instance].galaxy];
 			const int i = q.pix % g.DW, j = q.pix / g.DW;
 			const double hx = g.sx / 2., hy = g.sy / 2.;
 			const double y = hy + j * g.sx;
 			const double x = hx + i * g.sy;
+			mine = c.type == TYPE;
 			// centre-rule pixels belong to the heavy list: any found here go
-			// to the walker, which applies the rule
-			deep = !lanes || centre_pixel(c, x, y);
-			if (c.type == TYPE && !deep) {
+			// to the tree walk, which applies the rule
+			if (mine && centre_pixel(c, x, y)) nref = kBigTree;
+			else if (mine) {
 				const int res = c.res, ncell = res * res;
 				const bool recurse = res > 1 && c.maxrec > 0;
 				const bool fuse = kJac && TYPE == SERSIC && !c.boxy && !c.grad_box;
 				const Node n = make_node(c, x - hx, x + hx, y - hy, y + hy, res);
 				const double weight = kInvCells[res];
 				const bool fp64 = g.render_fp64 != 0;
-				double sum = 0;
-				float gj[NGRAD];
-#pragma unroll
-				for (int s = 0; s < NGRAD; ++s) gj[s] = 0.f;
-				for (int cell = 0; cell < ncell && !deep; ++cell)
-					deep = cell_step<TYPE, kJac>(c, n, cell, recurse, fp64, fuse, weight, sum, gj);
-				if (!deep) {
-					const bool to_aux = split && !c.convolve;
-					if (g.canvas64 && !to_aux) atomicAdd(&I.canvas64[q.pix], c.flux_scale * sum);
-					else atomicAdd(&(to_aux ? I.aux : I.canvas)[q.pix], (float)(c.flux_scale * sum));
-					if (kJac) {
-						float *J = wq.ljac + (long)(lb + e) * kJacStride;
-#pragma unroll
-						for (int s = 0; s < G_S0 + n_shape(TYPE); ++s) J[s] = gj[s];
-						J[kJacStride - 1] = (float)sum;
-					}
-				}
+				for (int cell = sub; cell < ncell; cell += grp)
+					nref += cell_step<TYPE, kJac>(c, n, cell, recurse, fp64, fuse, weight, sum, gj) ? 1 : 0;
 			}
 		}
-		// the deep entries appended, one atomic per wave
-		const unsigned long long m = __ballot(deep);
-		if (m) {
+		double gd[kSlots];
+		if (kJac) {
+#pragma unroll
+			for (int s = 0; s < kSlots; ++s) gd[s] = (double)gj[s];
+		}
+		for (int o = grp >> 1; o > 0; o >>= 1) {
+			nref += __shfl_xor(nref, o);
+			sum += __shfl_xor(sum, o);
+			if (kJac) {
+#pragma unroll
+				for (int s = 0; s < kSlots; ++s) gd[s] += __shfl_xor(gd[s], o);
+			}
+		}
+		const bool lead = mine && sub == 0;
+		if (lead && nref == 0) {
+			const Comp &c = comps[q.comp];
+			const InstDev &I = insts[c.instance];
+			const bool to_aux = split && !c.convolve;
+			if (gals[I.galaxy].canvas64 && !to_aux) atomicAdd(&I.canvas64[q.pix], c.flux_scale * sum);
+			else atomicAdd(&(to_aux ? I.aux : I.canvas)[q.pix], (float)(c.flux_scale * sum));
+			if (kJac) {
+				float *J = wq.ljac + (long)(lb + e) * kJacStride;
+#pragma unroll
+				for (int s = 0; s < kSlots; ++s) J[s] = (float)gd[s];
+				J[kJacStride - 1] = (float)sum;
+			}
+		}
+		// the deep entries appended, one atomic per wavefront and list
+		const bool big = lead && split_big && nref >= kBigTree, deep = lead && nref > 0 && !big;
+#pragma unroll
+		for (int k = 0; k < 2; ++k) {
+			const unsigned long long m = __ballot(k ? big : deep);
+			if (!m) continue;
 			const int leader = __ffsll((long long)m) - 1;
 			int at = 0;
-			if (lane == leader) at = atomicAdd(&wq.count[deep_count(TYPE)], __popcll(m));
-			at = __shfl(at, leader);
-			if (deep) wq.deep[lb + at + __popcll(m & ((1ull << lane) - 1ull))] = e;
+			if (lane == leader) at = atomicAdd(&wq.count[k ? big_count(TYPE) : deep_count(TYPE)], __popcll(m));
+			at = __shfl(at, leader) + __popcll(m & ((1ull << lane) - 1ull));
+			if (k ? big : deep) wq.deep[lb + (k ? cap - 1 - at : at)] = e;
 		}
+	}
+}
+
+// ------------------------------------------------------------------ trees
+
+// The pending nodes of the trees a block walks, in LDS: wavefront w's quarter
+// holds kTreeQuarter of them (its own stack while each wavefront walks a tree
+// of its own; a quarter of the block's while the block walks one together).
+constexpr int kTreeQuarter = 256;
+struct TreeStack {
+	struct Quarter {
+		double x0[kTreeQuarter], x1[kTreeQuarter], y0[kTreeQuarter], y1[kTreeQuarter], weight[kTreeQuarter];
+		uint8_t level[kTreeQuarter];
+	} q[4];
+	int count[2][4];  // refined cells per wavefront of a round, double-buffered
+};
+
+// Walks the recursion tree of one pixel of a TYPE profile with T threads (a
+// wavefront, T = 64, or a block of four, T = 256), starting from stack slot
+// `base` (T = 64: the wavefront's quarter).  A round takes as many pending
+// nodes off the stack as T threads have cells for, one cell per thread (a node
+// of more cells alone, its cells T at a time); a cell to be refined pushes its
+// own FP64 node bounds (libprofit's additions).  Every thread returns its share
+// of sum_s weight_s f(s) in `sum` and, with kJac, of the weighted FP32
+// derivatives in gj.  Returns false when the stack (cap nodes) would overflow:
+// the sums are then void.
+//
+// `top`, `n` and `total` are equal on all T threads, so all take the same
+// barriers; each round removes a node and a node's children lie one level
+// deeper (at most maxrec), so the rounds end.
+template <int TYPE, bool kJac, int T>
+__device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack &S, int base, int tid, double x0, double x1,
+                                          double y0, double y1, int res, int maxrec, bool fp64, double &sum, float *gj)
+{
+	constexpr int cap = T == 64 ? kTreeQuarter : 4 * kTreeQuarter;
+	const bool fuse = kJac && TYPE == SERSIC && !c.boxy && !c.grad_box;
+	const int ncell = res * res, wv = tid >> 6, lane = tid & 63;
+	const double inv_cells = kInvCells[res];
+	// the thread's node of a round and its first cell
+	const int per = ncell >= T ? 1 : T / ncell;
+	const int slot = ncell >= T ? 0 : tid / ncell;
+	const int cell0 = tid - slot * ncell;
+	auto put = [&](int at, double a, double b, double d, double e, double w, int level) {
+		TreeStack::Quarter &q = S.q[(base + at) / kTreeQuarter];
+		const int k = (base + at) % kTreeQuarter;
+		q.x0[k] = a;
+		q.x1[k] = b;
+		q.y0[k] = d;
+		q.y1[k] = e;
+		q.weight[k] = w;
+		q.level[k] = (uint8_t)level;
+	};
+	auto sync = [&]() {
+		if constexpr (T == 64) {
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+		}
+		else {
+			__syncthreads();
+		}
+	};
+	if (tid == 0) put(0, x0, x1, y0, y1, inv_cells, 0);
+	sync();
+	int top = 1, buf = 0;
+	while (top > 0) {
+		const int n = min(per, top);
+		const bool on = slot < n;
+		const int r = base + top - 1 - (on ? slot : 0);
+		const TreeStack::Quarter &Q = S.q[r / kTreeQuarter];
+		const int k = r % kTreeQuarter;
+		const Node node = make_node(c, Q.x0[k], Q.x1[k], Q.y0[k], Q.y1[k], res);
+		const double weight = Q.weight[k];
+		const int level = Q.level[k];
+		const bool recurse = res > 1 && level < maxrec;
+		top -= n;
+		bool pushed = false;
+		for (int at = 0; at < ncell; at += T) {
+			const int cell = cell0 + at;
+			const bool fail = on && cell < ncell && cell_step<TYPE, kJac>(c, node, cell, recurse, fp64, fuse, weight, sum, gj);
+			const unsigned long long m = __ballot(fail);
+			int off = __popcll(m & ((1ull << lane) - 1ull)), total = __popcll(m);
+			if constexpr (T == 256) {
+				// every thread has read its node before a push may overwrite it
+				if (lane == 0) S.count[buf][wv] = total;
+				__syncthreads();
+				total = 0;
+				for (int w = 0; w < 4; ++w) {
+					const int v = S.count[buf][w];
+					off += w < wv ? v : 0;
+					total += v;
+				}
+				buf ^= 1;
+			}
+			if (total == 0) continue;
+			if (top + total > cap) return false;
+			if (fail) {
+				const double hx = (node.x1 - node.x0) / res / 2., hy = (node.y1 - node.y0) / res / 2.;
+				const int ci = (int)(((float)cell + 0.5f) * node.inv_res), cj = cell - ci * res;
+				const double cx = cell_centre(node.x0, hx, ci), cy = cell_centre(node.y0, hy, cj);
+				put(top + off, cx - hx, cx + hx, cy - hy, cy + hy, weight * inv_cells, level + 1);
+			}
+			top += total;
+			pushed = true;
+		}
+		if (pushed) sync();
+	}
+	return true;
+}
+
+// The trees of a TYPE family: the centre pixels (heavy list, Sersic) and the
+// entries with kBigTree or more refined root cells (the back of the deep list),
+// a block each; then the other deep entries, a wavefront each.  Adds flux_scale
+// * value to the canvas (or the aux canvas, or the FP64 canvas) and, with kJac,
+// writes the entry's Jacobian and value.  Entries are dealt out by index; an
+// overflowing tree is counted in count[0] and the evaluation runs again with
+// the mask walk (k_subsample), whose memory does not depend on the tree.
+//
+// A centre tree (res 8, depth 10: 160 nodes, 16 a level) is a chain of levels:
+// one wavefront walking its nodes in turn took 220 to 300 us, whatever the
+// batch; four share each level.
+template <int TYPE, bool kJac>
+__global__ __launch_bounds__(256, 3) void k_subsample_tree(const GalaxyDev *__restrict__ gals,
+                                                           const InstDev *__restrict__ insts,
+                                                           const Comp *__restrict__ comps, WorkQueue wq, int split)
+{
+	constexpr int kSlots = G_S0 + n_shape(TYPE), kJacPitch = 68;
+	__shared__ __align__(16) TreeStack S;
+	__shared__ double red[4][16];
+	static_assert(kSlots < kJacStride && kSlots + 1 <= 16, "Jacobian slots and the value");
+	static_assert(sizeof(float) * kSlots * kJacPitch <= sizeof(TreeStack::Quarter), "a wavefront's rows fit its quarter");
+	static_assert(sizeof(TreeStack::Quarter) % 16 == 0, "a wavefront's rows are 16-byte aligned");
+	const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int lb = wq.lbase[TYPE], cap = wq.lbase[TYPE + 1] - lb;
+	const int nd = min(wq.count[deep_count(TYPE)], cap), nb = min(wq.count[big_count(TYPE)], cap);
+	const int nh = TYPE == SERSIC ? min(wq.count[1], wq.hcap) : 0;
+	float gj[NGRAD];
+	double sum;
+	// the thread's sums of its wavefront: lane s < kSlots of the wavefront
+	// returns slot s, lane 15 the value (the wavefront's quarter as scratch:
+	// the walk is over)
+	auto wave_totals = [&]() {
+		float *R = reinterpret_cast<float *>(&S.q[wv]);
+		const double v = wave_sum(sum);
+		double t = 0.0;
+		if constexpr (kJac) {
+#pragma unroll
+			for (int s = 0; s < kSlots; ++s) R[s * kJacPitch + lane] = gj[s];
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+			const int slot = lane & 15, qt = lane >> 4;
+			if (slot < kSlots) {
+				const float4 *row = reinterpret_cast<const float4 *>(R + slot * kJacPitch + qt * 16);
+#pragma unroll
+				for (int k = 0; k < 4; ++k) {
+					const float4 w = row[k];
+					t += ((double)w.x + (double)w.y) + ((double)w.z + (double)w.w);
+				}
+			}
+			t += __shfl_xor(t, 16);
+			t += __shfl_xor(t, 32);
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			__builtin_amdgcn_wave_barrier();
+		}
+		return lane == 15 ? v : t;
+	};
+	auto finish = [&](const QEntry &q, const Comp &c, const InstDev &I, const GalaxyDev &g, bool heavy, int e, double t) {
+		if (kJac) {
+			float *J = (heavy ? wq.hjac : wq.ljac + (long)lb * kJacStride) + (long)e * kJacStride;
+			if (lane < kSlots) J[lane] = (float)t;
+			if (lane == 15) J[kJacStride - 1] = (float)t;
+		}
+		if (lane == 15) {
+			const bool to_aux = split && !c.convolve;
+			if (g.canvas64 && !to_aux) atomicAdd(&I.canvas64[q.pix], c.flux_scale * t);
+			else atomicAdd(&(to_aux ? I.aux : I.canvas)[q.pix], (float)(c.flux_scale * t));
+		}
+	};
+	auto clear = [&]() {
+		sum = 0;
+#pragma unroll
+		for (int s = 0; s < NGRAD; ++s) gj[s] = 0.f;
+	};
+	for (int t = blockIdx.x; t < nh + nb; t += gridDim.x) {
+		const bool heavy = t < nh;
+		const int e = heavy ? t : wq.deep[lb + cap - 1 - (t - nh)];
+		const QEntry q = heavy ? wq.heavy[e] : wq.light[lb + e];
+		const Comp &c = comps[q.comp];
+		if (c.type != TYPE) continue;
+		const InstDev &I = insts[c.instance];
+		const GalaxyDev &g = gals[I.galaxy];
+		const int i = q.pix % g.DW, j = q.pix / g.DW;
+		const double hx = g.sx / 2., hy = g.sy / 2.;
+		const double y = hy + j * g.sx, x = hx + i * g.sy;
+		const bool centre = centre_pixel(c, x, y);
+		clear();
+		const bool ok = walk_tree<TYPE, kJac, 256>(c, S, 0, threadIdx.x, x - hx, x + hx, y - hy, y + hy,
+		                                           centre ? 8 : c.res, centre ? 10 : c.maxrec, g.render_fp64 != 0, sum, gj);
+		if (ok) {
+			const double w = wave_totals();
+			if (lane < 16) red[wv][lane] = w;
+		}
+		else if (threadIdx.x == 0) {
+			atomicAdd(&wq.count[0], 1);
+		}
+		__syncthreads();
+		if (ok && wv == 0) {
+			const int s = lane & 15;
+			finish(q, c, I, g, heavy, e, (red[0][s] + red[1][s]) + (red[2][s] + red[3][s]));
+		}
+		__syncthreads();
+	}
+	for (int t = blockIdx.x * 4 + wv; t < nd; t += gridDim.x * 4) {
+		const int e = wq.deep[lb + t];
+		const QEntry q = wq.light[lb + e];
+		const Comp &c = comps[q.comp];
+		const InstDev &I = insts[c.instance];
+		const GalaxyDev &g = gals[I.galaxy];
+		const int i = q.pix % g.DW, j = q.pix / g.DW;
+		const double hx = g.sx / 2., hy = g.sy / 2.;
+		const double y = hy + j * g.sx, x = hx + i * g.sy;
+		clear();
+		if (walk_tree<TYPE, kJac, 64>(c, S, wv * kTreeQuarter, lane, x - hx, x + hx, y - hy, y + hy, c.res, c.maxrec,
+		                              g.render_fp64 != 0, sum, gj))
+			finish(q, c, I, g, false, e, wave_totals());
+		else if (lane == 0)
+			atomicAdd(&wq.count[0], 1);
 	}
 }
 

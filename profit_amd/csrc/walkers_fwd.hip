@@ -1,40 +1,42 @@
-// Forward recursion walker (libprofit's subsample_pixel, radial.cpp:54-134):
-// a root pass and the wavefront walker, one kernel each per radial profile
-// family; see kernel_common.h.
+// Forward recursion walk (libprofit's subsample_pixel, radial.cpp:54-134): a
+// root pass, the tree walk and the mask walk, one kernel each per radial
+// profile family; see kernel_common.h.
 #include "kernel_common.h"
 
 namespace profit_amd {
 
-// The root pass (one lane per light entry) and then the wavefront walker
-// over the heavy list and the entries the root pass left to it.
-template <int TYPE>
+// The root pass over the light entries, then the tree walk over the heavy list
+// and the entries the root pass left to it (mask: the mask walk instead, one
+// wavefront per tree).  The tree walk's blocks are those that fit at three
+// wavefronts per SIMD.
+template <int TYPE, bool kJac>
 static int fwd_launch(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps, WorkQueue wq,
-                      int split, bool jac, hipStream_t st)
+                      int split, bool mask, hipStream_t st)
 {
-	if (jac) {
-		k_subsample_root<TYPE, true><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, split);
-		k_subsample<TYPE, true><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, fwd_counter(TYPE), split);
-	}
-	else {
-		k_subsample_root<TYPE, false><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, split);
-		k_subsample<TYPE, false><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, fwd_counter(TYPE), split);
-	}
+	k_subsample_root<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, split, mask ? 0 : 1);
+	if (mask) k_subsample<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, fwd_counter(TYPE), split);
+	else k_subsample_tree<TYPE, kJac><<<(nblocks * 3 + 7) / 8, 256, 0, st>>>(gals, insts, comps, wq, split);
 	return (int)hipGetLastError();
 }
 
 int launch_subsample_fwd(int type, int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
-                         WorkQueue wq, int split, bool jac, hipStream_t st)
+                         WorkQueue wq, int split, bool jac, bool mask, hipStream_t st)
 {
 	if (nblocks <= 0) return 0;
+#define PA_FWD(T)                                                                                        \
+	case T:                                                                                              \
+		return jac ? fwd_launch<T, true>(nblocks, gals, insts, comps, wq, split, mask, st)               \
+		           : fwd_launch<T, false>(nblocks, gals, insts, comps, wq, split, mask, st)
 	switch (type) {
-	case SERSIC: return fwd_launch<SERSIC>(nblocks, gals, insts, comps, wq, split, jac, st);
-	case MOFFAT: return fwd_launch<MOFFAT>(nblocks, gals, insts, comps, wq, split, jac, st);
-	case FERRER: return fwd_launch<FERRER>(nblocks, gals, insts, comps, wq, split, jac, st);
-	case KING: return fwd_launch<KING>(nblocks, gals, insts, comps, wq, split, jac, st);
-	case CORESERSIC: return fwd_launch<CORESERSIC>(nblocks, gals, insts, comps, wq, split, jac, st);
-	case BROKENEXP: return fwd_launch<BROKENEXP>(nblocks, gals, insts, comps, wq, split, jac, st);
+		PA_FWD(SERSIC);
+		PA_FWD(MOFFAT);
+		PA_FWD(FERRER);
+		PA_FWD(KING);
+		PA_FWD(CORESERSIC);
+		PA_FWD(BROKENEXP);
 	default: return (int)hipErrorInvalidValue;
 	}
+#undef PA_FWD
 }
 
 }  // namespace profit_amd
