@@ -799,7 +799,7 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 	inst_ncomp_ = inst_ncomp;
 	inst_comp0_.assign(n, 0);
 	ct_off_.assign(n + 1, 0);
-	at_off_.assign(n + 1, 0);
+	n_at_blocks_ = 0;
 	ncomp_total_ = 0;
 	any_t_ = false;
 	all_gauss_ = true;
@@ -819,7 +819,7 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 		ncomp_total_ += inst_ncomp[i];
 		for (int k = 0; k < inst_ncomp[i]; ++k) comp_inst.push_back(i);
 		ct_off_[i + 1] = ct_off_[i] + (g.conv_kind == CK_VALU ? g.n_ctiles : 0);
-		at_off_[i + 1] = at_off_[i] + g.n_atiles;
+		n_at_blocks_ += g.n_atiles;
 		if (g.conv_kind == CK_VALU) kx_max_ = std::max(kx_max_, g.Kx);
 		const size_t ndraw = (size_t)g.DW * g.DH, npix = (size_t)g.W * g.H;
 		DevBuf canvas(ndraw * 4), w(npix * 4), G(ndraw * 4), aux(ndraw * 4), fbuf;
@@ -843,7 +843,6 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 		hneed += (long)inst_ncomp[i] * 4 * std::max(1L, fs * fs);
 	}
 	n_ct_blocks_ = ct_off_[n];
-	n_at_blocks_ = at_off_[n];
 	inst_aux_.assign(n, 0);
 	any_nonradial_ = false;
 	// brute-force model / adjoint tiles and the FFT passes, per instance
@@ -895,8 +894,14 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 		ri1_off_[i + 1] = ri1_off_[i] + (f ? row_blocks(g.DH) : 0);
 	}
 	n_bt_blocks_ = bt_off_[n];
-	// the adjoint render gives each thread about 32 canvas pixels of a component
-	adj_grp_ = std::max(1, 32 / conv_rows_);
+	// the renders give each thread about 32 canvas pixels of a component where
+	// that leaves 2,048 blocks (eight a CU), and fewer otherwise (a block's
+	// first pixel waits for a chain of loads, and the adjoint pays a reduction
+	// per component and block); below 1,024 tiles they split each tile over
+	// several blocks, to two rows a thread at the least
+	adj_grp_ = std::min(std::max(1, 32 / conv_rows_), std::max(1, n_at_blocks_ / 2048));
+	tile_parts_ = 1;
+	while (n_at_blocks_ * tile_parts_ < 1024 && conv_rows_ / tile_parts_ > 2) tile_parts_ *= 2;
 	ag_off_.assign(n + 1, 0);
 	for (int i = 0; i < n; ++i)
 		ag_off_[i + 1] = ag_off_[i] + (gal_host_[inst_galaxy[i]].n_atiles + adj_grp_ - 1) / adj_grp_;
@@ -942,9 +947,7 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 	d_insts_.alloc(std::max(1, n) * sizeof(InstDev));
 	if (n) hip_check(hipMemcpy(d_insts_.as<InstDev>(), insts.data(), n * sizeof(InstDev), hipMemcpyHostToDevice), "insts");
 	d_ct_off_.alloc((n + 1) * sizeof(int));
-	d_at_off_.alloc((n + 1) * sizeof(int));
 	hip_check(hipMemcpy(d_ct_off_.as<int>(), ct_off_.data(), (n + 1) * sizeof(int), hipMemcpyHostToDevice), "off");
-	hip_check(hipMemcpy(d_at_off_.as<int>(), at_off_.data(), (n + 1) * sizeof(int), hipMemcpyHostToDevice), "off");
 	const int nc = std::max(1, ncomp_total_);
 	d_comp_inst_.alloc(nc * sizeof(int));
 	if (ncomp_total_)
@@ -1011,7 +1014,7 @@ void Engine::record(bool grad)
 		if (!any_nonradial_ && radial_types_ == (1u << t)) rtype = t;
 	// the render's FP64 value path only where a pixel can take it
 	const bool fp64 = render_fp64_ || canvas64_ || (radial_types_ & ((1u << KING) | (1u << FERRER)));
-	hip_check(launch_render(gals, insts, d_at_off_.as<int>(), n, n_at_blocks_, d_comps_.as<Comp>(),
+	hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), n, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
 	                        work_queue(), -1, 0, nullptr, st, rtype, fp64),
 	          "render");
 	mark(2);
@@ -1030,7 +1033,7 @@ void Engine::record(bool grad)
 		mark(6);
 		for (int key = 0; key < 12; ++key)
 			if ((grad_keys_ >> key) & 1u)
-				hip_check(launch_adj_render(key >> 1, key & 1, gals, insts, d_ag_off_.as<int>(), n, n_ag_blocks_, adj_grp_,
+				hip_check(launch_adj_render(key >> 1, key & 1, gals, insts, d_ag_off_.as<int>(), n, n_ag_blocks_, adj_grp_, tile_parts_,
 				                            d_comps_.as<Comp>(), d_grad_acc_.as<double>(), st),
 				          "adjoint render");
 		if (any_nonradial_)
@@ -1235,7 +1238,7 @@ void Engine::diagnostics(const ProfileParams *params, int *cls, int *nodes)
 		                       d_err_.as<int>(), nc, st),
 		          "setup");
 		hip_check(launch_zero_i(d_qcount_.as<int>(), kQueueCounters, st), "zero");
-		hip_check(launch_render(gals, insts, d_at_off_.as<int>(), 1, n_at_blocks_, d_comps_.as<Comp>(),
+		hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), 1, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
 		                        work_queue(), -1, 0, dcls.as<int>(), st),
 		          "render");
 		hip_check(launch_subsample_nodes(subsample_blocks_, gals, insts, d_comps_.as<Comp>(), work_queue(), dnodes.as<int>(), st),
@@ -1299,7 +1302,7 @@ void Engine::model_images(const ProfileParams *params, float *out)
 		                       d_err_.as<int>(), nc, st),
 		          "setup");
 		hip_check(launch_zero_i(d_qcount_.as<int>(), kQueueCounters, st), "zero");
-		hip_check(launch_render(gals, insts, d_at_off_.as<int>(), n, n_at_blocks_, d_comps_.as<Comp>(),
+		hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), n, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
 		                        work_queue(), -1, 0, nullptr, st),
 		          "render");
 		launch_walkers_fwd(0, false, st);
@@ -1346,11 +1349,11 @@ void Engine::model_canvas(const ProfileParams *params, float *out, float *out_di
 		          "setup");
 		hip_check(launch_zero_i(d_qcount_.as<int>(), kQueueCounters, st), "zero");
 		// convolved profiles into the canvas, the others into the aux canvas
-		hip_check(launch_render(gals, insts, d_at_off_.as<int>(), 1, n_at_blocks_, d_comps_.as<Comp>(),
+		hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), 1, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
 		                        work_queue(), conv ? 1 : -1, 0, nullptr, st),
 		          "render");
 		if (conv)
-			hip_check(launch_render(gals, insts, d_at_off_.as<int>(), 1, n_at_blocks_, d_comps_.as<Comp>(),
+			hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), 1, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
 			                        work_queue(), 0, 1, nullptr, st),
 			          "render");
 		launch_walkers_fwd(conv ? 1 : 0, false, st);

@@ -23,7 +23,9 @@ int launch_zero_d(double *p, long n, hipStream_t st);
 int launch_zero_i(int *p, long n, hipStream_t st);
 // fp64: some pixel may take an FP64 value (the FP64 model modes, King or
 // Ferrer components in the batch); false only when none can
-int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *tile_off, int ninst, int nblocks,
+// grp: canvas tiles per block, or parts: blocks per tile (a divisor of the
+// tile's rows per thread); one of them is 1
+int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *grp_off, int ninst, int nblocks, int grp, int parts,
                   const Comp *comps, WorkQueue wq, int filter, int target, int *diag_cls, hipStream_t st, int type = -1,
                   bool fp64 = true);
 // the forward walker and the adjoint render, one launch per radial family
@@ -46,7 +48,7 @@ int launch_adj_nonradial(const GalaxyDev *gals, const InstDev *insts, int ninst,
 int launch_like_t(const GalaxyDev *gals, const InstDev *insts, int ninst, int grad, double *ll, double *gscale,
                   hipStream_t st);
 int launch_adj_render(int type, int prec, const GalaxyDev *gals, const InstDev *insts, const int *grp_off, int ninst,
-                      int nblocks, int grp, const Comp *comps, double *grad_acc, hipStream_t st);
+                      int nblocks, int grp, int parts, const Comp *comps, double *grad_acc, hipStream_t st);
 int launch_grad_finalize(const Comp *comps, const double *gscale, const double *grad_acc, double *grad_out,
                          int ncomp, unsigned slot_mask, hipStream_t st);
 int launch_dilate(const uint8_t *in, uint8_t *tmp, uint8_t *out, int w, int h, int padx, int pady, hipStream_t st);
@@ -313,11 +315,13 @@ class Engine {
 	void retry_evaluation();
 	void launch_walkers_fwd(int split, bool jac, hipStream_t st);
 	bool sync_aux_flags(bool enable);
-	std::vector<int> ct_off_, at_off_, ag_off_;
-	int n_ct_blocks_ = 0, n_at_blocks_ = 0, n_ag_blocks_ = 0;
-	int adj_grp_ = 1;  // canvas tiles per block of the adjoint render
+	std::vector<int> ct_off_, ag_off_;
+	int n_ct_blocks_ = 0, n_ag_blocks_ = 0;
+	int n_at_blocks_ = 0;  // canvas tiles of all instances
+	int adj_grp_ = 1;  // canvas tiles per block of the renders
+	int tile_parts_ = 1;  // blocks per tile of the renders (short tile lists)
 	int kx_max_ = 0;
-	DevBuf d_insts_, d_ct_off_, d_at_off_, d_ag_off_, d_comp_inst_;
+	DevBuf d_insts_, d_ct_off_, d_ag_off_, d_comp_inst_;
 	// the set-up's order of the components (grouped by profile family) and
 	// the types it was formed from
 	DevBuf d_setup_order_;

@@ -42,6 +42,13 @@ __device__ inline double wave_sum(double v)
 	return v;
 }
 
+// A 64-bit value that is the same on every lane, moved to scalar registers.
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long v)
+{
+	const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+	return (unsigned long long)hi << 32 | lo;
+}
+
 // 1 / res^2 and 1 / res for the recursion's resolutions 1 .. 16 (setup
 // rejects higher ones), correctly rounded like the divisions they replace
 static __constant__ double kInvCells[17] = {0.0,        1.0 / 1,   1.0 / 4,   1.0 / 9,   1.0 / 16,  1.0 / 25,
@@ -73,6 +80,61 @@ __device__ __forceinline__ double cell_centre(double lo, double half, int idx)
 	}
 	return v + half;
 }
+
+// The rectangle of pixel centres a canvas tile (64 x 4 rows, at tile
+// coordinates t) spans.
+struct TileRect {
+	double x0, x1, y0, y1;
+};
+
+__device__ __forceinline__ TileRect tile_rect(const GalaxyDev &g, int2 t, int rows)
+{
+	const double hx = g.sx / 2., hy = g.sy / 2.;
+	const int i0 = t.x * kTileW, i1 = min(i0 + kTileW, g.DW) - 1;
+	const int j0 = t.y * 4 * rows, j1 = min(j0 + 4 * rows, g.DH) - 1;
+	return TileRect{hx + i0 * g.sy, hx + i1 * g.sy, hy + j0 * g.sx, hy + j1 * g.sx};
+}
+
+// What a component does on a tile: 0 nothing (every pixel beyond rscale_max),
+// 2 every pixel drawn directly, 1 anything else.  The profile radius is at
+// least the distance from the centre (axrat <= 1) and, being convex, largest
+// at a corner; the margins of 1e-4 are far beyond the FP32 errors here and
+// beyond classify32's band, so a 0 or 2 agrees with every pixel's own class.
+// The render leaves dmask untouched where this is 0, and the adjoint render
+// asks again before it reads dmask: both through this function.
+__device__ __forceinline__ int tile_class(const Comp &c, const TileRect &r)
+{
+	if (!is_radial(c.type)) return 1;
+	const float ax = (float)(r.x0 - c.xc), bx = (float)(r.x1 - c.xc);
+	const float ay = (float)(r.y0 - c.yc), by = (float)(r.y1 - c.yc);
+	const float dx = fmaxf(fmaxf(ax, -bx), 0.f), dy = fmaxf(fmaxf(ay, -by), 0.f);
+	const float near2 = dx * dx + dy * dy;
+	if (c.has_rmax) {
+		const float lim = 1.0001f;
+		const float cq = c.f.cos_ang, sq = c.f.sin_ang, q = c.f.axrat;
+		// half extents of the ellipse of radius rscale_max, squared
+		const float ex2 = c.f.rmax2 * (cq * cq + q * q * sq * sq), ey2 = c.f.rmax2 * (sq * sq + q * q * cq * cq);
+		if (near2 > lim * c.f.rmax2 || dx * dx > lim * ex2 || dy * dy > lim * ey2) return 0;
+	}
+	if (!c.rough && !(near2 > 1.0001f * c.f.rsw2)) return 1;
+	if (c.has_rmax) {
+		float far2 = 0.f;
+#pragma unroll
+		for (int k = 0; k < 4; ++k) {
+			const float x = (k & 1) ? bx : ax, y = (k & 2) ? by : ay;
+			const float xp = x * c.f.cos_ang + y * c.f.sin_ang, yp = -x * c.f.sin_over + y * c.f.cos_over;
+			far2 = fmaxf(far2, xp * xp + yp * yp);
+		}
+		if (!(far2 < 0.9999f * c.f.rmax2)) return 1;
+	}
+	return 2;
+}
+
+// rows whose masks and G an adjoint render thread loads together
+constexpr int kAdjRows = 4;
+// components whose tile classes a block keeps as bit masks (the ones beyond
+// are taken as class 1)
+constexpr int kCullWords = 64;
 
 // d(f)/d slot of one sample in precision T, chain rule to the component
 // slots, accumulated with weight wgt (FP64) into gs; returns f.  TYPE >= 0
@@ -919,26 +981,59 @@ __global__ __launch_bounds__(256) void k_adj_queue(const InstDev *__restrict__ i
 // which FP32 sums do not survive), the flux-scale term applied once per
 // component from sum_q G(q) fs f(q).  A block takes `grp` consecutive canvas
 // tiles of one instance (block offsets per instance in grp_off), so that the
-// per-component reduction and its atomics are paid once per grp tiles.
+// per-component reduction and its atomics are paid once per grp tiles, or one
+// of `parts` parts of a tile (grp = 1).  Components that do nothing on the
+// block's tiles are left out through a bit mask the block forms first.
 // Compiled per profile family TYPE and G64; components of other kinds are
 // left to the launch made for them.
 template <int TYPE, bool G64>
 __global__ __launch_bounds__(256) void k_adj_render(const GalaxyDev *__restrict__ gals,
                                                     const InstDev *__restrict__ insts,
-                                                    const int *__restrict__ grp_off, int ninst, int grp,
+                                                    const int *__restrict__ grp_off, int ninst, int grp, int parts,
                                                     const Comp *__restrict__ comps, double *grad_acc)
 {
 	__shared__ double red[4][NGRAD];
-	const int b = blockIdx.x;
+	__shared__ unsigned long long hit[kCullWords];
+	const int b = blockIdx.x / parts, part = blockIdx.x - b * parts;
 	const int inst = owner_of(grp_off, ninst, b);
 	const InstDev I = insts[inst];
 	const GalaxyDev &g = gals[I.galaxy];
-	const int rows = g.conv_rows;
+	const int rows = g.conv_rows / parts;  // rows per thread
 	const int t0 = (b - grp_off[inst]) * grp, t1 = min(t0 + grp, g.n_atiles);
 	const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int wpr = (g.DW + 63) >> 6;
+	const int nwords = (I.ncomp + 63) >> 6;
+	for (int w = wv; w < min(nwords, kCullWords); w += 4) {
+		const int k = w * 64 + lane;
+		bool on = false;
+		if (k < I.ncomp) {
+			const Comp &c = comps[I.comp0 + k];
+			if (c.type == TYPE && (bool)c.grad64 == G64)
+				for (int ti = t0; ti < t1 && !on; ++ti) on = tile_class(c, tile_rect(g, g.atiles[ti], g.conv_rows)) != 0;
+		}
+		const unsigned long long m = __ballot(on);
+		if (lane == 0) hit[w] = m;
+	}
+	__syncthreads();
 	const double hx = g.sx / 2., hy = g.sy / 2.;
-	for (int k = 0; k < I.ncomp; ++k) {
+	// G at column i of rows j .. j + kAdjRows - 1 (n of them this thread's), 0
+	// where component k did not draw the pixel directly: the loads of all rows
+	// are in flight together
+	auto load_rows = [&](int k, int tx, int i, int j, int n, float *Gr) {
+		unsigned long long m[kAdjRows];
+#pragma unroll
+		for (int u = 0; u < kAdjRows; ++u) {
+			const bool ok = u < n && j + u < g.DH;
+			m[u] = ok ? I.dmask[((long)k * g.DH + j + u) * wpr + tx] : 0ull;
+			Gr[u] = ok && i < g.DW ? I.G[i + (j + u) * g.DW] : 0.f;
+		}
+#pragma unroll
+		for (int u = 0; u < kAdjRows; ++u) Gr[u] = (m[u] >> lane) & 1ull ? Gr[u] : 0.f;
+	};
+	for (int w = 0; w < nwords; ++w) {
+	  for (unsigned long long left = w < kCullWords ? uniform64(hit[w]) : ~0ull; left; left &= left - 1ull) {
+		const int k = w * 64 + __ffsll((long long)left) - 1;
+		if (k >= I.ncomp) break;
 		const Comp &c = comps[I.comp0 + k];
 		if (c.type != TYPE || (bool)c.grad64 != G64) continue;
 		double gl[NGRAD];
@@ -948,22 +1043,24 @@ __global__ __launch_bounds__(256) void k_adj_render(const GalaxyDev *__restrict_
 		if (G64) {
 			for (int ti = t0; ti < t1; ++ti) {
 				const int2 t = g.atiles[ti];
+				if (tile_class(c, tile_rect(g, t, g.conv_rows)) == 0) continue;
 				const int i = t.x * kTileW + lane;
-				const int j0 = t.y * 4 * rows + wv * rows;
+				const int j0 = t.y * 4 * g.conv_rows + (part * 4 + wv) * rows;
 				const double x = hx + i * g.sy;
-				for (int r = 0; r < rows; ++r) {
-					const int j = j0 + r;
-					if (j >= g.DH) break;
-					const unsigned long long m = I.dmask[((long)k * g.DH + j) * wpr + t.x];
-					if (!((m >> lane) & 1ull)) continue;
-					const float Gq = I.G[i + j * g.DW];
+				for (int r0 = 0; r0 < rows; r0 += kAdjRows) {
+				  float Gr[kAdjRows];
+				  load_rows(k, t.x, i, j0 + r0, rows - r0, Gr);
+#pragma unroll
+				  for (int u = 0; u < kAdjRows; ++u) {
+					const float Gq = Gr[u];
 					if (Gq == 0.f) continue;
-					const double y = hy + j * g.sx;
+					const double y = hy + (j0 + r0 + u) * g.sx;
 					const double xr = x - c.xc, yr = y - c.yc;
 					const double xp = xr * c.cos_ang + yr * c.sin_ang;
 					const double yp = -xr * c.sin_over + yr * c.cos_over;
 					const double wq = (double)Gq * c.flux_scale;
 					vsum += wq * sample_accumulate<float, TYPE>(c, xp, yp, wq, gl);
+				  }
 				}
 			}
 		}
@@ -978,19 +1075,20 @@ __global__ __launch_bounds__(256) void k_adj_render(const GalaxyDev *__restrict_
 			const bool fuse = TYPE == SERSIC && !c.boxy && !c.grad_box;
 			for (int ti = t0; ti < t1; ++ti) {
 				const int2 t = g.atiles[ti];
+				if (tile_class(c, tile_rect(g, t, g.conv_rows)) == 0) continue;
 				const int i = t.x * kTileW + lane;
-				const int j0 = t.y * 4 * rows + wv * rows;
+				const int j0 = t.y * 4 * g.conv_rows + (part * 4 + wv) * rows;
 				const double x = hx + i * g.sy;
-				for (int r = 0; r < rows; ++r) {
-					const int j = j0 + r;
-					if (j >= g.DH) break;
-					const unsigned long long m = I.dmask[((long)k * g.DH + j) * wpr + t.x];
-					if (!m) continue;
-					if (!((m >> lane) & 1ull)) continue;
-					const float Gq = I.G[i + j * g.DW];
+				const float xr = (float)(x - c.xc);
+				for (int r0 = 0; r0 < rows; r0 += kAdjRows) {
+				  float Gr[kAdjRows];
+				  load_rows(k, t.x, i, j0 + r0, rows - r0, Gr);
+#pragma unroll
+				  for (int u = 0; u < kAdjRows; ++u) {
+					const float Gq = Gr[u];
 					if (Gq == 0.f) continue;
-					const double y = hy + j * g.sx;
-					const float xr = (float)(x - c.xc), yr = (float)(y - c.yc);
+					const double y = hy + (j0 + r0 + u) * g.sx;
+					const float yr = (float)(y - c.yc);
 					const float xp = xr * c.f.cos_ang + yr * c.f.sin_ang;
 					const float yp = -xr * c.f.sin_over + yr * c.f.cos_over;
 					const float wq = Gq * fs;
@@ -1003,6 +1101,7 @@ __global__ __launch_bounds__(256) void k_adj_render(const GalaxyDev *__restrict_
 					else {
 						vf += wq * pixel_accumulate_f32<TYPE>(c, xp, yp, wq, gf);
 					}
+				  }
 				}
 			}
 #pragma unroll
@@ -1022,6 +1121,7 @@ __global__ __launch_bounds__(256) void k_adj_render(const GalaxyDev *__restrict_
 			if (v != 0) atomicAdd(&grad_acc[(long)(I.comp0 + k) * NGRAD + s], v);
 		}
 		__syncthreads();
+	  }
 	}
 }
 

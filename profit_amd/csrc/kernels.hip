@@ -206,108 +206,289 @@ __device__ double point_value(const GalaxyDev &g, const PointFoot &f, int px, in
 	return val;
 }
 
-// Tiles are 64 x (4*rows) pixels; thread (tx, ty) covers column tx and rows
-// ty*rows .. ty*rows+rows-1.  filter: -1 every component, 0/1 only those whose
-// convolve flag equals it.  target: 0 canvas, 1 the aux canvas.  With filter
-// -1, point sources and sky drawn without convolution go to the aux canvas
-// when the instance has one in use (InstDev::has_aux); radial profiles are
-// always convolved there.  F64: the kernel holds the FP64 value path (the
-// FP64 model modes, GalaxyDev::render_fp64 / canvas64, and King or Ferrer
-// pixels near their cut-off); without it a Sersic render needs 48 VGPRs
-// instead of 109, eight waves per SIMD instead of four.
+// Rows a render thread draws together (one in the kernels with the FP64 path).
+constexpr int kRowGroup = 4;
+// Sub-sampled pixels a render block gathers in LDS before it appends them (the
+// rest of a tile that has more are appended one wavefront row at a time).
+constexpr int kRenderBuf = 2048;
+
+// Tiles are 64 x (4*rows) pixels; a block draws `grp` consecutive tiles of an
+// instance, or one of `parts` parts of a tile (grp = 1; parts divides rows):
+// thread (tx, ty) covers column tx and rows / parts rows of a tile.
+// filter: -1 every component, 0/1 only those whose convolve flag equals it.
+// target: 0 canvas, 1 the aux canvas.  With filter -1, point sources and sky
+// drawn without convolution go to the aux canvas when the instance has one in
+// use (InstDev::has_aux); radial profiles are always convolved there.  F64: the
+// kernel holds the FP64 value path (the FP64 model modes, GalaxyDev::render_fp64
+// / canvas64, and King or Ferrer pixels near their cut-off); without it a Sersic
+// render needs half the registers.
+//
+// The block first forms each component's tile class (tile_class): components
+// that do nothing on the tile are skipped for all its pixels, and where every
+// pixel is drawn directly none is classified.  Sub-sampled pixels are gathered
+// in LDS and appended with one atomic per work list and block.
 template <int TYPE, bool F64>
 __global__ __launch_bounds__(256) void k_render(const GalaxyDev *__restrict__ gals, const InstDev *__restrict__ insts,
-                                                const int *__restrict__ tile_off, int ninst,
+                                                const int *__restrict__ grp_off, int ninst, int grp, int parts,
                                                 const Comp *__restrict__ comps, WorkQueue wq, int filter, int target,
                                                 int *diag_cls)
 {
-	const int b = blockIdx.x;
-	const int inst = owner_of(tile_off, ninst, b);
+	constexpr int kHeavy = kFamilies;  // list index of the centre pixels
+	__shared__ QEntry buf[kRenderBuf];
+	__shared__ uint8_t buf_list[kRenderBuf];
+	__shared__ unsigned long long hit[kCullWords], whole[kCullWords];
+	__shared__ int nbuf, list_n[kFamilies + 1], list_base[kFamilies + 1];
+	const int b = blockIdx.x / parts, part = blockIdx.x - b * parts;
+	const int inst = owner_of(grp_off, ninst, b);
 	const InstDev I = insts[inst];
 	const GalaxyDev &g = gals[I.galaxy];
-	const int rows = g.conv_rows;
-	const int2 t = g.atiles[b - tile_off[inst]];
-	const int lane = threadIdx.x & 63;
-	const int i = t.x * kTileW + lane;
-	const int j0 = t.y * 4 * rows + (threadIdx.x >> 6) * rows;
+	const int rows = g.conv_rows / parts;  // rows per thread
+	const int t0 = (b - grp_off[inst]) * grp, t1 = min(t0 + grp, g.n_atiles);
+	const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const double hx = g.sx / 2., hy = g.sy / 2.;
 	float *out = target ? I.aux : I.canvas;
-	for (int r = 0; r < rows; ++r) {
-		const int j = j0 + r;
-		const bool inb = i < g.DW && j < g.DH;
-		const int pix = i + j * g.DW;
-		const bool active = inb && (!g.has_calc || g.calc[pix]);
-		// radial.cpp:313-314: the x centre uses scale.y and the y centre scale.x
-		const double y = hy + j * g.sx;
-		const double x = hx + i * g.sy;
-		float acc = 0.f, aux_acc = 0.f;
+	const int nwords = (I.ncomp + 63) >> 6;
+	if (threadIdx.x == 0) nbuf = 0;
+	if (threadIdx.x <= kFamilies) list_n[threadIdx.x] = 0;
+	// gathers the pixel's entry (heavy: a centre pixel) where `take`; the ones
+	// beyond the LDS list are appended directly
+	auto gather = [&](bool take, bool heavy, int fam, QEntry e) {
+		const unsigned long long m = __ballot(take);
+		if (!m) return;
+		const int leader = __ffsll((long long)m) - 1;
+		int at = 0;
+		if (lane == leader) at = atomicAdd(&nbuf, __popcll(m));
+		at = __shfl(at, leader) + __popcll(m & ((1ull << lane) - 1ull));
+		const bool fits = at < kRenderBuf;
+		if (take && fits) {
+			buf[at] = e;
+			buf_list[at] = (uint8_t)(heavy ? kHeavy : fam);
+		}
+		if (__ballot(take && !fits)) {
+			append_entry(take && !heavy && !fits, lane, wq.light + wq.lbase[fam], wq.count + light_count(fam),
+			             wq.lbase[fam + 1] - wq.lbase[fam], e);
+			append_entry(take && heavy && !fits, lane, wq.heavy, wq.count + 1, wq.hcap, e);
+		}
+	};
+	const int wpr = (g.DW + 63) >> 6;
+	for (int ti = t0; ti < t1; ++ti) {
+	  const int2 t = g.atiles[ti];
+	  const int i = t.x * kTileW + lane;
+	  const int j0 = t.y * 4 * g.conv_rows + (part * 4 + wv) * rows;
+	  if (ti > t0) __syncthreads();  // the last tile's masks have been read
+	  {
+		const TileRect rect = tile_rect(g, t, g.conv_rows);
+		for (int w = wv; w < min(nwords, kCullWords); w += 4) {
+			const int k = w * 64 + lane;
+			int tc = 0;
+			// the diagnostics write every component's class
+			if (k < I.ncomp) tc = diag_cls ? 1 : tile_class(comps[I.comp0 + k], rect);
+			const unsigned long long h = __ballot(tc != 0), v = __ballot(tc == 2);
+			if (lane == 0) {
+				hit[w] = h;
+				whole[w] = v;
+			}
+		}
+	  }
+	  __syncthreads();
+	// radial.cpp:313-314: the x centre uses scale.y and the y centre scale.x
+	const double x = hx + i * g.sy;
+	// kRowGroup rows at a time with the component loop outside: a component's
+	// constants are loaded once a group, and the group's rows are independent
+	constexpr int U = F64 ? 1 : kRowGroup;
+	for (int r0 = 0; r0 < rows; r0 += U) {
+		bool inb[U], active[U];
+		float acc[U];
+#pragma unroll
+		for (int u = 0; u < U; ++u) {
+			const int j = j0 + r0 + u;
+			inb[u] = i < g.DW && j < g.DH && r0 + u < rows;
+			active[u] = inb[u] && (!g.has_calc || g.calc[i + j * g.DW]);
+			acc[u] = 0.f;
+		}
+		float aux_acc[U] = {};
 		double acc64 = 0.0;  // the FP64 canvas's sum (GalaxyDev::canvas64)
-		for (int k = 0; k < I.ncomp; ++k) {
+		for (int w = 0; w < nwords; ++w) {
+		  const unsigned long long wm = w < kCullWords ? uniform64(whole[w]) : 0ull;
+		  for (unsigned long long left = w < kCullWords ? uniform64(hit[w]) : ~0ull; left; left &= left - 1ull) {
+			const int k = w * 64 + __ffsll((long long)left) - 1;
+			if (k >= I.ncomp) break;
 			const Comp &c = comps[I.comp0 + k];
 			if (filter >= 0 && c.convolve != filter) continue;
+			const int fam = TYPE >= 0 ? TYPE : c.type;
+			// component k's masks of directly drawn pixels for the adjoint
+			// render: lane u holds row j0 + r0 + u's and writes it
+			unsigned mlo = 0, mhi = 0;
+			auto keep_mask = [&](int u, unsigned long long m) {
+				mlo = lane == u ? (unsigned)m : mlo;
+				mhi = lane == u ? (unsigned)(m >> 32) : mhi;
+			};
+			auto store_masks = [&]() {
+				const int j = j0 + r0 + lane;
+				if (I.dmask && lane < U && r0 + lane < rows && j < g.DH)
+					I.dmask[((long)k * g.DH + j) * wpr + t.x] = (unsigned long long)mhi << 32 | mlo;
+			};
 			if (TYPE < 0 && !is_radial(c.type)) {
 				// sky.cpp:47-63 (calc pixels only) and psf.cpp:58-145 (mask ignored)
-				float v = 0.f;
-				if (c.type == SKY) {
-					if (active) v = (float)c.flux_scale;
-				}
-				else if (c.type == POINTSRC && inb) {
-					const PointFoot f = point_footprint(c, g);
-					if (i >= f.x0 && i <= f.x1 && j >= f.y0 && j <= f.y1) {
-						double dvx, dvy;
-						v = (float)(point_value(g, f, i, j, &dvx, &dvy) * c.flux_scale);
+#pragma unroll
+				for (int u = 0; u < U; ++u) {
+					const int j = j0 + r0 + u;
+					float v = 0.f;
+					if (c.type == SKY) {
+						if (active[u]) v = (float)c.flux_scale;
 					}
+					else if (c.type == POINTSRC && inb[u]) {
+						const PointFoot f = point_footprint(c, g);
+						if (i >= f.x0 && i <= f.x1 && j >= f.y0 && j <= f.y1) {
+							double dvx, dvy;
+							v = (float)(point_value(g, f, i, j, &dvx, &dvy) * c.flux_scale);
+						}
+					}
+					if (filter < 0 && !c.convolve && I.has_aux) aux_acc[u] += v;
+					else if (F64 && g.canvas64 && !target) acc64 += (double)v;
+					else acc[u] += v;
+					if (diag_cls && inb[u]) diag_cls[(long)(I.comp0 + k) * g.DW * g.DH + i + j * g.DW] = 0;
 				}
-				if (filter < 0 && !c.convolve && I.has_aux) aux_acc += v;
-				else if (F64 && g.canvas64 && !target) acc64 += (double)v;
-				else acc += v;
-				if (diag_cls && inb) diag_cls[(long)(I.comp0 + k) * g.DW * g.DH + pix] = 0;
-				if (I.dmask && lane == 0 && j < g.DH) I.dmask[((long)k * g.DH + j) * ((g.DW + 63) >> 6) + t.x] = 0ull;
+				store_masks();
 				continue;
 			}
-			bool sub = false, heavy = false;
-			int cls = 0;
-			if (active) {
-				// FP32 profile coordinates from the FP64 offsets; FP64 ones
-				// (libprofit's) only where the class or the value needs them
-				const float fxr = (float)(x - c.xc), fyr = (float)(y - c.yc);
-				const float fxp = fxr * c.f.cos_ang + fyr * c.f.sin_ang;
-				const float fyp = -fxr * c.f.sin_over + fyr * c.f.cos_over;
-				cls = classify32(c, fxp, fyp);
-				if (cls < 0) cls = classify(c, x, y).cls;
-				if (cls == 2) {
-					const bool c64 = F64 && g.canvas64 && !target;
-					if (F64 && (c64 || g.render_fp64 || near_cut_fp64<TYPE>(c, fxp, fyp))) {
-						const PixelClass pc = classify(c, x, y);
-						const double v = c.flux_scale * eval_at<double, TYPE>(c, pc.xp, pc.yp);
-						if (c64) acc64 += v;
-						else acc += (float)v;
-					}
-					else {
-						acc += (float)c.flux_scale * eval_at<float, TYPE>(c, fxp, fyp);
-					}
+			const bool all_direct = (wm & (left & (0ull - left))) != 0ull;
+			const float fs = (float)c.flux_scale;
+			const float fxr = (float)(x - c.xc);
+			// FP32 profile coordinates from the FP64 offsets
+			float fxp[U], fyp[U];
+#pragma unroll
+			for (int u = 0; u < U; ++u) {
+				const float fyr = (float)(hy + (j0 + r0 + u) * g.sx - c.yc);
+				fxp[u] = fxr * c.f.cos_ang + fyr * c.f.sin_ang;
+				fyp[u] = -fxr * c.f.sin_over + fyr * c.f.cos_over;
+			}
+			// the group's FP32 values: a Sersic without box as one straight
+			// run of instructions
+			float val[U];
+			auto values = [&]() {
+				if (TYPE == SERSIC && !c.boxy) {
+					float base, l2, rf;
+#pragma unroll
+					for (int u = 0; u < U; ++u) val[u] = sersic_parts_f32(c, fxp[u], fyp[u], base, l2, rf);
 				}
-				else if (cls == 3) {
-					// the deep centre-pixel trees (sersic.cpp:331-347) go to their own list
-					heavy = centre_pixel(c, x, y);
-					sub = !heavy;
+				else {
+#pragma unroll
+					for (int u = 0; u < U; ++u) val[u] = eval_at<float, TYPE>(c, fxp[u], fyp[u]);
+				}
+			};
+			if (!F64 && all_direct) {
+				values();
+#pragma unroll
+				for (int u = 0; u < U; ++u) {
+					if (active[u]) acc[u] += fs * val[u];
+					keep_mask(u, __ballot(active[u]));
+				}
+				store_masks();
+				continue;
+			}
+			// the rows' classes as bits: drawn directly, sub-sampled, or (too
+			// close to a threshold for FP32) left to libprofit's FP64 coordinates
+			unsigned direct = 0, sub = 0, unsure = 0;
+#pragma unroll
+			for (int u = 0; u < U; ++u) {
+				const int cls = active[u] ? all_direct ? 2 : classify32(c, fxp[u], fyp[u]) : 0;
+				direct |= (cls == 2 ? 1u : 0u) << u;
+				sub |= (cls == 3 ? 1u : 0u) << u;
+				unsure |= (cls < 0 ? 1u : 0u) << u;
+			}
+			if (__ballot(unsure != 0)) {
+#pragma unroll 1
+				for (int u = 0; u < U; ++u) {
+					if (!((unsure >> u) & 1u)) continue;
+					const int cls = classify(c, x, hy + (j0 + r0 + u) * g.sx).cls;
+					direct |= (cls == 2 ? 1u : 0u) << u;
+					sub |= (cls == 3 ? 1u : 0u) << u;
 				}
 			}
-			if (diag_cls && inb) diag_cls[(long)(I.comp0 + k) * g.DW * g.DH + pix] = cls;
-			// direct-pixel mask for the adjoint render
-			const unsigned long long dm = __ballot(cls == 2);
-			if (I.dmask && lane == 0 && j < g.DH)
-				I.dmask[((long)k * g.DH + j) * ((g.DW + 63) >> 6) + t.x] = dm;
-			const int fam = TYPE >= 0 ? TYPE : c.type;
-			append_entry(sub, lane, wq.light + wq.lbase[fam], wq.count + light_count(fam),
-			             wq.lbase[fam + 1] - wq.lbase[fam], QEntry{I.comp0 + k, pix});
-			append_entry(heavy, lane, wq.heavy, wq.count + 1, wq.hcap, QEntry{I.comp0 + k, pix});
+			if (!F64 && __ballot(direct != 0)) values();
+#pragma unroll
+			for (int u = 0; u < U; ++u) {
+				const unsigned long long m = __ballot((direct >> u) & 1u);
+				keep_mask(u, m);
+				if (!m) continue;
+				const bool on = (direct >> u) & 1u, c64 = F64 && g.canvas64 && !target;
+				if (F64 && on && (c64 || g.render_fp64 || near_cut_fp64<TYPE>(c, fxp[u], fyp[u]))) {
+					const PixelClass pc = classify(c, x, hy + (j0 + r0 + u) * g.sx);
+					const double v = c.flux_scale * eval_at<double, TYPE>(c, pc.xp, pc.yp);
+					if (c64) acc64 += v;
+					else acc[u] += (float)v;
+				}
+				else if (on) {
+					acc[u] += fs * (F64 ? eval_at<float, TYPE>(c, fxp[u], fyp[u]) : val[u]);
+				}
+			}
+			store_masks();
+			if (diag_cls || __ballot(sub != 0)) {
+#pragma unroll 1
+				for (int u = 0; u < U; ++u) {
+					const int j = j0 + r0 + u, pix = i + j * g.DW;
+					const bool take = (sub >> u) & 1u;
+					if (diag_cls && i < g.DW && j < g.DH && r0 + u < rows) {
+						const bool on = !g.has_calc || g.calc[pix];
+						diag_cls[(long)(I.comp0 + k) * g.DW * g.DH + pix] = take ? 3 : (direct >> u) & 1u ? 2 : on ? 1 : 0;
+					}
+					// the deep centre-pixel trees (sersic.cpp:331-347) go to their own list
+					gather(take, take && centre_pixel(c, x, hy + j * g.sx), fam, QEntry{I.comp0 + k, pix});
+				}
+			}
+		  }
 		}
-		if (inb) {
+#pragma unroll
+		for (int u = 0; u < U; ++u) {
+			if (!inb[u]) continue;
+			const int pix = i + (j0 + r0 + u) * g.DW;
 			if (F64 && g.canvas64 && !target) I.canvas64[pix] = acc64;
-			else out[pix] = acc;
+			else out[pix] = acc[u];
+			if (filter < 0 && I.has_aux) I.aux[pix] = aux_acc[u];
 		}
-		if (inb && filter < 0 && I.has_aux) I.aux[pix] = aux_acc;
+	}
+	}
+	// the gathered entries: places within the block's share of each list, then
+	// one atomic per list, then the writes
+	__syncthreads();
+	const int n = min(nbuf, kRenderBuf);
+	if (n == 0) return;
+	constexpr int kPer = kRenderBuf / 256;
+	int place[kPer];
+#pragma unroll
+	for (int u = 0; u < kPer; ++u) {
+		const int e = u * 256 + threadIdx.x;
+		const int list = e < n ? buf_list[e] : -1;
+		place[u] = 0;
+		if (u * 256 >= n) continue;
+		for (int f = TYPE >= 0 ? TYPE : 0; f <= kHeavy; f = TYPE >= 0 && f != kHeavy ? kHeavy : f + 1) {
+			const unsigned long long m = __ballot(list == f);
+			if (!m) continue;
+			const int leader = __ffsll((long long)m) - 1;
+			int at = 0;
+			if (lane == leader) at = atomicAdd(&list_n[f], __popcll(m));
+			at = __shfl(at, leader);
+			if (list == f) place[u] = at + __popcll(m & ((1ull << lane) - 1ull));
+		}
+	}
+	__syncthreads();
+	if (threadIdx.x <= kHeavy) {
+		const int f = threadIdx.x, cnt = list_n[f];
+		if (cnt) list_base[f] = atomicAdd(f == kHeavy ? wq.count + 1 : wq.count + light_count(f), cnt);
+	}
+	__syncthreads();
+#pragma unroll
+	for (int u = 0; u < kPer; ++u) {
+		const int e = u * 256 + threadIdx.x;
+		if (e >= n) continue;
+		const int list = buf_list[e], slot = list_base[list] + place[u];
+		if (list == kHeavy) {
+			if (slot < wq.hcap) wq.heavy[slot] = buf[e];
+		}
+		else if (slot < wq.lbase[list + 1] - wq.lbase[list]) {
+			wq.light[wq.lbase[list] + slot] = buf[e];
+		}
 	}
 }
 
@@ -866,16 +1047,17 @@ int launch_zero_i(int *p, long n, hipStream_t st)
 	return (int)hipGetLastError();
 }
 
-int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *tile_off, int ninst, int nblocks,
+int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *grp_off, int ninst, int nblocks, int grp, int parts,
                   const Comp *comps, WorkQueue wq, int filter, int target, int *diag_cls, hipStream_t st, int type,
                   bool fp64)
 {
 	if (nblocks <= 0) return 0;
+	if (grp < 1 || parts < 1 || (grp > 1 && parts > 1)) return (int)hipErrorInvalidValue;
 	// type >= 0: every component of the batch is of that radial family (the
 	// kernel then holds that family's code alone); -1 any mix.  King and
 	// Ferrer always take the kernel with the FP64 value path.
 	if (type == KING || type == FERRER) fp64 = true;
-#define PA_RENDER(T, F) k_render<T, F><<<nblocks, 256, 0, st>>>(gals, insts, tile_off, ninst, comps, wq, filter, target, diag_cls)
+#define PA_RENDER(T, F) k_render<T, F><<<nblocks * parts, 256, 0, st>>>(gals, insts, grp_off, ninst, grp, parts, comps, wq, filter, target, diag_cls)
 	if (fp64) {
 		switch (type) {
 		case SERSIC: PA_RENDER(SERSIC, true); break;

@@ -9,9 +9,10 @@ namespace profit_amd {
 
 template <int TYPE, int PREC>
 static int adj_render_launch(const GalaxyDev *gals, const InstDev *insts, const int *grp_off, int ninst, int nblocks,
-                             int grp, const Comp *comps, double *grad_acc, hipStream_t st)
+                             int grp, int parts, const Comp *comps, double *grad_acc, hipStream_t st)
 {
-	k_adj_render<TYPE, PREC != 0><<<nblocks, 256, 0, st>>>(gals, insts, grp_off, ninst, grp, comps, grad_acc);
+	k_adj_render<TYPE, PREC != 0><<<nblocks * parts, 256, 0, st>>>(gals, insts, grp_off, ninst, grp, parts, comps,
+	                                                               grad_acc);
 	return (int)hipGetLastError();
 }
 
@@ -55,11 +56,11 @@ int launch_adj_queue(int type, int nblocks, const InstDev *insts, const Comp *co
 }
 
 int launch_adj_render(int type, int prec, const GalaxyDev *gals, const InstDev *insts, const int *grp_off, int ninst,
-                      int nblocks, int grp, const Comp *comps, double *grad_acc, hipStream_t st)
+                      int nblocks, int grp, int parts, const Comp *comps, double *grad_acc, hipStream_t st)
 {
 	if (nblocks <= 0) return 0;
-	if (grp < 1) return (int)hipErrorInvalidValue;
-#define PA_RENDER(T, P) adj_render_launch<T, P>(gals, insts, grp_off, ninst, nblocks, grp, comps, grad_acc, st)
+	if (grp < 1 || parts < 1 || (grp > 1 && parts > 1)) return (int)hipErrorInvalidValue;
+#define PA_RENDER(T, P) adj_render_launch<T, P>(gals, insts, grp_off, ninst, nblocks, grp, parts, comps, grad_acc, st)
 	PA_ADJ_CASES(PA_RENDER)
 #undef PA_RENDER
 }
