@@ -140,5 +140,10 @@ __host__ __device__ constexpr int light_count(int type) { return 14 + type; }
 __host__ __device__ constexpr int big_count(int type) { return 20 + type; }
 __host__ __device__ constexpr int deep_count(int type) { return 26 + type; }
 
+// Where an evaluation's results go (pinned host memory); ll and grad nullable.
+struct HostReport {
+	double *ll, *grad;
+	int *errors, *qcount;
+};
 
 }  // namespace profit_amd

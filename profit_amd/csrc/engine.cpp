@@ -961,14 +961,12 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 		hip_check(hipMemcpy(d_setup_order_.as<int>(), order.data(), nc * sizeof(int), hipMemcpyHostToDevice), "order");
 		setup_types_.assign(nc, -1);
 	}
-	d_params_.alloc(nc * sizeof(ProfileParams));
 	d_comps_.alloc(nc * sizeof(Comp));
 	d_err_.alloc(nc * sizeof(int));
 	d_partial_.alloc(std::max(1, lk_off_[n]) * sizeof(double));
 	d_ll_.alloc(std::max(1, n) * sizeof(double));
 	d_gscale_.alloc(std::max(1, n) * sizeof(double));
 	d_grad_acc_.alloc((size_t)nc * NGRAD * sizeof(double));
-	d_grad_out_.alloc((size_t)nc * NGRAD * sizeof(double));
 	d_qcount_.alloc(kQueueCounters * sizeof(int));
 	h_params_.alloc(nc * sizeof(ProfileParams));
 	h_ll_.alloc(std::max(1, n) * sizeof(double));
@@ -995,18 +993,13 @@ void Engine::record(bool grad)
 	const int nc = ncomp_total_;
 	const GalaxyDev *gals = d_gals_.as<GalaxyDev>();
 	const InstDev *insts = d_insts_.as<InstDev>();
-	hip_check(hipMemcpyAsync(d_params_.as<ProfileParams>(), h_params_.as<ProfileParams>(), nc * sizeof(ProfileParams),
-	                         hipMemcpyHostToDevice, st),
-	          "params");
 	mark(0);
-	hip_check(launch_setup(d_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
-	                       d_err_.as<int>(), nc, st),
+	hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
+	                       d_err_.as<int>(), nc, d_qcount_.as<int>(), grad ? d_grad_acc_.as<double>() : nullptr, st),
 	          "setup");
 	if (grad && (radial_types_ & ((1u << KING) | (1u << CORESERSIC) | (1u << BROKENEXP))))
 		hip_check(launch_setup_grad(d_setup_order_.as<int>(), d_comps_.as<Comp>(), d_err_.as<int>(), nc, st),
 		          "setup grad");
-	hip_check(launch_zero_i(d_qcount_.as<int>(), kQueueCounters, st), "zero");
-	if (grad) hip_check(launch_zero_d(d_grad_acc_.as<double>(), (long)nc * NGRAD, st), "zero");
 	mark(1);
 	// a batch of one radial family alone takes the render compiled for it
 	int rtype = -1;
@@ -1048,18 +1041,19 @@ void Engine::record(bool grad)
 				                           d_grad_acc_.as<double>(), st),
 				          "adjoint subsample");
 		mark(8);
-		hip_check(launch_grad_finalize(d_comps_.as<Comp>(), d_gscale_.as<double>(), d_grad_acc_.as<double>(),
-		                               d_grad_out_.as<double>(), nc, grad_slots_, st),
-		          "grad");
-		mark(9);
-		hip_check(hipMemcpyAsync(h_grad_.as<double>(), d_grad_out_.as<double>(), (size_t)nc * NGRAD * sizeof(double),
-		                         hipMemcpyDeviceToHost, st),
-		          "grad copy");
 	}
-	hip_check(hipMemcpyAsync(h_ll_.as<double>(), d_ll_.as<double>(), n * sizeof(double), hipMemcpyDeviceToHost, st),
-	          "ll copy");
-	hip_check(hipMemcpyAsync(h_err_.as<int>(), d_err_.as<int>(), nc * sizeof(int), hipMemcpyDeviceToHost, st), "err");
-	hip_check(hipMemcpyAsync(h_qcount_.as<int>(), d_qcount_.as<int>(), kQueueCounters * sizeof(int), hipMemcpyDeviceToHost, st), "qcount");
+	report(true, grad, st);
+	if (grad) mark(9);
+}
+
+// the results to the pinned host buffers (the last launch of an evaluation)
+void Engine::report(bool ll, bool grad, hipStream_t st)
+{
+	const HostReport out{ll ? h_ll_.as<double>() : nullptr, grad ? h_grad_.as<double>() : nullptr, h_err_.as<int>(),
+	                     h_qcount_.as<int>()};
+	hip_check(launch_report(d_comps_.as<Comp>(), d_gscale_.as<double>(), d_grad_acc_.as<double>(), d_ll_.as<double>(),
+	                        d_err_.as<int>(), d_qcount_.as<int>(), ncomp_total_, ninst(), grad_slots_, out, st),
+	          "report");
 }
 
 void Engine::check_setup_errors()
@@ -1231,21 +1225,15 @@ void Engine::diagnostics(const ProfileParams *params, int *cls, int *nodes)
 	const GalaxyDev *gals = d_gals_.as<GalaxyDev>();
 	const InstDev *insts = d_insts_.as<InstDev>();
 	for (int attempt = 0; attempt < 4; ++attempt) {
-		hip_check(hipMemcpyAsync(d_params_.as<ProfileParams>(), h_params_.as<ProfileParams>(), nc * sizeof(ProfileParams),
-		                         hipMemcpyHostToDevice, st),
-		          "params");
-		hip_check(launch_setup(d_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
-		                       d_err_.as<int>(), nc, st),
+		hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
+		                       d_err_.as<int>(), nc, d_qcount_.as<int>(), nullptr, st),
 		          "setup");
-		hip_check(launch_zero_i(d_qcount_.as<int>(), kQueueCounters, st), "zero");
 		hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), 1, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
 		                        work_queue(), -1, 0, dcls.as<int>(), st),
 		          "render");
 		hip_check(launch_subsample_nodes(subsample_blocks_, gals, insts, d_comps_.as<Comp>(), work_queue(), dnodes.as<int>(), st),
 		          "nodes");
-		hip_check(hipMemcpyAsync(h_err_.as<int>(), d_err_.as<int>(), nc * sizeof(int), hipMemcpyDeviceToHost, st), "err");
-		hip_check(hipMemcpyAsync(h_qcount_.as<int>(), d_qcount_.as<int>(), kQueueCounters * sizeof(int), hipMemcpyDeviceToHost, st),
-		          "qcount");
+		report(false, false, st);
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
 		if (queue_ok()) break;
@@ -1263,11 +1251,8 @@ void Engine::adjusted_settings(const ProfileParams *params, int *res, int *maxre
 	if (nc == 0) return;
 	std::memcpy(h_params_.as<ProfileParams>(), params, nc * sizeof(ProfileParams));
 	hipStream_t st = stream_;
-	hip_check(hipMemcpyAsync(d_params_.as<ProfileParams>(), h_params_.as<ProfileParams>(), nc * sizeof(ProfileParams),
-	                         hipMemcpyHostToDevice, st),
-	          "params");
-	hip_check(launch_setup(d_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), d_insts_.as<InstDev>(),
-	                       d_gals_.as<GalaxyDev>(), d_comps_.as<Comp>(), d_err_.as<int>(), nc, st),
+	hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), d_insts_.as<InstDev>(),
+	                       d_gals_.as<GalaxyDev>(), d_comps_.as<Comp>(), d_err_.as<int>(), nc, nullptr, nullptr, st),
 	          "setup");
 	std::vector<Comp> comps(nc);
 	hip_check(hipMemcpyAsync(comps.data(), d_comps_.as<Comp>(), nc * sizeof(Comp), hipMemcpyDeviceToHost, st), "comps");
@@ -1295,21 +1280,15 @@ void Engine::model_images(const ProfileParams *params, float *out)
 	const InstDev *insts = d_insts_.as<InstDev>();
 	mask_walk_ = false;
 	for (int attempt = 0; attempt < 4; ++attempt) {
-		hip_check(hipMemcpyAsync(d_params_.as<ProfileParams>(), h_params_.as<ProfileParams>(), nc * sizeof(ProfileParams),
-		                         hipMemcpyHostToDevice, st),
-		          "params");
-		hip_check(launch_setup(d_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
-		                       d_err_.as<int>(), nc, st),
+		hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
+		                       d_err_.as<int>(), nc, d_qcount_.as<int>(), nullptr, st),
 		          "setup");
-		hip_check(launch_zero_i(d_qcount_.as<int>(), kQueueCounters, st), "zero");
 		hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), n, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
 		                        work_queue(), -1, 0, nullptr, st),
 		          "render");
 		launch_walkers_fwd(0, false, st);
 		conv_forward(1, st);
-		hip_check(hipMemcpyAsync(h_err_.as<int>(), d_err_.as<int>(), nc * sizeof(int), hipMemcpyDeviceToHost, st), "err");
-		hip_check(hipMemcpyAsync(h_qcount_.as<int>(), d_qcount_.as<int>(), kQueueCounters * sizeof(int), hipMemcpyDeviceToHost, st),
-		          "qcount");
+		report(false, false, st);
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
 		if (queue_ok()) break;
@@ -1341,13 +1320,9 @@ void Engine::model_canvas(const ProfileParams *params, float *out, float *out_di
 	const bool conv = g.has_psf != 0;
 	mask_walk_ = false;
 	for (int attempt = 0; attempt < 4; ++attempt) {
-		hip_check(hipMemcpyAsync(d_params_.as<ProfileParams>(), h_params_.as<ProfileParams>(), nc * sizeof(ProfileParams),
-		                         hipMemcpyHostToDevice, st),
-		          "params");
-		hip_check(launch_setup(d_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
-		                       d_err_.as<int>(), nc, st),
+		hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
+		                       d_err_.as<int>(), nc, d_qcount_.as<int>(), nullptr, st),
 		          "setup");
-		hip_check(launch_zero_i(d_qcount_.as<int>(), kQueueCounters, st), "zero");
 		// convolved profiles into the canvas, the others into the aux canvas
 		hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), 1, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
 		                        work_queue(), conv ? 1 : -1, 0, nullptr, st),
@@ -1358,9 +1333,7 @@ void Engine::model_canvas(const ProfileParams *params, float *out, float *out_di
 			          "render");
 		launch_walkers_fwd(conv ? 1 : 0, false, st);
 		if (conv && !out_direct) conv_forward(1, st);
-		hip_check(hipMemcpyAsync(h_err_.as<int>(), d_err_.as<int>(), nc * sizeof(int), hipMemcpyDeviceToHost, st), "err");
-		hip_check(hipMemcpyAsync(h_qcount_.as<int>(), d_qcount_.as<int>(), kQueueCounters * sizeof(int), hipMemcpyDeviceToHost, st),
-		          "qcount");
+		report(false, false, st);
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
 		if (queue_ok()) break;

@@ -15,12 +15,12 @@ namespace profit_amd {
 
 // kernel launchers (kernels.hip)
 // order: the components grouped by profile family (one thread each)
+// qcount, grad_acc (nullable): the work-list counters and gradient sums to clear
 int launch_setup(const ProfileParams *params, const int *order, const int *comp_inst, const InstDev *insts,
-                 const GalaxyDev *gals, Comp *comps, int *errors, int ncomp, hipStream_t st);
+                 const GalaxyDev *gals, Comp *comps, int *errors, int ncomp, int *qcount, double *grad_acc,
+                 hipStream_t st);
 // the QUADPACK luminosity gradients (King, core-Sersic, broken exponential)
 int launch_setup_grad(const int *order, Comp *comps, const int *errors, int ncomp, hipStream_t st);
-int launch_zero_d(double *p, long n, hipStream_t st);
-int launch_zero_i(int *p, long n, hipStream_t st);
 // fp64: some pixel may take an FP64 value (the FP64 model modes, King or
 // Ferrer components in the batch); false only when none can
 // grp: canvas tiles per block, or parts: blocks per tile (a divisor of the
@@ -49,8 +49,9 @@ int launch_like_t(const GalaxyDev *gals, const InstDev *insts, int ninst, int gr
                   hipStream_t st);
 int launch_adj_render(int type, int prec, const GalaxyDev *gals, const InstDev *insts, const int *grp_off, int ninst,
                       int nblocks, int grp, int parts, const Comp *comps, double *grad_acc, hipStream_t st);
-int launch_grad_finalize(const Comp *comps, const double *gscale, const double *grad_acc, double *grad_out,
-                         int ncomp, unsigned slot_mask, hipStream_t st);
+// an evaluation's results to pinned host memory
+int launch_report(const Comp *comps, const double *gscale, const double *grad_acc, const double *ll, const int *errors,
+                  const int *qcount, int ncomp, int ninst, unsigned slot_mask, const HostReport &out, hipStream_t st);
 int launch_dilate(const uint8_t *in, uint8_t *tmp, uint8_t *out, int w, int h, int padx, int pady, hipStream_t st);
 // FFT path (fft.hip)
 int launch_fft_rows_fwd(int nblocks, int nmax, const GalaxyDev *gals, const InstDev *insts, const int *row_off,
@@ -260,6 +261,7 @@ class Engine {
 	WorkQueue work_queue();
 	bool queue_ok() const;
 	void grow_queue();
+	void report(bool ll, bool grad, hipStream_t st);
 	void check_setup_errors();
 
 	int device_ = 0;
@@ -329,7 +331,7 @@ class Engine {
 	// per instance: canvas, w, G, aux, FFT frame, direct-pixel mask, FP64 canvas
 	static constexpr int kInstBufs = 7;
 	std::vector<DevBuf> inst_bufs_;
-	DevBuf d_params_, d_comps_, d_err_, d_queue_, d_qcount_, d_partial_, d_ll_, d_gscale_, d_grad_acc_, d_grad_out_;
+	DevBuf d_comps_, d_err_, d_queue_, d_qcount_, d_partial_, d_ll_, d_gscale_, d_grad_acc_;
 	long lcap_[kFamilies] = {}, hcap_ = 0;
 	DevBuf d_hqueue_, d_qjac_, d_hjac_, d_qdeep_;
 	HostBuf h_params_, h_ll_, h_grad_, h_err_, h_qcount_;

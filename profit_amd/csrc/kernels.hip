@@ -21,6 +21,8 @@
 // and of the recursion rounds exactly as libprofit's own build does.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernel_common.h"
 
 namespace profit_amd {
@@ -30,14 +32,19 @@ namespace profit_amd {
 // The components' set-up in `order` (grouped by profile family), one
 // wavefront per component: the set-up runs alike on every lane and the
 // Kronrod points of its luminosity integrals spread over the lanes; the
-// QUADPACK luminosity gradients are left to k_setup_grad.
+// QUADPACK luminosity gradients are left to k_setup_grad.  It also clears the
+// evaluation's work-list counters and (where given) gradient sums, which spares
+// two launches of 4.6 us; `params` may be pinned host memory, which spares a
+// copy of 5 us.
 __global__ __launch_bounds__(256, 2) void k_setup(const ProfileParams *__restrict__ params,
                                                   const int *__restrict__ order, const int *__restrict__ comp_inst,
                                                   const InstDev *__restrict__ insts,
                                                   const GalaxyDev *__restrict__ gals, Comp *comps, int *errors,
-                                                  int ncomp)
+                                                  int ncomp, int *qcount, double *grad_acc)
 {
 	const int t = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+	if (blockIdx.x == 0 && threadIdx.x < kQueueCounters && qcount) qcount[threadIdx.x] = 0;
+	if (t < ncomp && (threadIdx.x & 63) < NGRAD && grad_acc) grad_acc[(long)t * NGRAD + (threadIdx.x & 63)] = 0;
 	if (t >= ncomp) return;
 	const int c = order[t];
 	const int inst = comp_inst[c];
@@ -70,18 +77,6 @@ __global__ __launch_bounds__(256, 4) void k_setup_grad(const int *__restrict__ o
 	sf::QuadState qs;
 	const double v = lum_gradient<true>(comps[c], w, &qs);
 	if ((threadIdx.x & 63) == 0) comps[c].dlnfs[G_S0 + w] = v;
-}
-
-__global__ void k_fill_zero_d(double *p, long n)
-{
-	const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n) p[i] = 0;
-}
-
-__global__ void k_fill_zero_i(int *p, long n)
-{
-	const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n) p[i] = 0;
 }
 
 // ------------------------------------------------------------------ classification
@@ -777,22 +772,31 @@ __global__ __launch_bounds__(256) void k_conv(const GalaxyDev *__restrict__ gals
 // ------------------------------------------------------------------ likelihood finalisation
 
 // The likelihood partials of instance i sit at [lk_off[i], lk_off[i+1]),
-// written by whichever convolution kernel its galaxy uses.
-__global__ void k_like_finalize(const GalaxyDev *__restrict__ gals, const InstDev *__restrict__ insts,
-                                const int *__restrict__ lk_off, int ninst, const double *__restrict__ partial,
-                                double *ll, double *gscale)
+// written by whichever convolution kernel its galaxy uses.  One wavefront per
+// instance: the 269 partials of a 2048x2048 field took one thread 100 us.
+__global__ __launch_bounds__(256) void k_like_finalize(const GalaxyDev *__restrict__ gals,
+                                                       const InstDev *__restrict__ insts,
+                                                       const int *__restrict__ lk_off, int ninst,
+                                                       const double *__restrict__ partial, double *ll, double *gscale)
 {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6), lane = threadIdx.x & 63;
 	if (i >= ninst) return;
 	const GalaxyDev &g = gals[insts[i].galaxy];
-	// Neumaier-compensated sum of the block partials
+	// Neumaier-compensated sum of the block partials, per lane and then across
+	// the lanes (the compensations add up beside the sums)
 	double s = 0, comp = 0;
-	for (int b = lk_off[i]; b < lk_off[i + 1]; ++b) {
-		const double v = partial[b];
+	auto add = [&](double v) {
 		const double tsum = s + v;
 		if (fabs(s) >= fabs(v)) comp += (s - tsum) + v;
 		else comp += (v - tsum) + s;
 		s = tsum;
+	};
+	for (int b = lk_off[i] + lane; b < lk_off[i + 1]; b += 64) add(partial[b]);
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1) {
+		const double s2 = __shfl_xor(s, o), c2 = __shfl_xor(comp, o);
+		comp += c2;
+		add(s2);
 	}
 	const double X = s + comp;
 	const double N = g.n_region;
@@ -816,8 +820,10 @@ __global__ void k_like_finalize(const GalaxyDev *__restrict__ gals, const InstDe
 		break;
 	default: L = NAN; break;
 	}
-	ll[i] = L;
-	gscale[i] = gsc;
+	if (lane == 0) {
+		ll[i] = L;
+		gscale[i] = gsc;
+	}
 }
 
 // Adjoint weight of canvas pixel (x, y) for a component drawn into the
@@ -974,13 +980,23 @@ __global__ __launch_bounds__(256) void k_adj_nonradial(const GalaxyDev *__restri
 	}
 }
 
-__global__ void k_grad_finalize(const Comp *__restrict__ comps, const double *__restrict__ gscale,
-                                const double *__restrict__ grad_acc, double *grad_out, int ncomp, unsigned slot_mask)
+// The evaluation's results, written straight to pinned host memory: logL of
+// every instance, the scaled gradient (where given), the set-up errors and the
+// work-list counters.  One launch in place of the gradient's scaling and up to
+// four copies of 5 us each.
+__global__ __launch_bounds__(256) void k_report(const Comp *__restrict__ comps, const double *__restrict__ gscale,
+                                                const double *__restrict__ grad_acc, const double *__restrict__ ll,
+                                                const int *__restrict__ errors, const int *__restrict__ qcount,
+                                                int ncomp, int ninst, unsigned slot_mask, HostReport out)
 {
 	const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-	if (idx >= ncomp * NGRAD) return;
-	const int c = idx / NGRAD, s = idx - c * NGRAD;
-	grad_out[idx] = ((slot_mask >> s) & 1u) ? gscale[comps[c].instance] * grad_acc[idx] : 0.0;
+	if (out.grad && idx < ncomp * NGRAD) {
+		const int c = idx / NGRAD, s = idx - c * NGRAD;
+		out.grad[idx] = ((slot_mask >> s) & 1u) ? gscale[comps[c].instance] * grad_acc[idx] : 0.0;
+	}
+	if (out.ll && idx < ninst) out.ll[idx] = ll[idx];
+	if (idx < ncomp) out.errors[idx] = errors[idx];
+	if (idx < kQueueCounters) out.qcount[idx] = qcount[idx];
 }
 
 // ------------------------------------------------------------------ masks
@@ -1018,11 +1034,12 @@ __global__ void k_dilate_cols(const uint8_t *__restrict__ in, uint8_t *out, int 
 	} while (0)
 
 int launch_setup(const ProfileParams *params, const int *order, const int *comp_inst, const InstDev *insts,
-                 const GalaxyDev *gals, Comp *comps, int *errors, int ncomp, hipStream_t st)
+                 const GalaxyDev *gals, Comp *comps, int *errors, int ncomp, int *qcount, double *grad_acc,
+                 hipStream_t st)
 {
-	if (ncomp <= 0) return 0;
-	k_setup<<<(unsigned)(((long)ncomp * 64 + 255) / 256), 256, 0, st>>>(params, order, comp_inst, insts, gals, comps,
-	                                                                   errors, ncomp);
+	if (ncomp <= 0 && !qcount) return 0;
+	k_setup<<<(unsigned)(((long)std::max(ncomp, 1) * 64 + 255) / 256), 256, 0, st>>>(
+	    params, order, comp_inst, insts, gals, comps, errors, ncomp, qcount, grad_acc);
 	return (int)hipGetLastError();
 }
 
@@ -1030,20 +1047,6 @@ int launch_setup_grad(const int *order, Comp *comps, const int *errors, int ncom
 {
 	if (ncomp <= 0) return 0;
 	k_setup_grad<<<(unsigned)(((long)ncomp * 5 * 64 + 255) / 256), 256, 0, st>>>(order, comps, errors, ncomp);
-	return (int)hipGetLastError();
-}
-
-int launch_zero_d(double *p, long n, hipStream_t st)
-{
-	if (n <= 0) return 0;
-	k_fill_zero_d<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(p, n);
-	return (int)hipGetLastError();
-}
-
-int launch_zero_i(int *p, long n, hipStream_t st)
-{
-	if (n <= 0) return 0;
-	k_fill_zero_i<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(p, n);
 	return (int)hipGetLastError();
 }
 
@@ -1127,7 +1130,7 @@ int launch_like_finalize(const GalaxyDev *gals, const InstDev *insts, const int 
                          const double *partial, double *ll, double *gscale, hipStream_t st)
 {
 	if (ninst <= 0) return 0;
-	k_like_finalize<<<(ninst + 63) / 64, 64, 0, st>>>(gals, insts, lk_off, ninst, partial, ll, gscale);
+	k_like_finalize<<<(ninst + 3) / 4, 256, 0, st>>>(gals, insts, lk_off, ninst, partial, ll, gscale);
 	return (int)hipGetLastError();
 }
 
@@ -1147,12 +1150,11 @@ int launch_like_t(const GalaxyDev *gals, const InstDev *insts, int ninst, int gr
 	return (int)hipGetLastError();
 }
 
-int launch_grad_finalize(const Comp *comps, const double *gscale, const double *grad_acc, double *grad_out,
-                         int ncomp, unsigned slot_mask, hipStream_t st)
+int launch_report(const Comp *comps, const double *gscale, const double *grad_acc, const double *ll, const int *errors,
+                  const int *qcount, int ncomp, int ninst, unsigned slot_mask, const HostReport &out, hipStream_t st)
 {
-	if (ncomp <= 0) return 0;
-	const int n = ncomp * NGRAD;
-	k_grad_finalize<<<(n + 255) / 256, 256, 0, st>>>(comps, gscale, grad_acc, grad_out, ncomp, slot_mask);
+	const int n = std::max({out.grad ? ncomp * NGRAD : ncomp, ninst, kQueueCounters});
+	k_report<<<(n + 255) / 256, 256, 0, st>>>(comps, gscale, grad_acc, ll, errors, qcount, ncomp, ninst, slot_mask, out);
 	return (int)hipGetLastError();
 }
 
