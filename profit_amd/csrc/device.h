@@ -146,4 +146,10 @@ struct HostReport {
 	int *errors, *qcount;
 };
 
+// How a brute-force launch of few tiles fills the GPU: each tile's rows in
+// `parts` blocks (one likelihood partial each), kernel columns in `slices`.
+struct ConvSplit {
+	int parts = 1, slices = 1;
+};
+
 }  // namespace profit_amd

@@ -377,7 +377,7 @@ void Engine::conv_forward(int mode, hipStream_t st)
 	const int *lk = d_lk_off_.as<int>();
 	if (mode == 0) {
 		hip_check(launch_conv(CONV_LIKE, conv_rows_, n_ct_blocks_, kx_max_, kc_max_, gals, insts, d_ct_off_.as<int>(),
-		                      n, lk, partial, st),
+		                      n, lk, partial, st, split_like_),
 		          "conv");
 		hip_check(launch_conv_mfma(CONV_LIKE, ml_off_[n], mfma_pitch_, mfma_kch_, gals, insts, d_ml_off_.as<int>(), n,
 		                           lk, partial, st),
@@ -385,7 +385,7 @@ void Engine::conv_forward(int mode, hipStream_t st)
 	}
 	else {
 		hip_check(launch_conv(CONV_MODEL, conv_rows_, n_bt_blocks_, kx_max_, kc_max_, gals, insts, d_bt_off_.as<int>(),
-		                      n, lk, partial, st),
+		                      n, lk, partial, st, split_canvas_),
 		          "conv");
 		hip_check(launch_conv_mfma(CONV_MODEL, mc_off_[n], mfma_pitch_, mfma_kch_, gals, insts, d_mc_off_.as<int>(), n,
 		                           lk, partial, st),
@@ -425,7 +425,7 @@ void Engine::conv_adjoint(hipStream_t st)
 	const InstDev *insts = d_insts_.as<InstDev>();
 	const int *lk = d_lk_off_.as<int>();
 	hip_check(launch_conv(CONV_ADJ, conv_rows_, n_bt_blocks_, kx_max_, kc_max_, gals, insts, d_bt_off_.as<int>(), n, lk,
-	                      nullptr, st),
+	                      nullptr, st, split_canvas_),
 	          "adjoint conv");
 	hip_check(launch_conv_mfma(CONV_ADJ, mc_off_[n], mfma_pitch_, mfma_kch_, gals, insts, d_mc_off_.as<int>(), n, lk,
 	                           nullptr, st),
@@ -874,6 +874,7 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 		if (mfma_kch_ < 1) throw std::invalid_argument("PSF too wide for the split-BF16x3 convolution");
 	}
 	fft_cb_ = fft_cols_per_block(std::max(fft_nmax2_, 2));
+	split_like_ = conv_split(conv_rows_, n_ct_blocks_);
 	for (int i = 0; i < n; ++i) {
 		const GalaxyDev &g = gal_host_[inst_galaxy[i]];
 		const bool f = g.conv_kind == CK_FFT;
@@ -884,7 +885,7 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 		// columns span the half-spectrum
 		const int rpb = f ? 2 * fft_pairs_per_block(g.fft_n1) : 2;
 		auto row_blocks = [rpb](int rows) { return (rows + rpb - 1) / rpb; };
-		lk_off_[i + 1] = lk_off_[i] + (g.conv_kind == CK_VALU   ? g.n_ctiles
+		lk_off_[i + 1] = lk_off_[i] + (g.conv_kind == CK_VALU   ? g.n_ctiles * split_like_.parts
 		                               : g.conv_kind == CK_MFMA ? g.n_mtl
 		                                                        : row_blocks(g.H));
 		rf0_off_[i + 1] = rf0_off_[i] + (f ? row_blocks(g.DH) : 0);
@@ -894,6 +895,7 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 		ri1_off_[i + 1] = ri1_off_[i] + (f ? row_blocks(g.DH) : 0);
 	}
 	n_bt_blocks_ = bt_off_[n];
+	split_canvas_ = conv_split(conv_rows_, n_bt_blocks_);
 	// the renders give each thread about 32 canvas pixels of a component where
 	// that leaves 2,048 blocks (eight a CU), and fewer otherwise (a block's
 	// first pixel waits for a chain of loads, and the adjoint pays a reduction

@@ -39,8 +39,12 @@ int launch_adj_queue(int type, int nblocks, const InstDev *insts, const Comp *co
                      hipStream_t st);
 int launch_subsample_nodes(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
                            WorkQueue wq, int *nodes, hipStream_t st);
+// parts until there is a block per CU (two rows a thread at the least), four
+// slices below two blocks per CU
+ConvSplit conv_split(int rows, int nblocks);
 int launch_conv(int mode, int rows, int nblocks, int kx_max, int kc, const GalaxyDev *gals, const InstDev *insts,
-                const int *tile_off, int ninst, const int *lk_base, double *partial, hipStream_t st);
+                const int *tile_off, int ninst, const int *lk_base, double *partial, hipStream_t st,
+                ConvSplit split = ConvSplit{});
 int launch_like_finalize(const GalaxyDev *gals, const InstDev *insts, const int *lk_off, int ninst,
                          const double *partial, double *ll, double *gscale, hipStream_t st);
 int launch_adj_nonradial(const GalaxyDev *gals, const InstDev *insts, int ninst, const Comp *comps, double *grad_acc,
@@ -285,6 +289,7 @@ class Engine {
 	// galaxy's PSF spectrum columns (and pixel data) in the L2
 	DevBuf d_col_blk_, d_ri0_blk_, d_ri1_blk_;
 	int n_bt_blocks_ = 0;
+	ConvSplit split_like_, split_canvas_;  // of the brute-force launches on the image and the canvas
 	int mfma_pitch_ = 0, mfma_kch_ = 0;
 	int fft_cb_ = 8;
 	bool render_fp64_ = false;

@@ -611,20 +611,27 @@ __global__ __launch_bounds__(256) void k_subsample_nodes(const GalaxyDev *__rest
 // thread produces R consecutive output rows of one column with a sliding
 // register window along ky and PSF weights read through the scalar cache.
 // The kernel rows are processed in chunks of at most KC rows held in LDS.
-template <int R, int MODE>
-__global__ __launch_bounds__(256) void k_conv(const GalaxyDev *__restrict__ gals, const InstDev *__restrict__ insts,
-                                              const int *__restrict__ tile_off, int ninst, int kc_max,
+//
+// A thread is a chain of Kx * Ky steps of one LDS read and R FMAs, so a launch
+// of few blocks is bound by that chain (19 tiles of a 183x201 image: 79 us, with
+// 31 x 31 taps).  Such a launch takes S = 4 slices per block, each with every
+// fourth kernel column, whose FP64 sums are added in slice order, and the tile
+// in `parts` parts of 4 R rows.
+template <int R, int MODE, int S>
+__global__ __launch_bounds__(256 * S) void k_conv(const GalaxyDev *__restrict__ gals, const InstDev *__restrict__ insts,
+                                              const int *__restrict__ tile_off, int ninst, int kc_max, int parts,
                                               const int *__restrict__ lk_base, double *partial)
 {
-	extern __shared__ float lds[];
-	const int b = blockIdx.x;
+	extern __shared__ __align__(16) float lds[];
+	const int b = blockIdx.x / parts, part_y = blockIdx.x - b * parts;
 	const int inst = owner_of(tile_off, ninst, b);
 	const InstDev I = insts[inst];
 	const GalaxyDev &g = gals[I.galaxy];
 	const int2 t = (MODE == CONV_LIKE) ? g.ctiles[b - tile_off[inst]] : g.atiles[b - tile_off[inst]];
 	const int Kx = g.Kx, Ky = g.Ky;
-	const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-	const int x0 = t.x * kTileW, y0 = t.y * 4 * R;
+	const int tx = threadIdx.x & 63, ty = (threadIdx.x >> 6) & 3;
+	const int slice = S == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+	const int x0 = t.x * kTileW, y0 = (t.y * parts + part_y) * 4 * R;
 
 	const float *__restrict__ in;
 	const float *__restrict__ wt;
@@ -669,7 +676,7 @@ __global__ __launch_bounds__(256) void k_conv(const GalaxyDev *__restrict__ gals
 		const int LH = 4 * R + kc - 1;
 		__syncthreads();
 		const int gy0 = y0 + oy + ky0, gx0 = x0 + ox;
-		for (int idx = threadIdx.x; idx < LH * LW; idx += 256) {
+		for (int idx = threadIdx.x; idx < LH * LW; idx += 256 * S) {
 			const int rr = idx / LW, cc = idx - rr * LW;
 			const int gy = gy0 + rr, gx = gx0 + cc;
 			float v = 0.f;
@@ -678,7 +685,7 @@ __global__ __launch_bounds__(256) void k_conv(const GalaxyDev *__restrict__ gals
 		}
 		__syncthreads();
 		const float *colbase = lds + ty * R * LW + tx;
-		for (int kx = 0; kx < Kx; ++kx) {
+		for (int kx = slice; kx < Kx; kx += S) {
 			const float *col = colbase + kx;
 			const float *wcol = wt + (long)ky0 * Kx + kx;
 			float part[R];
@@ -707,6 +714,22 @@ __global__ __launch_bounds__(256) void k_conv(const GalaxyDev *__restrict__ gals
 		}
 	}
 
+	if constexpr (S > 1) {
+		// the slices' sums, in slice order
+		double *sums = reinterpret_cast<double *>(lds);
+		const int tid = threadIdx.x & 255;
+		__syncthreads();
+		if (slice) {
+#pragma unroll
+			for (int r = 0; r < R; ++r) sums[((slice - 1) * R + r) * 256 + tid] = acc[r];
+		}
+		__syncthreads();
+		if (!slice) {
+#pragma unroll
+			for (int r = 0; r < R; ++r)
+				for (int k = 0; k < S - 1; ++k) acc[r] += sums[(k * R + r) * 256 + tid];
+		}
+	}
 	const int oxx = x0 + tx;
 	if (MODE == CONV_LIKE) {
 		double part = 0;
@@ -715,7 +738,7 @@ __global__ __launch_bounds__(256) void k_conv(const GalaxyDev *__restrict__ gals
 #pragma unroll
 		for (int r = 0; r < R; ++r) {
 			const int oyy = y0 + ty * R + r;
-			if (oxx < OW && oyy < OH) {
+			if (slice == 0 && oxx < OW && oyy < OH) {
 				const long o = (long)oyy * OW + oxx;
 				float wv = 0.f;
 				if (g.region[o]) {
@@ -748,16 +771,17 @@ __global__ __launch_bounds__(256) void k_conv(const GalaxyDev *__restrict__ gals
 		}
 		__shared__ double red[4];
 		part = wave_sum(part);
-		if (tx == 0) red[ty] = part;
+		if (tx == 0 && slice == 0) red[ty] = part;
 		__syncthreads();
-		if (threadIdx.x == 0) partial[lk_base[inst] + (b - tile_off[inst])] = (red[0] + red[1]) + (red[2] + red[3]);
+		if (threadIdx.x == 0)
+			partial[lk_base[inst] + (b - tile_off[inst]) * parts + part_y] = (red[0] + red[1]) + (red[2] + red[3]);
 	}
 	else {
 		float *out = I.G;
 #pragma unroll
 		for (int r = 0; r < R; ++r) {
 			const int oyy = y0 + ty * R + r;
-			if (oxx < OW && oyy < OH) {
+			if (slice == 0 && oxx < OW && oyy < OH) {
 				const long o = (long)oyy * OW + oxx;
 				float v = (float)acc[r];
 				if (MODE == CONV_MODEL && g.canvas64) v = (float)I.canvas64[o];
@@ -1093,30 +1117,46 @@ int launch_subsample_nodes(int nblocks, const GalaxyDev *gals, const InstDev *in
 	return (int)hipGetLastError();
 }
 
-template <int R, int MODE>
+template <int R, int MODE, int S>
 static int conv_launch(int nblocks, size_t lds, const GalaxyDev *gals, const InstDev *insts, const int *tile_off,
-                       int ninst, int kc, const int *lk_base, double *partial, hipStream_t st)
+                       int ninst, int kc, int parts, const int *lk_base, double *partial, hipStream_t st)
 {
+	if (S > 1) lds = std::max(lds, sizeof(double) * (S - 1) * R * 256);
+	if (lds > 160 * 1024) return (int)hipErrorInvalidValue;
 	if (lds > 64 * 1024) {
-		PA_CHECK(hipFuncSetAttribute((const void *)k_conv<R, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+		PA_CHECK(hipFuncSetAttribute((const void *)k_conv<R, MODE, S>, hipFuncAttributeMaxDynamicSharedMemorySize,
 		                             (int)lds));
 	}
-	k_conv<R, MODE><<<nblocks, 256, lds, st>>>(gals, insts, tile_off, ninst, kc, lk_base, partial);
+	k_conv<R, MODE, S><<<nblocks * parts, 256 * S, lds, st>>>(gals, insts, tile_off, ninst, kc, parts, lk_base, partial);
 	return (int)hipGetLastError();
 }
 
+ConvSplit conv_split(int rows, int nblocks)
+{
+	ConvSplit p;
+	while (nblocks * p.parts < 256 && rows / p.parts > 2) p.parts *= 2;
+	p.slices = nblocks * p.parts < 512 ? 4 : 1;
+	return p;
+}
+
 int launch_conv(int mode, int rows, int nblocks, int kx_max, int kc, const GalaxyDev *gals, const InstDev *insts,
-                const int *tile_off, int ninst, const int *lk_base, double *partial, hipStream_t st)
+                const int *tile_off, int ninst, const int *lk_base, double *partial, hipStream_t st, ConvSplit split)
 {
 	if (nblocks <= 0) return 0;
-	const size_t lds = sizeof(float) * (size_t)(4 * rows + kc - 1) * (size_t)(kTileW + kx_max - 1);
-	if (lds > 160 * 1024) return (int)hipErrorInvalidValue;
-#define PA_CONV_CASE(RR)                                                                                  \
-	case RR:                                                                                              \
-		if (mode == CONV_LIKE) return conv_launch<RR, CONV_LIKE>(nblocks, lds, gals, insts, tile_off, ninst, kc, lk_base, partial, st); \
-		if (mode == CONV_MODEL) return conv_launch<RR, CONV_MODEL>(nblocks, lds, gals, insts, tile_off, ninst, kc, lk_base, partial, st); \
-		return conv_launch<RR, CONV_ADJ>(nblocks, lds, gals, insts, tile_off, ninst, kc, lk_base, partial, st);
-	switch (rows) {
+	const int r = rows / split.parts;
+	if (r * split.parts != rows) return (int)hipErrorInvalidValue;
+	const size_t lds = sizeof(float) * (size_t)(4 * r + kc - 1) * (size_t)(kTileW + kx_max - 1);
+#define PA_CONV_MODE(RR, SS)                                                                                    \
+	if (mode == CONV_LIKE) return conv_launch<RR, CONV_LIKE, SS>(nblocks, lds, gals, insts, tile_off, ninst, kc, split.parts, lk_base, partial, st); \
+	if (mode == CONV_MODEL) return conv_launch<RR, CONV_MODEL, SS>(nblocks, lds, gals, insts, tile_off, ninst, kc, split.parts, lk_base, partial, st); \
+	return conv_launch<RR, CONV_ADJ, SS>(nblocks, lds, gals, insts, tile_off, ninst, kc, split.parts, lk_base, partial, st);
+#define PA_CONV_CASE(RR)               \
+	case RR:                           \
+		if (split.slices == 4) {       \
+			PA_CONV_MODE(RR, 4)        \
+		}                              \
+		PA_CONV_MODE(RR, 1)
+	switch (r) {
 		PA_CONV_CASE(2)
 		PA_CONV_CASE(4)
 		PA_CONV_CASE(8)
@@ -1124,6 +1164,7 @@ int launch_conv(int mode, int rows, int nblocks, int kx_max, int kc, const Galax
 	default: return (int)hipErrorInvalidValue;
 	}
 #undef PA_CONV_CASE
+#undef PA_CONV_MODE
 }
 
 int launch_like_finalize(const GalaxyDev *gals, const InstDev *insts, const int *lk_off, int ninst,
