@@ -1134,7 +1134,7 @@ void Engine::launch_walkers_fwd(int split, bool jac, hipStream_t st)
 	for (int t = 0; t < 6; ++t)
 		if ((radial_types_ >> t) & 1u)
 			hip_check(launch_subsample_fwd(t, subsample_blocks_, d_gals_.as<GalaxyDev>(), d_insts_.as<InstDev>(),
-			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, st),
+			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, ncomp_total_, st),
 			          "subsample");
 }
 

@@ -32,9 +32,10 @@ int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *grp_of
 // (and per sum precision in the adjoint render: 1 = FP64 per-thread sums,
 // steep cores only).  jac: the forward walk also writes each entry's Jacobian
 // (wq.ljac, wq.hjac), which launch_adj_queue weighs by G(q).  mask: the trees
-// by the mask walk (after a tree overflowed the tree walk's stack).
+// by the mask walk (after a tree overflowed the tree walk's stack).  ncomp: the
+// batch's components.
 int launch_subsample_fwd(int type, int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
-                         WorkQueue wq, int split, bool jac, bool mask, hipStream_t st);
+                         WorkQueue wq, int split, bool jac, bool mask, int ncomp, hipStream_t st);
 int launch_adj_queue(int type, int nblocks, const InstDev *insts, const Comp *comps, WorkQueue wq, double *grad_acc,
                      hipStream_t st);
 int launch_subsample_nodes(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,

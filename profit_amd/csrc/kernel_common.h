@@ -696,21 +696,23 @@ __global__ __launch_bounds__(256) void k_subsample_root(const GalaxyDev *__restr
 
 // ------------------------------------------------------------------ trees
 
-// The pending nodes of the trees a block walks, in LDS: wavefront w's quarter
-// holds kTreeQuarter of them (its own stack while each wavefront walks a tree
-// of its own; a quarter of the block's while the block walks one together).
-constexpr int kTreeQuarter = 256;
+// The pending nodes of the trees a block of W wavefronts walks, in LDS:
+// wavefront w's share holds kTreeShare of them (its own stack while each
+// wavefront walks a tree of its own; a part of the block's while the block
+// walks one together).
+constexpr int kTreeShare = 256;
+template <int W>
 struct TreeStack {
-	struct Quarter {
-		double x0[kTreeQuarter], x1[kTreeQuarter], y0[kTreeQuarter], y1[kTreeQuarter], weight[kTreeQuarter];
-		uint8_t level[kTreeQuarter];
-	} q[4];
-	int count[2][4];  // refined cells per wavefront of a round, double-buffered
+	struct Share {
+		double x0[kTreeShare], x1[kTreeShare], y0[kTreeShare], y1[kTreeShare], weight[kTreeShare];
+		uint8_t level[kTreeShare];
+	} q[W];
+	int count[2][W];  // refined cells per wavefront of a round, double-buffered
 };
 
 // Walks the recursion tree of one pixel of a TYPE profile with T threads (a
-// wavefront, T = 64, or a block of four, T = 256), starting from stack slot
-// `base` (T = 64: the wavefront's quarter).  A round takes as many pending
+// wavefront, T = 64, or the block of W wavefronts, T = 64 W), starting from
+// stack slot `base` (T = 64: the wavefront's share).  A round takes as many pending
 // nodes off the stack as T threads have cells for, one cell per thread (a node
 // of more cells alone, its cells T at a time); a cell to be refined pushes its
 // own FP64 node bounds (libprofit's additions).  Every thread returns its share
@@ -721,11 +723,12 @@ struct TreeStack {
 // `top`, `n` and `total` are equal on all T threads, so all take the same
 // barriers; each round removes a node and a node's children lie one level
 // deeper (at most maxrec), so the rounds end.
-template <int TYPE, bool kJac, int T>
-__device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack &S, int base, int tid, double x0, double x1,
+template <int TYPE, bool kJac, int T, int W>
+__device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack<W> &S, int base, int tid, double x0, double x1,
                                           double y0, double y1, int res, int maxrec, bool fp64, double &sum, float *gj)
 {
-	constexpr int cap = T == 64 ? kTreeQuarter : 4 * kTreeQuarter;
+	static_assert(T == 64 || T == 64 * W, "a wavefront or the block");
+	constexpr int cap = (T / 64) * kTreeShare;
 	const bool fuse = kJac && TYPE == SERSIC && !c.boxy && !c.grad_box;
 	const int ncell = res * res, wv = tid >> 6, lane = tid & 63;
 	const double inv_cells = kInvCells[res];
@@ -734,8 +737,8 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack &S, int base,
 	const int slot = ncell >= T ? 0 : tid / ncell;
 	const int cell0 = tid - slot * ncell;
 	auto put = [&](int at, double a, double b, double d, double e, double w, int level) {
-		TreeStack::Quarter &q = S.q[(base + at) / kTreeQuarter];
-		const int k = (base + at) % kTreeQuarter;
+		typename TreeStack<W>::Share &q = S.q[(base + at) / kTreeShare];
+		const int k = (base + at) % kTreeShare;
 		q.x0[k] = a;
 		q.x1[k] = b;
 		q.y0[k] = d;
@@ -759,8 +762,8 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack &S, int base,
 		const int n = min(per, top);
 		const bool on = slot < n;
 		const int r = base + top - 1 - (on ? slot : 0);
-		const TreeStack::Quarter &Q = S.q[r / kTreeQuarter];
-		const int k = r % kTreeQuarter;
+		const typename TreeStack<W>::Share &Q = S.q[r / kTreeShare];
+		const int k = r % kTreeShare;
 		const Node node = make_node(c, Q.x0[k], Q.x1[k], Q.y0[k], Q.y1[k], res);
 		const double weight = Q.weight[k];
 		const int level = Q.level[k];
@@ -772,12 +775,12 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack &S, int base,
 			const bool fail = on && cell < ncell && cell_step<TYPE, kJac>(c, node, cell, recurse, fp64, fuse, weight, sum, gj);
 			const unsigned long long m = __ballot(fail);
 			int off = __popcll(m & ((1ull << lane) - 1ull)), total = __popcll(m);
-			if constexpr (T == 256) {
+			if constexpr (T > 64) {
 				// every thread has read its node before a push may overwrite it
 				if (lane == 0) S.count[buf][wv] = total;
 				__syncthreads();
 				total = 0;
-				for (int w = 0; w < 4; ++w) {
+				for (int w = 0; w < W; ++w) {
 					const int v = S.count[buf][w];
 					off += w < wv ? v : 0;
 					total += v;
@@ -810,18 +813,19 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack &S, int base,
 //
 // A centre tree (res 8, depth 10: 160 nodes, 16 a level) is a chain of levels:
 // one wavefront walking its nodes in turn took 220 to 300 us, whatever the
-// batch; four share each level.
-template <int TYPE, bool kJac>
-__global__ __launch_bounds__(256, 3) void k_subsample_tree(const GalaxyDev *__restrict__ gals,
+// batch.  W = 4 wavefronts share each level (four rounds of 1.5 us, three blocks
+// a CU) where there are trees for all blocks, W = 8 where there are not.
+template <int TYPE, bool kJac, int W>
+__global__ __launch_bounds__(64 * W, W == 4 ? 3 : 2) void k_subsample_tree(const GalaxyDev *__restrict__ gals,
                                                            const InstDev *__restrict__ insts,
                                                            const Comp *__restrict__ comps, WorkQueue wq, int split)
 {
 	constexpr int kSlots = G_S0 + n_shape(TYPE), kJacPitch = 68;
-	__shared__ __align__(16) TreeStack S;
-	__shared__ double red[4][16];
+	__shared__ __align__(16) TreeStack<W> S;
+	__shared__ double red[W][16];
 	static_assert(kSlots < kJacStride && kSlots + 1 <= 16, "Jacobian slots and the value");
-	static_assert(sizeof(float) * kSlots * kJacPitch <= sizeof(TreeStack::Quarter), "a wavefront's rows fit its quarter");
-	static_assert(sizeof(TreeStack::Quarter) % 16 == 0, "a wavefront's rows are 16-byte aligned");
+	static_assert(sizeof(float) * kSlots * kJacPitch <= sizeof(typename TreeStack<W>::Share), "a wavefront's rows fit its share");
+	static_assert(sizeof(typename TreeStack<W>::Share) % 16 == 0, "a wavefront's rows are 16-byte aligned");
 	const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int lb = wq.lbase[TYPE], cap = wq.lbase[TYPE + 1] - lb;
 	const int nd = min(wq.count[deep_count(TYPE)], cap), nb = min(wq.count[big_count(TYPE)], cap);
@@ -829,7 +833,7 @@ __global__ __launch_bounds__(256, 3) void k_subsample_tree(const GalaxyDev *__re
 	float gj[NGRAD];
 	double sum;
 	// the thread's sums of its wavefront: lane s < kSlots of the wavefront
-	// returns slot s, lane 15 the value (the wavefront's quarter as scratch:
+	// returns slot s, lane 15 the value (the wavefront's share as scratch:
 	// the walk is over)
 	auto wave_totals = [&]() {
 		float *R = reinterpret_cast<float *>(&S.q[wv]);
@@ -886,7 +890,7 @@ __global__ __launch_bounds__(256, 3) void k_subsample_tree(const GalaxyDev *__re
 		const double y = hy + j * g.sx, x = hx + i * g.sy;
 		const bool centre = centre_pixel(c, x, y);
 		clear();
-		const bool ok = walk_tree<TYPE, kJac, 256>(c, S, 0, threadIdx.x, x - hx, x + hx, y - hy, y + hy,
+		const bool ok = walk_tree<TYPE, kJac, 64 * W>(c, S, 0, threadIdx.x, x - hx, x + hx, y - hy, y + hy,
 		                                           centre ? 8 : c.res, centre ? 10 : c.maxrec, g.render_fp64 != 0, sum, gj);
 		if (ok) {
 			const double w = wave_totals();
@@ -897,12 +901,14 @@ __global__ __launch_bounds__(256, 3) void k_subsample_tree(const GalaxyDev *__re
 		}
 		__syncthreads();
 		if (ok && wv == 0) {
-			const int s = lane & 15;
-			finish(q, c, I, g, heavy, e, (red[0][s] + red[1][s]) + (red[2][s] + red[3][s]));
+			double v = 0;
+#pragma unroll
+			for (int w = 0; w < W; ++w) v += red[w][lane & 15];
+			finish(q, c, I, g, heavy, e, v);
 		}
 		__syncthreads();
 	}
-	for (int t = blockIdx.x * 4 + wv; t < nd; t += gridDim.x * 4) {
+	for (int t = blockIdx.x * W + wv; t < nd; t += gridDim.x * W) {
 		const int e = wq.deep[lb + t];
 		const QEntry q = wq.light[lb + e];
 		const Comp &c = comps[q.comp];
@@ -912,7 +918,7 @@ __global__ __launch_bounds__(256, 3) void k_subsample_tree(const GalaxyDev *__re
 		const double hx = g.sx / 2., hy = g.sy / 2.;
 		const double y = hy + j * g.sx, x = hx + i * g.sy;
 		clear();
-		if (walk_tree<TYPE, kJac, 64>(c, S, wv * kTreeQuarter, lane, x - hx, x + hx, y - hy, y + hy, c.res, c.maxrec,
+		if (walk_tree<TYPE, kJac, 64>(c, S, wv * kTreeShare, lane, x - hx, x + hx, y - hy, y + hy, c.res, c.maxrec,
 		                              g.render_fp64 != 0, sum, gj))
 			finish(q, c, I, g, false, e, wave_totals());
 		else if (lane == 0)

@@ -5,28 +5,34 @@
 
 namespace profit_amd {
 
+constexpr int kFewComponents = 64;
+
 // The root pass over the light entries, then the tree walk over the heavy list
 // and the entries the root pass left to it (mask: the mask walk instead, one
-// wavefront per tree).  The tree walk's blocks are those that fit at three
-// wavefronts per SIMD.
+// wavefront per tree).  `few`: at most kFewComponents components, whose centre
+// trees (four each) do not reach every CU: the tree walk then takes blocks of
+// eight wavefronts, one a CU (one bulge+disk image: 53 -> 47 us), and otherwise
+// blocks of four, three a CU.
 template <int TYPE, bool kJac>
 static int fwd_launch(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps, WorkQueue wq,
-                      int split, bool mask, hipStream_t st)
+                      int split, bool mask, bool few, hipStream_t st)
 {
 	k_subsample_root<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, split, mask ? 0 : 1);
 	if (mask) k_subsample<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, fwd_counter(TYPE), split);
-	else k_subsample_tree<TYPE, kJac><<<(nblocks * 3 + 7) / 8, 256, 0, st>>>(gals, insts, comps, wq, split);
+	else if (few) k_subsample_tree<TYPE, kJac, 8><<<(nblocks + 7) / 8, 512, 0, st>>>(gals, insts, comps, wq, split);
+	else k_subsample_tree<TYPE, kJac, 4><<<(nblocks * 3 + 7) / 8, 256, 0, st>>>(gals, insts, comps, wq, split);
 	return (int)hipGetLastError();
 }
 
 int launch_subsample_fwd(int type, int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
-                         WorkQueue wq, int split, bool jac, bool mask, hipStream_t st)
+                         WorkQueue wq, int split, bool jac, bool mask, int ncomp, hipStream_t st)
 {
 	if (nblocks <= 0) return 0;
+	const bool few = ncomp <= kFewComponents;
 #define PA_FWD(T)                                                                                        \
 	case T:                                                                                              \
-		return jac ? fwd_launch<T, true>(nblocks, gals, insts, comps, wq, split, mask, st)               \
-		           : fwd_launch<T, false>(nblocks, gals, insts, comps, wq, split, mask, st)
+		return jac ? fwd_launch<T, true>(nblocks, gals, insts, comps, wq, split, mask, few, st)               \
+		           : fwd_launch<T, false>(nblocks, gals, insts, comps, wq, split, mask, few, st)
 	switch (type) {
 		PA_FWD(SERSIC);
 		PA_FWD(MOFFAT);

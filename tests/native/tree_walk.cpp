@@ -40,8 +40,6 @@ template <class A, class B> static long min(A a, B b) { return (long)a < (long)b
 
 using namespace profit_amd;
 
-static TreeStack *S;
-
 template <int TYPE>
 static void recurse(const Comp &c, double x0, double x1, double y0, double y1, double w, int res, int maxrec, int level,
                     double &sum, float *gj, long &leaves)
@@ -67,8 +65,9 @@ static bool check(const char *name, ProfileParams p, double px, double py, int r
 	p.type = TYPE;
 	if (setup_component(p, 0, 1, 1, 1, 1, 0, 0, &qs, &c) != SE_OK) return false;
 	c.grad_box = 0;
+	constexpr int W = T == 64 ? 4 : T / 64;
 	// guard memory on both sides of the stack is the sanitizer's
-	S = new TreeStack;
+	TreeStack<W> *S = new TreeStack<W>;
 	std::vector<double> sum(T, 0.0);
 	std::vector<float> gj((size_t)T * NGRAD, 0.f);
 	std::vector<char> ok(T);
@@ -130,6 +129,8 @@ int main()
 	ok &= check<SERSIC, 64>("full16", all, 2, 1, 16, 1, false);
 	ok &= check<SERSIC, 64>("full16", all, 2, 1, 16, 2, true);
 	ok &= check<SERSIC, 256>("full16", all, 2, 1, 16, 5, true);
+	ok &= check<SERSIC, 512>("centre", cusp, 0, 0, 8, 10, false);
+	ok &= check<SERSIC, 512>("full10", all, 2, 1, 10, 1, false);
 	ok &= check<KING, 256>("king", par(KING, 0.3, 2.0, 2.0), 0, 0, 10, 3, false);
 	ok &= check<FERRER, 64>("ferrer", par(FERRER, 1.3, 1.0, 0.5), 0, 1, 6, 3, false);
 	return ok ? 0 : 1;

@@ -23,7 +23,7 @@ def test_tree_walk_equals_the_recursion(tmp_path):
     assert r.returncode == 0, r.stderr[-4000:]
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300, env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
     assert r.returncode == 0, r.stdout + r.stderr[-4000:]
-    assert r.stdout.count("ok ") == 14, r.stdout
+    assert r.stdout.count("ok ") == 16, r.stdout
 
 
 @pytest.mark.gpu
