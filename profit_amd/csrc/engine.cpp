@@ -1098,12 +1098,14 @@ bool Engine::sync_aux_flags(bool enable)
 	}
 	bool any = false, changed = false;
 	unsigned types = 0, keys = 0;
+	int family[kFamilies] = {};
 	for (int i = 0; i < ninst(); ++i) {
 		int aux = 0;
 		for (int k = 0; k < inst_ncomp_[i]; ++k) {
 			const ProfileParams &q = p[inst_comp0_[i] + k];
 			if (is_radial(q.type)) {
 				types |= 1u << q.type;
+				++family[q.type];
 				keys |= 1u << (2 * q.type + (wants_grad64(q) ? 1 : 0));
 				continue;
 			}
@@ -1118,7 +1120,9 @@ bool Engine::sync_aux_flags(bool enable)
 			changed = true;
 		}
 	}
-	if (any != any_nonradial_ || types != radial_types_ || keys != grad_keys_) {
+	if (any != any_nonradial_ || types != radial_types_ || keys != grad_keys_ ||
+	    std::memcmp(family, family_comps_, sizeof(family)) != 0) {
+		std::memcpy(family_comps_, family, sizeof(family));
 		any_nonradial_ = any;
 		radial_types_ = types;
 		grad_keys_ = keys;
@@ -1134,7 +1138,7 @@ void Engine::launch_walkers_fwd(int split, bool jac, hipStream_t st)
 	for (int t = 0; t < 6; ++t)
 		if ((radial_types_ >> t) & 1u)
 			hip_check(launch_subsample_fwd(t, subsample_blocks_, d_gals_.as<GalaxyDev>(), d_insts_.as<InstDev>(),
-			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, ncomp_total_, st),
+			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, family_comps_[t], st),
 			          "subsample");
 }
 

@@ -33,7 +33,7 @@ int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *grp_of
 // steep cores only).  jac: the forward walk also writes each entry's Jacobian
 // (wq.ljac, wq.hjac), which launch_adj_queue weighs by G(q).  mask: the trees
 // by the mask walk (after a tree overflowed the tree walk's stack).  ncomp: the
-// batch's components.
+// batch's components of the family.
 int launch_subsample_fwd(int type, int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
                          WorkQueue wq, int split, bool jac, bool mask, int ncomp, hipStream_t st);
 int launch_adj_queue(int type, int nblocks, const InstDev *insts, const Comp *comps, WorkQueue wq, double *grad_acc,
@@ -316,6 +316,7 @@ class Engine {
 	// radial families present (bit t) and the adjoint's (family, precision)
 	// keys present (bit 2t + prec), which decide the walker launches
 	unsigned radial_types_ = 0, grad_keys_ = 0;
+	int family_comps_[kFamilies] = {};  // components of each radial family
 	// trees by the mask walk: set while an evaluation runs again because a
 	// tree overflowed the tree walk's stack
 	bool mask_walk_ = false;

@@ -593,8 +593,9 @@ __global__ __launch_bounds__(256, kJac && (TYPE == SERSIC || TYPE == MOFFAT || T
 // is to be refined (most pixels: 98% on a 400x400 bulge+disk) the group adds
 // the value to the canvas and, with kJac, writes the entry's Jacobian and
 // value.  An entry with a cell to refine goes to the family's deep list: to its
-// front, or, with `split_big` and from kBigTree refined cells on, to its back;
-// k_subsample_tree walks those trees from the root.
+// front, or, with `split_big` and from kBigTree refined cells or 64 cells a node
+// on, to its back; k_subsample_tree walks those trees from the root, the front's
+// with a wavefront each.
 //
 // Bound by VALU issue on long lists and by latency on short ones, so the group
 // is as wide as the list leaves room for in kRootLanes lanes (four wavefronts
@@ -628,7 +629,7 @@ __global__ __launch_bounds__(256) void k_subsample_root(const GalaxyDev *__restr
 #pragma unroll
 		for (int s = 0; s < NGRAD; ++s) gj[s] = 0.f;
 		QEntry q{-1, 0};
-		bool mine = false;
+		bool mine = false, wide = false;
 		if (e < nl) {
 			q = wq.light[lb + e];
 			const Comp &c = comps[q.comp];
@@ -643,6 +644,7 @@ __global__ __launch_bounds__(256) void k_subsample_root(const GalaxyDev *__restr
 			if (mine && centre_pixel(c, x, y)) nref = kBigTree;
 			else if (mine) {
 				const int res = c.res, ncell = res * res;
+				wide = ncell > 64;
 				const bool recurse = res > 1 && c.maxrec > 0;
 				const bool fuse = kJac && TYPE == SERSIC && !c.boxy && !c.grad_box;
 				const Node n = make_node(c, x - hx, x + hx, y - hy, y + hy, res);
@@ -680,7 +682,7 @@ __global__ __launch_bounds__(256) void k_subsample_root(const GalaxyDev *__restr
 			}
 		}
 		// the deep entries appended, one atomic per wavefront and list
-		const bool big = lead && split_big && nref >= kBigTree, deep = lead && nref > 0 && !big;
+		const bool big = lead && split_big && nref > 0 && (wide || nref >= kBigTree), deep = lead && nref > 0 && !big;
 #pragma unroll
 		for (int k = 0; k < 2; ++k) {
 			const unsigned long long m = __ballot(k ? big : deep);
@@ -804,8 +806,8 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack<W> &S, int ba
 }
 
 // The trees of a TYPE family: the centre pixels (heavy list, Sersic) and the
-// entries with kBigTree or more refined root cells (the back of the deep list),
-// a block each; then the other deep entries, a wavefront each.  Adds flux_scale
+// entries with kBigTree or more refined root cells or more than 64 cells a node
+// (the back of the deep list), a block each; then the other deep entries, a wavefront each.  Adds flux_scale
 // * value to the canvas (or the aux canvas, or the FP64 canvas) and, with kJac,
 // writes the entry's Jacobian and value.  Entries are dealt out by index; an
 // overflowing tree is counted in count[0] and the evaluation runs again with
@@ -813,10 +815,12 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack<W> &S, int ba
 //
 // A centre tree (res 8, depth 10: 160 nodes, 16 a level) is a chain of levels:
 // one wavefront walking its nodes in turn took 220 to 300 us, whatever the
-// batch.  W = 4 wavefronts share each level (four rounds of 1.5 us, three blocks
-// a CU) where there are trees for all blocks, W = 8 where there are not.
+// batch; a core-Sersic pixel of resolution 16 is a chain of 300 nodes of 256
+// cells.  W = 4 wavefronts share a tree (three blocks a CU) where there are trees
+// for all blocks, W = 12 (one block a CU, the same registers) where there are
+// not.
 template <int TYPE, bool kJac, int W>
-__global__ __launch_bounds__(64 * W, W == 4 ? 3 : 2) void k_subsample_tree(const GalaxyDev *__restrict__ gals,
+__global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *__restrict__ gals,
                                                            const InstDev *__restrict__ insts,
                                                            const Comp *__restrict__ comps, WorkQueue wq, int split)
 {

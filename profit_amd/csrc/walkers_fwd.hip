@@ -5,21 +5,23 @@
 
 namespace profit_amd {
 
-constexpr int kFewComponents = 64;
+constexpr int kFewComponents = 512;
 
 // The root pass over the light entries, then the tree walk over the heavy list
 // and the entries the root pass left to it (mask: the mask walk instead, one
-// wavefront per tree).  `few`: at most kFewComponents components, whose centre
-// trees (four each) do not reach every CU: the tree walk then takes blocks of
-// eight wavefronts, one a CU (one bulge+disk image: 53 -> 47 us), and otherwise
-// blocks of four, three a CU.
+// wavefront per tree).  `few`: at most kFewComponents components of the family:
+// their big trees (four centre pixels a component, or the like) do not fill the
+// GPU, so the tree walk takes blocks of twelve wavefronts, one a CU, and
+// otherwise blocks of four, three a CU.  Four and twelve, measured: 384 survey
+// galaxies (about 150 components a family), Sersic 336 and 188 us, King 740 and
+// 711, core-Sersic 1354 and 701; one bulge+disk image 53 and 30.
 template <int TYPE, bool kJac>
 static int fwd_launch(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps, WorkQueue wq,
                       int split, bool mask, bool few, hipStream_t st)
 {
 	k_subsample_root<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, split, mask ? 0 : 1);
 	if (mask) k_subsample<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, fwd_counter(TYPE), split);
-	else if (few) k_subsample_tree<TYPE, kJac, 8><<<(nblocks + 7) / 8, 512, 0, st>>>(gals, insts, comps, wq, split);
+	else if (few) k_subsample_tree<TYPE, kJac, 12><<<(nblocks + 7) / 8, 768, 0, st>>>(gals, insts, comps, wq, split);
 	else k_subsample_tree<TYPE, kJac, 4><<<(nblocks * 3 + 7) / 8, 256, 0, st>>>(gals, insts, comps, wq, split);
 	return (int)hipGetLastError();
 }

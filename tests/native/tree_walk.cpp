@@ -129,8 +129,8 @@ int main()
 	ok &= check<SERSIC, 64>("full16", all, 2, 1, 16, 1, false);
 	ok &= check<SERSIC, 64>("full16", all, 2, 1, 16, 2, true);
 	ok &= check<SERSIC, 256>("full16", all, 2, 1, 16, 5, true);
-	ok &= check<SERSIC, 512>("centre", cusp, 0, 0, 8, 10, false);
-	ok &= check<SERSIC, 512>("full10", all, 2, 1, 10, 1, false);
+	ok &= check<SERSIC, 768>("centre", cusp, 0, 0, 8, 10, false);
+	ok &= check<SERSIC, 768>("full10", all, 2, 1, 10, 1, false);
 	ok &= check<KING, 256>("king", par(KING, 0.3, 2.0, 2.0), 0, 0, 10, 3, false);
 	ok &= check<FERRER, 64>("ferrer", par(FERRER, 1.3, 1.0, 0.5), 0, 1, 6, 3, false);
 	return ok ? 0 : 1;
