@@ -514,7 +514,7 @@ __device__ __forceinline__ bool near_cut_fp64(const Comp &c, float xp, float yp)
 
 // The profile in FP32 with the plain transcendental forms (2^(e log2 x),
 // errors of about |e log2 x| ulps): the refinement test's second value,
-// which only has to fall on the right side of a guard band of 1e-3.
+// which only has to fall on the right side of a guard band of 2.5e-4.
 template <int TYPE = -1>
 __device__ __forceinline__ float eval_fast(const Comp &c, float x, float y)
 {
