@@ -231,11 +231,12 @@ def make_model(width, height, profiles, psf=None, mask=None, magzero=0.0, scale=
     dw, dh = C.c_uint32(), C.c_uint32()
     _check(L.profit_amd_output_dims(C.byref(d), arr, len(profiles), C.byref(dw), C.byref(dh)))
     cap = max(1, dw.value * dh.value)
-    out = np.zeros(cap)
+    out = np.empty(cap)
     ow, oh, ox, oy = C.c_uint32(), C.c_uint32(), C.c_int32(), C.c_int32()
     _check(L.profit_amd_make_model(C.byref(d), arr, len(profiles), _d(out), cap, C.byref(ow),
                                    C.byref(oh), C.byref(ox), C.byref(oy)))
-    img = out[: ow.value * oh.value].reshape(oh.value, ow.value).copy()
+    n = ow.value * oh.value
+    img = (out if n == cap else out[:n].copy()).reshape(oh.value, ow.value)
     return {"image": img, "offset": (ox.value, oy.value)}
 
 

@@ -181,6 +181,16 @@ int profit_amd_convolve(int32_t convolver, const double *src, uint32_t src_w, ui
                         uint32_t krn_w, uint32_t krn_h, const uint8_t *mask, double *out, int32_t device)
 {
 	return guarded([&] {
+		// a source at least as large as its kernel needs no Image of its own
+		const int method = convolver == PROFIT_AMD_CONV_FFT            ? (int)profit_amd::CK_FFT
+		                   : convolver == PROFIT_AMD_CONV_BRUTE_BF16X3 ? (int)profit_amd::CK_MFMA
+		                                                               : (int)profit_amd::CK_VALU;
+		const bool sized = src_w >= krn_w && src_h >= krn_h && krn_w > 0 && krn_h > 0;
+		if (sized && (method != profit_amd::CK_VALU || convolver == PROFIT_AMD_CONV_BRUTE ||
+		              convolver == PROFIT_AMD_CONV_BRUTE_OLD)) {
+			profit_amd::convolve_image(src, (int)src_w, (int)src_h, krn, (int)krn_w, (int)krn_h, mask, out, device, method);
+			return;
+		}
 		profit::ConvolverCreationPreferences prefs;
 		prefs.device = device;
 		profit::ConvolverPtr c;

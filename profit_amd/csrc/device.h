@@ -152,4 +152,12 @@ struct ConvSplit {
 	int parts = 1, slices = 1;
 };
 
+// Instances [first, first + count), whose images (W * H floats each) go to
+// off[k] of a group's buffer.
+constexpr int kCropGroup = 64;
+struct CropGroup {
+	int first, count;
+	long off[kCropGroup + 1];
+};
+
 }  // namespace profit_amd

@@ -8,6 +8,9 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <list>
+#include <memory>
+#include <mutex>
 #include <sstream>
 
 namespace profit_amd {
@@ -81,6 +84,22 @@ static int next_pow2(int v)
 // FFT frame length for v points: a power of two, at least 8 (the row passes
 // fold the bit reversal into their first and last three radix-2 stages)
 static int fft_frame(int v) { return std::max(8, next_pow2(v)); }
+
+// rows per thread of the brute-force convolution of a bare image (the
+// allocation-free entry point takes the same)
+static constexpr int kImageRows = 4;
+
+// exp(-2 pi i t / n), t < n / 2
+static std::vector<double2> twiddles(int n)
+{
+	std::vector<double2> tw(n / 2);
+	const long double pi = 3.141592653589793238462643383279502884L;
+	for (int t = 0; t < n / 2; ++t) {
+		const long double a = 2 * pi * (long double)t / (long double)n;
+		tw[t] = make_double2((double)cosl(a), (double)(-sinl(a)));
+	}
+	return tw;
+}
 
 static int ilog2(int n)
 {
@@ -308,12 +327,7 @@ void Engine::ensure_fft_spectra()
 		}
 	if (twn > 4096) throw std::invalid_argument("FFT frame above 4096 points per axis is not supported");
 	if (twn != twn_) {
-		std::vector<double2> tw(twn / 2);
-		const long double pi = 3.141592653589793238462643383279502884L;
-		for (int t = 0; t < twn / 2; ++t) {
-			const long double a = 2 * pi * (long double)t / (long double)twn;
-			tw[t] = make_double2((double)cosl(a), (double)(-sinl(a)));
-		}
+		const std::vector<double2> tw = twiddles(twn);
 		d_tw_.alloc(tw.size() * sizeof(double2));
 		hip_check(hipMemcpy(d_tw_.as<double2>(), tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice), "tw");
 		twn_ = twn;
@@ -329,16 +343,10 @@ void Engine::ensure_fft_spectra()
 		g.fft_l1 = ilog2(n1);
 		g.fft_l2 = ilog2(n2);
 		const int m1 = n1 / 2 + 1;  // half-spectrum width
-		std::vector<double> frame((size_t)n1 * n2, 0.0);
-		const int ax = g.Kx - 1 - g.Kx / 2, ay = g.Ky - 1 - g.Ky / 2;
-		for (int ky = 0; ky < g.Ky; ++ky)
-			for (int kx = 0; kx < g.Kx; ++kx) {
-				const int dx = kx - ax, dy = ky - ay;
-				frame[(size_t)((dy + n2) % n2) * n1 + (dx + n1) % n1] = b.psf64[(size_t)ky * g.Kx + kx];
-			}
 		b.fft_spec.alloc((size_t)fft_pitch(n1) * n2 * sizeof(double2));
-		DevBuf src(frame.size() * sizeof(double));
-		hip_check(hipMemcpy(src.as<double>(), frame.data(), frame.size() * sizeof(double), hipMemcpyHostToDevice), "psf");
+		DevBuf krn(b.psf64.size() * sizeof(double)), src((size_t)n1 * n2 * sizeof(double));
+		hip_check(hipMemcpy(krn.as<double>(), b.psf64.data(), krn.size(), hipMemcpyHostToDevice), "psf");
+		hip_check(launch_psf_frame(krn.as<double>(), g.Kx, g.Ky, n1, n2, src.as<double>(), stream_), "psf frame");
 		g.fft_spec = b.fft_spec.as<double2>();
 		// one-instance context pointing at this galaxy
 		DevBuf dg(sizeof(GalaxyDev)), di(sizeof(InstDev));
@@ -970,11 +978,19 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 	d_gscale_.alloc(std::max(1, n) * sizeof(double));
 	d_grad_acc_.alloc((size_t)nc * NGRAD * sizeof(double));
 	d_qcount_.alloc(kQueueCounters * sizeof(int));
-	h_params_.alloc(nc * sizeof(ProfileParams));
-	h_ll_.alloc(std::max(1, n) * sizeof(double));
-	h_grad_.alloc((size_t)nc * NGRAD * sizeof(double));
-	h_err_.alloc(nc * sizeof(int));
-	h_qcount_.alloc(kQueueCounters * sizeof(int));
+	{
+		const size_t sizes[5] = {nc * sizeof(ProfileParams), std::max(1, n) * sizeof(double),
+		                         (size_t)nc * NGRAD * sizeof(double), nc * sizeof(int), kQueueCounters * sizeof(int)};
+		HostView *views[5] = {&h_params_, &h_ll_, &h_grad_, &h_err_, &h_qcount_};
+		size_t total = 0;
+		for (size_t v : sizes) total += (v + 255) / 256 * 256;
+		h_eval_.alloc(total);
+		char *at = h_eval_.as<char>();
+		for (int k = 0; k < 5; ++k) {
+			*views[k] = HostView(at);
+			at += (sizes[k] + 255) / 256 * 256;
+		}
+	}
 	for (int f = 0; f < kFamilies; ++f) lcap_[f] = 0;
 	hcap_ = 0;
 	// each family may take a third of the estimate; a list that overflows
@@ -986,6 +1002,21 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 	hipDeviceProp_t prop;
 	if (hipGetDeviceProperties(&prop, device_) == hipSuccess) ncu = prop.multiProcessorCount;
 	subsample_blocks_ = ncu * 8;
+}
+
+// the render of the whole batch into the canvas (target 0) or the aux canvas
+// (1), of the components whose convolve flag is `filter` (-1: all)
+void Engine::render(int filter, int target, hipStream_t st)
+{
+	// a batch of one radial family alone takes the render compiled for it
+	int type = -1;
+	for (int t = 0; t < kFamilies; ++t)
+		if (!any_nonradial_ && radial_types_ == (1u << t)) type = t;
+	// the render's FP64 value path only where a pixel can take it
+	const bool fp64 = render_fp64_ || canvas64_ || (radial_types_ & ((1u << KING) | (1u << FERRER)));
+	hip_check(launch_render(d_gals_.as<GalaxyDev>(), d_insts_.as<InstDev>(), d_ag_off_.as<int>(), ninst(), n_ag_blocks_,
+	                        adj_grp_, tile_parts_, d_comps_.as<Comp>(), work_queue(), filter, target, nullptr, st, type, fp64),
+	          "render");
 }
 
 void Engine::record(bool grad)
@@ -1003,15 +1034,7 @@ void Engine::record(bool grad)
 		hip_check(launch_setup_grad(d_setup_order_.as<int>(), d_comps_.as<Comp>(), d_err_.as<int>(), nc, st),
 		          "setup grad");
 	mark(1);
-	// a batch of one radial family alone takes the render compiled for it
-	int rtype = -1;
-	for (int t = 0; t < 6; ++t)
-		if (!any_nonradial_ && radial_types_ == (1u << t)) rtype = t;
-	// the render's FP64 value path only where a pixel can take it
-	const bool fp64 = render_fp64_ || canvas64_ || (radial_types_ & ((1u << KING) | (1u << FERRER)));
-	hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), n, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
-	                        work_queue(), -1, 0, nullptr, st, rtype, fp64),
-	          "render");
+	render(-1, 0, st);
 	mark(2);
 	launch_walkers_fwd(0, grad, st);
 	mark(3);
@@ -1289,9 +1312,7 @@ void Engine::model_images(const ProfileParams *params, float *out)
 		hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
 		                       d_err_.as<int>(), nc, d_qcount_.as<int>(), nullptr, st),
 		          "setup");
-		hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), n, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
-		                        work_queue(), -1, 0, nullptr, st),
-		          "render");
+		render(-1, 0, st);
 		launch_walkers_fwd(0, false, st);
 		conv_forward(1, st);
 		report(false, false, st);
@@ -1300,19 +1321,47 @@ void Engine::model_images(const ProfileParams *params, float *out)
 		if (queue_ok()) break;
 		retry_evaluation();
 	}
-	size_t off = 0;
-	for (int i = 0; i < n; ++i) {
+	// the images leave the canvases in groups, through the two halves of a
+	// pinned buffer: while the host copies one group out, a kernel crops the
+	// next one straight into the other half
+	auto pixels = [&](int i) {
 		const GalaxyDev &g = gal_host_[inst_galaxy_[i]];
-		std::vector<float> canvas((size_t)g.DW * g.DH);
-		const float *src = inst_bufs_[kInstBufs * i + 2].as<float>();
-		hip_check(hipMemcpy(canvas.data(), src, canvas.size() * 4, hipMemcpyDeviceToHost), "model");
-		for (int j = 0; j < g.H; ++j)
-			for (int k = 0; k < g.W; ++k) out[off + (size_t)j * g.W + k] = canvas[(size_t)(j + g.pady) * g.DW + k + g.padx];
-		off += (size_t)g.W * g.H;
+		return (size_t)g.W * g.H;
+	};
+	size_t half = 1u << 19;  // floats
+	for (int i = 0; i < n; ++i) half = std::max(half, pixels(i));
+	if (h_images_.size() < 2 * half * sizeof(float)) h_images_.alloc(2 * half * sizeof(float));
+	auto group_end = [&](int first) {
+		size_t sum = 0;
+		int i = first;
+		for (; i < n && i - first < kCropGroup && sum + pixels(i) <= half; ++i) sum += pixels(i);
+		return i;
+	};
+	auto crop = [&](int first, int end, float *dst) {
+		CropGroup c;
+		c.first = first;
+		c.count = end - first;
+		c.off[0] = 0;
+		for (int i = first; i < end; ++i) c.off[i - first + 1] = c.off[i - first] + (long)pixels(i);
+		hip_check(launch_crop(gals, insts, c, dst, st), "crop");
+	};
+	float *buf[2] = {h_images_.as<float>(), h_images_.as<float>() + half};
+	int first = 0, end = group_end(0);
+	if (n) crop(first, end, buf[0]);
+	for (int k = 0; first < n; ++k) {
+		hip_check(hipStreamSynchronize(st), "sync");
+		const int next = end, next_end = group_end(next);
+		if (next < n) crop(next, next_end, buf[(k + 1) & 1]);
+		size_t sum = 0;
+		for (int i = first; i < end; ++i) sum += pixels(i);
+		std::memcpy(out, buf[k & 1], sum * sizeof(float));
+		out += sum;
+		first = next;
+		end = next_end;
 	}
 }
 
-void Engine::model_canvas(const ProfileParams *params, float *out, float *out_direct)
+const float *Engine::model_canvas(const ProfileParams *params, const float **direct, bool convolve)
 {
 	if (ninst() != 1) throw std::invalid_argument("model_canvas needs a batch of one instance");
 	hip_check(hipSetDevice(device_), "hipSetDevice");
@@ -1324,48 +1373,34 @@ void Engine::model_canvas(const ProfileParams *params, float *out, float *out_di
 	const InstDev *insts = d_insts_.as<InstDev>();
 	const GalaxyDev &g = gal_host_[inst_galaxy_[0]];
 	const bool conv = g.has_psf != 0;
+	// profiles drawn beside the convolved ones: without any, the aux canvas
+	// (all zeros) is neither drawn nor copied
+	bool beside = false;
+	for (int c = 0; c < nc; ++c) beside |= conv && !params[c].convolve;
+	const size_t nd = (size_t)g.DW * g.DH;
+	if (h_images_.size() < 2 * nd * sizeof(float)) h_images_.alloc(2 * nd * sizeof(float));
+	float *canvas = h_images_.as<float>(), *aux = canvas + nd;
 	mask_walk_ = false;
 	for (int attempt = 0; attempt < 4; ++attempt) {
 		hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
 		                       d_err_.as<int>(), nc, d_qcount_.as<int>(), nullptr, st),
 		          "setup");
 		// convolved profiles into the canvas, the others into the aux canvas
-		hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), 1, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
-		                        work_queue(), conv ? 1 : -1, 0, nullptr, st),
-		          "render");
-		if (conv)
-			hip_check(launch_render(gals, insts, d_ag_off_.as<int>(), 1, n_ag_blocks_, adj_grp_, tile_parts_, d_comps_.as<Comp>(),
-			                        work_queue(), 0, 1, nullptr, st),
-			          "render");
-		launch_walkers_fwd(conv ? 1 : 0, false, st);
-		if (conv && !out_direct) conv_forward(1, st);
+		render(beside ? 1 : -1, 0, st);
+		if (beside) render(0, 1, st);
+		launch_walkers_fwd(beside ? 1 : 0, false, st);
+		if (conv && convolve) conv_forward(1, st);
+		const float *src = inst_bufs_[conv && convolve ? 2 : 0].as<float>();
+		hip_check(hipMemcpyAsync(canvas, src, nd * 4, hipMemcpyDeviceToHost, st), "model");
+		if (beside) hip_check(hipMemcpyAsync(aux, inst_bufs_[3].as<float>(), nd * 4, hipMemcpyDeviceToHost, st), "model");
 		report(false, false, st);
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
 		if (queue_ok()) break;
 		retry_evaluation();
 	}
-	const size_t nd = (size_t)g.DW * g.DH;
-	if (out_direct) {
-		// the two canvases before any convolution
-		if (conv) {
-			hip_check(hipMemcpy(out, inst_bufs_[0].as<float>(), nd * 4, hipMemcpyDeviceToHost), "model");
-			hip_check(hipMemcpy(out_direct, inst_bufs_[3].as<float>(), nd * 4, hipMemcpyDeviceToHost), "model");
-		}
-		else {
-			std::memset(out, 0, nd * 4);
-			hip_check(hipMemcpy(out_direct, inst_bufs_[0].as<float>(), nd * 4, hipMemcpyDeviceToHost), "model");
-		}
-	}
-	else if (conv) {
-		std::vector<float> aux(nd);
-		hip_check(hipMemcpy(out, inst_bufs_[2].as<float>(), nd * 4, hipMemcpyDeviceToHost), "model");
-		hip_check(hipMemcpy(aux.data(), inst_bufs_[3].as<float>(), nd * 4, hipMemcpyDeviceToHost), "model");
-		for (size_t k = 0; k < nd; ++k) out[k] += aux[k];
-	}
-	else {
-		hip_check(hipMemcpy(out, inst_bufs_[0].as<float>(), nd * 4, hipMemcpyDeviceToHost), "model");
-	}
+	*direct = beside ? aux : nullptr;
+	return canvas;
 }
 
 void Engine::convolve_canvas(const float *canvas, float *out)
@@ -1396,12 +1431,179 @@ void Engine::dilate(const uint8_t *in, uint8_t *out, int w, int h, int padx, int
 	hip_check(hipMemcpy(out, c.as<uint8_t>(), n, hipMemcpyDeviceToHost), "mask");
 }
 
+// ------------------------------------------------------------------ bare convolutions
+
+// What a convolution of one geometry needs on the device besides its inputs:
+// buffers, tile list or FFT tables, pinned staging and a stream.  Every call
+// uploads its source, kernel and mask afresh (their contents are never kept
+// for a later call).
+class ConvPlan {
+  public:
+	ConvPlan(int w, int h, int kw, int kh, int device, int method);
+	~ConvPlan()
+	{
+		if (st_) (void)hipStreamDestroy(st_);
+	}
+	ConvPlan(const ConvPlan &) = delete;
+	ConvPlan &operator=(const ConvPlan &) = delete;
+	bool fits(int w, int h, int kw, int kh, int device, int method) const
+	{
+		return w == w_ && h == h_ && kw == kw_ && kh == kh_ && device == device_ && method == method_;
+	}
+	size_t bytes() const { return bytes_; }
+	void run(const double *src, const double *krn, const uint8_t *mask, double *out);
+
+  private:
+	int w_, h_, kw_, kh_, device_, method_;
+	size_t bytes_ = 0;
+	hipStream_t st_ = nullptr;
+	GalaxyDev g_{};
+	DevBuf src_, out_, krn_, mask_, tiles_, gal_, inst_, off_;
+	DevBuf frame_, spec_, fbuf_, tw_, col_blk_, inv_blk_;  // FFT
+	HostBuf h_src_, h_krn_, h_mask_, h_out_;
+	int twn_ = 0, ncol_ = 0, nrow_ = 0;
+};
+
+ConvPlan::ConvPlan(int w, int h, int kw, int kh, int device, int method)
+    : w_(w), h_(h), kw_(kw), kh_(kh), device_(device), method_(method)
+{
+	const size_t n = (size_t)w * h, nk = (size_t)kw * kh;
+	g_.W = g_.DW = w;
+	g_.H = g_.DH = h;
+	g_.Kx = kw;
+	g_.Ky = kh;
+	std::vector<int2> tiles, cols, inv;
+	if (method == CK_FFT) {
+		const int n1 = fft_frame(w + kw), n2 = fft_frame(h + kh);
+		if (std::max(n1, n2) > 4096) throw std::invalid_argument("FFT frame above 4096 points per axis is not supported");
+		g_.conv_kind = CK_FFT;
+		g_.fft_n1 = n1;
+		g_.fft_n2 = n2;
+		g_.fft_l1 = ilog2(n1);
+		g_.fft_l2 = ilog2(n2);
+		const size_t half = (size_t)fft_pitch(n1) * n2 * sizeof(double2);
+		frame_.alloc((size_t)n1 * n2 * sizeof(double));
+		spec_.alloc(half);
+		fbuf_.alloc(half);
+		bytes_ += frame_.size() + 2 * half;
+		twn_ = std::max(n1, n2);
+		const std::vector<double2> tw = twiddles(twn_);
+		tw_.alloc(tw.size() * sizeof(double2));
+		hip_check(hipMemcpy(tw_.as<double2>(), tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice), "tw");
+		const int cb = fft_cols_per_block(n2), rpb = 2 * fft_pairs_per_block(n1);
+		ncol_ = (n1 / 2 + 1 + cb - 1) / cb;
+		nrow_ = (h + rpb - 1) / rpb;
+		for (int t = 0; t < ncol_; ++t) cols.push_back(make_int2(0, t));
+		for (int t = 0; t < nrow_; ++t) inv.push_back(make_int2(0, t));
+		col_blk_.alloc(cols.size() * sizeof(int2));
+		inv_blk_.alloc(inv.size() * sizeof(int2));
+		hip_check(hipMemcpy(col_blk_.as<int2>(), cols.data(), cols.size() * sizeof(int2), hipMemcpyHostToDevice), "blocks");
+		hip_check(hipMemcpy(inv_blk_.as<int2>(), inv.data(), inv.size() * sizeof(int2), hipMemcpyHostToDevice), "blocks");
+		g_.fft_spec = spec_.as<double2>();
+		nrow_ = std::max(nrow_, 1);
+	}
+	else {
+		g_.conv_rows = kImageRows;
+		const int th = 4 * kImageRows;
+		for (int ty = 0; ty * th < h; ++ty)
+			for (int tx = 0; tx * kTileW < w; ++tx) tiles.push_back(make_int2(tx, ty));
+		tiles_.alloc(tiles.size() * sizeof(int2));
+		hip_check(hipMemcpy(tiles_.as<int2>(), tiles.data(), tiles.size() * sizeof(int2), hipMemcpyHostToDevice), "tiles");
+		g_.atiles = tiles_.as<int2>();
+		g_.n_atiles = (int)tiles.size();
+	}
+	src_.alloc(n * 4);
+	out_.alloc(n * 4);
+	mask_.alloc(n);
+	krn_.alloc(nk * sizeof(double));
+	gal_.alloc(sizeof(GalaxyDev));
+	inst_.alloc(sizeof(InstDev));
+	off_.alloc(2 * sizeof(int));
+	h_src_.alloc(n * 4);
+	h_out_.alloc(n * 4);
+	h_krn_.alloc(nk * sizeof(double));
+	h_mask_.alloc(n);
+	bytes_ += 18 * n + 2 * krn_.size();
+	g_.psf_fwd = krn_.as<float>();
+	g_.calc = mask_.as<uint8_t>();
+	InstDev I{};
+	I.canvas = src_.as<float>();
+	I.G = out_.as<float>();
+	I.fbuf = fbuf_.as<double2>();
+	const int off[2] = {0, method == CK_FFT ? nrow_ : g_.n_atiles};
+	hip_check(hipMemcpy(gal_.as<GalaxyDev>(), &g_, sizeof(g_), hipMemcpyHostToDevice), "gal");
+	hip_check(hipMemcpy(inst_.as<InstDev>(), &I, sizeof(I), hipMemcpyHostToDevice), "inst");
+	hip_check(hipMemcpy(off_.as<int>(), off, sizeof(off), hipMemcpyHostToDevice), "off");
+	hip_check(hipStreamCreateWithFlags(&st_, hipStreamNonBlocking), "hipStreamCreate");
+}
+
+void ConvPlan::run(const double *src, const double *krn, const uint8_t *mask, double *out)
+{
+	const size_t n = (size_t)w_ * h_, nk = (size_t)kw_ * kh_;
+	float *hs = h_src_.as<float>();
+	for (size_t k = 0; k < n; ++k) hs[k] = (float)src[k];
+	hip_check(hipMemcpyAsync(src_.as<float>(), hs, n * 4, hipMemcpyHostToDevice, st_), "src");
+	if (mask) {
+		std::memcpy(h_mask_.as<uint8_t>(), mask, n);
+		hip_check(hipMemcpyAsync(mask_.as<uint8_t>(), h_mask_.as<uint8_t>(), n, hipMemcpyHostToDevice, st_), "mask");
+	}
+	if (g_.has_calc != (mask ? 1 : 0)) {
+		// the previous run on this stream has ended
+		g_.has_calc = mask ? 1 : 0;
+		hip_check(hipMemcpy(gal_.as<GalaxyDev>(), &g_, sizeof(g_), hipMemcpyHostToDevice), "gal");
+	}
+	const GalaxyDev *gal = gal_.as<GalaxyDev>();
+	const InstDev *inst = inst_.as<InstDev>();
+	if (method_ == CK_FFT) {
+		std::memcpy(h_krn_.as<double>(), krn, nk * sizeof(double));
+		hip_check(hipMemcpyAsync(krn_.as<double>(), h_krn_.as<double>(), nk * sizeof(double), hipMemcpyHostToDevice, st_),
+		          "krn");
+		const int n1 = g_.fft_n1, n2 = g_.fft_n2, cb = fft_cols_per_block(n2);
+		const double2 *tw = tw_.as<double2>();
+		hip_check(launch_psf_frame(krn_.as<double>(), kw_, kh_, n1, n2, frame_.as<double>(), st_), "psf frame");
+		hip_check(launch_fft_psf_rows(n1, n2, gal, tw, twn_, frame_.as<double>(), spec_.as<double2>(), st_), "psf rows");
+		hip_check(launch_fft_cols(ncol_, n2, cb, gal, inst, col_blk_.as<int2>(), 0, 2, 0, tw, twn_, spec_.as<double2>(), st_),
+		          "psf cols");
+		hip_check(launch_fft_rows_fwd(nrow_, n1, gal, inst, off_.as<int>(), 1, 0, tw, twn_, st_), "fft rows");
+		hip_check(launch_fft_cols(ncol_, n2, cb, gal, inst, col_blk_.as<int2>(), 1, 0, 1, tw, twn_, nullptr, st_), "fft cols");
+		hip_check(launch_fft_rows_inv(nrow_, n1, gal, inst, inv_blk_.as<int2>(), 1, tw, twn_, nullptr, nullptr, st_),
+		          "fft rows inv");
+	}
+	else {
+		float *f = h_krn_.as<float>();
+		for (int ky = 0; ky < kh_; ++ky)
+			for (int kx = 0; kx < kw_; ++kx)
+				f[(size_t)ky * kw_ + kx] = (float)krn[(size_t)(kh_ - 1 - ky) * kw_ + (kw_ - 1 - kx)];
+		hip_check(hipMemcpyAsync(krn_.as<float>(), f, nk * 4, hipMemcpyHostToDevice, st_), "krn");
+		hip_check(launch_conv(CONV_MODEL, kImageRows, g_.n_atiles, kw_, std::min(kh_, 64), gal, inst, off_.as<int>(), 1, nullptr,
+		                      nullptr, st_, conv_split(kImageRows, g_.n_atiles)),
+		          "conv");
+	}
+	hip_check(hipMemcpyAsync(h_out_.as<float>(), out_.as<float>(), n * 4, hipMemcpyDeviceToHost, st_), "out");
+	hip_check(hipStreamSynchronize(st_), "sync");
+	const float *ho = h_out_.as<float>();
+	for (size_t k = 0; k < n; ++k) out[k] = ho[k];
+}
+
+// Idle plans, most recently used first.  A call takes a plan out of the pool
+// for its own use (so callers on several threads never share one) and gives it
+// back; the pool keeps the last few within a bound on their memory.
+static std::mutex g_plan_mu;
+static std::list<std::unique_ptr<ConvPlan>> g_plans;
+static constexpr size_t kPlanEntries = 4, kPlanBytes = 512u << 20;
+
+void clear_convolution_plans()
+{
+	std::lock_guard<std::mutex> lock(g_plan_mu);
+	g_plans.clear();
+}
+
 void convolve_image(const double *src, int w, int h, const double *krn, int kw, int kh, const uint8_t *mask,
                     double *out, int device, int method)
 {
 	hip_check(hipSetDevice(device), "hipSetDevice");
-	if (method == CK_FFT || method == CK_MFMA) {
-		// FFT or matrix-core path: a one-instance engine whose canvas is the source image
+	if (method == CK_MFMA) {
+		// matrix-core path: a one-instance engine whose canvas is the source image
 		// (no padding, the kernel as given, the mask as its calc region)
 		const size_t n = (size_t)w * h;
 		std::vector<double> zeros(n, 0.0), ones(n, 1.0);
@@ -1434,46 +1636,29 @@ void convolve_image(const double *src, int w, int h, const double *krn, int kw, 
 		for (size_t k = 0; k < n; ++k) out[k] = r[k];
 		return;
 	}
-	const int rows = 4;
-	const size_t n = (size_t)w * h;
-	std::vector<float> s(n), f((size_t)kw * kh);
-	for (size_t k = 0; k < n; ++k) s[k] = (float)src[k];
-	for (int ky = 0; ky < kh; ++ky)
-		for (int kx = 0; kx < kw; ++kx) f[(size_t)ky * kw + kx] = (float)krn[(size_t)(kh - 1 - ky) * kw + (kw - 1 - kx)];
-	std::vector<int2> tiles;
-	const int th = 4 * rows;
-	for (int ty = 0; ty * th < h; ++ty)
-		for (int tx = 0; tx * kTileW < w; ++tx) tiles.push_back(make_int2(tx, ty));
-	DevBuf d_src(n * 4), d_out(n * 4), d_krn(f.size() * 4), d_mask(mask ? n : 1), d_tiles(tiles.size() * sizeof(int2));
-	DevBuf d_gal(sizeof(GalaxyDev)), d_inst(sizeof(InstDev)), d_off(2 * sizeof(int));
-	hip_check(hipMemcpy(d_src.as<float>(), s.data(), n * 4, hipMemcpyHostToDevice), "src");
-	hip_check(hipMemcpy(d_krn.as<float>(), f.data(), f.size() * 4, hipMemcpyHostToDevice), "krn");
-	if (mask) hip_check(hipMemcpy(d_mask.as<uint8_t>(), mask, n, hipMemcpyHostToDevice), "mask");
-	hip_check(hipMemcpy(d_tiles.as<int2>(), tiles.data(), tiles.size() * sizeof(int2), hipMemcpyHostToDevice), "tiles");
-	GalaxyDev g{};
-	g.W = g.DW = w;
-	g.H = g.DH = h;
-	g.Kx = kw;
-	g.Ky = kh;
-	g.has_calc = mask != nullptr;
-	g.calc = mask ? d_mask.as<uint8_t>() : nullptr;
-	g.psf_fwd = d_krn.as<float>();
-	g.atiles = d_tiles.as<int2>();
-	g.n_atiles = (int)tiles.size();
-	g.conv_rows = rows;
-	InstDev I{0, 0, 0, 0, d_src.as<float>(), nullptr, d_out.as<float>(), nullptr, nullptr, nullptr};
-	const int off[2] = {0, (int)tiles.size()};
-	hip_check(hipMemcpy(d_gal.as<GalaxyDev>(), &g, sizeof(g), hipMemcpyHostToDevice), "gal");
-	hip_check(hipMemcpy(d_inst.as<InstDev>(), &I, sizeof(I), hipMemcpyHostToDevice), "inst");
-	hip_check(hipMemcpy(d_off.as<int>(), off, sizeof(off), hipMemcpyHostToDevice), "off");
-	const int kc = std::min(kh, 64);
-	hip_check(launch_conv(1, rows, (int)tiles.size(), kw, kc, d_gal.as<GalaxyDev>(), d_inst.as<InstDev>(), d_off.as<int>(),
-	                      1, nullptr, nullptr, nullptr),
-	          "conv");
-	hip_check(hipDeviceSynchronize(), "sync");
-	std::vector<float> o(n);
-	hip_check(hipMemcpy(o.data(), d_out.as<float>(), n * 4, hipMemcpyDeviceToHost), "out");
-	for (size_t k = 0; k < n; ++k) out[k] = o[k];
+	std::unique_ptr<ConvPlan> plan;
+	{
+		std::lock_guard<std::mutex> lock(g_plan_mu);
+		for (auto it = g_plans.begin(); it != g_plans.end(); ++it)
+			if ((*it)->fits(w, h, kw, kh, device, method)) {
+				plan = std::move(*it);
+				g_plans.erase(it);
+				break;
+			}
+	}
+	if (!plan) plan.reset(new ConvPlan(w, h, kw, kh, device, method));
+	plan->run(src, krn, mask, out);
+	std::list<std::unique_ptr<ConvPlan>> dropped;  // freed outside the lock
+	{
+		std::lock_guard<std::mutex> lock(g_plan_mu);
+		g_plans.push_front(std::move(plan));
+		size_t bytes = 0, count = 0;
+		for (auto it = g_plans.begin(); it != g_plans.end();) {
+			bytes += (*it)->bytes();
+			if (++count > kPlanEntries || bytes > kPlanBytes) dropped.splice(dropped.end(), g_plans, it++);
+			else ++it;
+		}
+	}
 }
 
 }  // namespace profit_amd

@@ -57,6 +57,8 @@ int launch_adj_render(int type, int prec, const GalaxyDev *gals, const InstDev *
 // an evaluation's results to pinned host memory
 int launch_report(const Comp *comps, const double *gscale, const double *grad_acc, const double *ll, const int *errors,
                   const int *qcount, int ncomp, int ninst, unsigned slot_mask, const HostReport &out, hipStream_t st);
+// crops the model images of a group of instances into dst (device or pinned)
+int launch_crop(const GalaxyDev *gals, const InstDev *insts, const CropGroup &group, float *dst, hipStream_t st);
 int launch_dilate(const uint8_t *in, uint8_t *tmp, uint8_t *out, int w, int h, int padx, int pady, hipStream_t st);
 // FFT path (fft.hip)
 int launch_fft_rows_fwd(int nblocks, int nmax, const GalaxyDev *gals, const InstDev *insts, const int *row_off,
@@ -75,6 +77,8 @@ int launch_fft_cols(int nblocks, int n2max, int cb, const GalaxyDev *gals, const
 int launch_fft_rows_inv(int nblocks, int nmax, const GalaxyDev *gals, const InstDev *insts, const int2 *blocks,
                         int mode, const double2 *tw, int twn, const int *lk_base, double *partial, hipStream_t st);
 int fft_cols_per_block(int n2);
+// a kernel wrapped about the origin of a zero n1 x n2 real frame (kernels.hip)
+int launch_psf_frame(const double *krn, int kw, int kh, int n1, int n2, double *frame, hipStream_t st);
 // split-BF16x3 matrix-core path (conv_mfma.hip)
 int mfma_kc(int kx);
 int mfma_pitch(int kc);
@@ -83,11 +87,14 @@ void mfma_fragments(const float *wt, int kx, int ky, std::vector<uint16_t> &out)
 int launch_conv_mfma(int mode, int nblocks, int pitch, int kch, const GalaxyDev *gals, const InstDev *insts,
                      const int *tile_off, int ninst, const int *lk_base, double *partial, hipStream_t st);
 
-// Convolver::convolve_impl on the GPU, masked output pixels are 0: method 0
-// tiled brute force, 1 FFT.  The kernel is used as given (libprofit
+// Convolver::convolve_impl on the GPU, masked output pixels are 0: method
+// CK_VALU tiled brute force, CK_FFT, CK_MFMA split-BF16x3.  The kernel is used as given (libprofit
 // normalises only the Model's PSF).
 void convolve_image(const double *src, int w, int h, const double *krn, int kw, int kh, const uint8_t *mask,
                     double *out, int device, int method = 0);
+
+// releases the device set-ups kept for repeated convolutions of one geometry
+void clear_convolution_plans();
 
 class hip_error : public std::runtime_error {
   public:
@@ -142,6 +149,17 @@ class HostBuf {
   private:
 	void *p_ = nullptr;
 	size_t n_ = 0;
+};
+
+// a part of a pinned allocation
+class HostView {
+  public:
+	HostView() = default;
+	explicit HostView(void *p) : p_(p) {}
+	template <class T> T *as() const { return static_cast<T *>(p_); }
+
+  private:
+	void *p_ = nullptr;
 };
 
 // A galaxy as the likelihood engine sees it: ProFit's profitSetupData output.
@@ -215,12 +233,13 @@ class Engine {
 	                       double *rmax);
 	// the convolved model of every instance (W*H floats each, region-independent)
 	void model_images(const ProfileParams *params, float *out);
-	// Model::evaluate's drawing canvas for a single instance: convolved profiles
-	// (masked by the calc region) plus the profiles drawn without convolution.
-	// With out_direct given, nothing is convolved: out receives the canvas of
-	// the profiles to be convolved and out_direct that of the others, as
-	// Model::produce_image holds them before its convolver runs.
-	void model_canvas(const ProfileParams *params, float *out, float *out_direct = nullptr);
+	// Model::evaluate's drawing canvas for a single instance (DW*DH floats in
+	// pinned memory, valid until the engine's next call): the profiles to be
+	// convolved, convolved or (convolve = false) as Model::produce_image holds
+	// them before its convolver runs.  *direct: the canvas of the profiles drawn
+	// without convolution, null when there is none; without a PSF every profile
+	// is on the returned canvas.
+	const float *model_canvas(const ProfileParams *params, const float **direct, bool convolve);
 	// Mask::expand_by on the device
 	static void dilate(const uint8_t *in, uint8_t *out, int w, int h, int padx, int pady, int device = 0);
 
@@ -262,6 +281,7 @@ class Engine {
 	void upload_galaxies();
 	void run(bool grad, bool use_graph);
 	void record(bool grad);
+	void render(int filter, int target, hipStream_t st);
 	void ensure_queue(const long *need, long hneed);
 	WorkQueue work_queue();
 	bool queue_ok() const;
@@ -341,7 +361,10 @@ class Engine {
 	DevBuf d_comps_, d_err_, d_queue_, d_qcount_, d_partial_, d_ll_, d_gscale_, d_grad_acc_;
 	long lcap_[kFamilies] = {}, hcap_ = 0;
 	DevBuf d_hqueue_, d_qjac_, d_hjac_, d_qdeep_;
-	HostBuf h_params_, h_ll_, h_grad_, h_err_, h_qcount_;
+	// the parameters and results of an evaluation, parts of one allocation
+	HostBuf h_eval_;
+	HostView h_params_, h_ll_, h_grad_, h_err_, h_qcount_;
+	HostBuf h_images_;  // staging of model images and canvases
 
 	hipGraphExec_t graph_exec_[2] = {nullptr, nullptr};
 	hipEvent_t events_[ST_COUNT + 1] = {};

@@ -1049,6 +1049,34 @@ __global__ void k_dilate_cols(const uint8_t *__restrict__ in, uint8_t *out, int 
 	out[(long)j * w + i] = v;
 }
 
+// The model images (the image part of G) of a group of instances, one after
+// another; blockIdx.y is the instance.
+__global__ __launch_bounds__(256) void k_crop(const GalaxyDev *__restrict__ gals, const InstDev *__restrict__ insts,
+                                              CropGroup group, float *__restrict__ dst)
+{
+	const InstDev &I = insts[group.first + blockIdx.y];
+	const GalaxyDev &g = gals[I.galaxy];
+	float *out = dst + group.off[blockIdx.y];
+	const int n = g.W * g.H;
+	for (int o = blockIdx.x * 256 + threadIdx.x; o < n; o += gridDim.x * 256) {
+		const int y = o / g.W, x = o - y * g.W;
+		out[o] = I.G[(long)(y + g.pady) * g.DW + x + g.padx];
+	}
+}
+
+// A kernel's weights as a function of the offset, g(d) = krn[K - 1 - K/2 + d],
+// wrapped about the origin of a zero real frame: the FFT path's PSF frame.
+__global__ __launch_bounds__(256) void k_psf_frame(const double *__restrict__ krn, int kw, int kh, int n1, int n2,
+                                                   double *frame)
+{
+	const int x = blockIdx.x * 256 + threadIdx.x, y = blockIdx.y;
+	if (x >= n1) return;
+	const int ax = kw - 1 - kw / 2, ay = kh - 1 - kh / 2;
+	// the taps at kx - ax and ky - ay, modulo the frame
+	const int kx = x + ax < kw ? x + ax : x + ax - n1, ky = y + ay < kh ? y + ay : y + ay - n2;
+	frame[(long)y * n1 + x] = kx >= 0 && ky >= 0 ? krn[(long)ky * kw + kx] : 0.0;
+}
+
 // ------------------------------------------------------------------ launch wrappers
 
 #define PA_CHECK(x)                                  \
@@ -1196,6 +1224,21 @@ int launch_report(const Comp *comps, const double *gscale, const double *grad_ac
 {
 	const int n = std::max({out.grad ? ncomp * NGRAD : ncomp, ninst, kQueueCounters});
 	k_report<<<(n + 255) / 256, 256, 0, st>>>(comps, gscale, grad_acc, ll, errors, qcount, ncomp, ninst, slot_mask, out);
+	return (int)hipGetLastError();
+}
+
+int launch_crop(const GalaxyDev *gals, const InstDev *insts, const CropGroup &group, float *dst, hipStream_t st)
+{
+	if (group.count <= 0) return 0;
+	if (group.count > kCropGroup) return (int)hipErrorInvalidValue;
+	k_crop<<<dim3(64, group.count), 256, 0, st>>>(gals, insts, group, dst);
+	return (int)hipGetLastError();
+}
+
+int launch_psf_frame(const double *krn, int kw, int kh, int n1, int n2, double *frame, hipStream_t st)
+{
+	if (kw < 1 || kh < 1 || n1 < kw || n2 < kh) return (int)hipErrorInvalidValue;
+	k_psf_frame<<<dim3((n1 + 255) / 256, n2), 256, 0, st>>>(krn, kw, kh, n1, n2, frame);
 	return (int)hipGetLastError();
 }
 

@@ -29,6 +29,15 @@ Image::Image(const std::vector<double> &data, unsigned int w, unsigned int h) : 
 	if (data_.size() != (size_t)w * h) throw std::invalid_argument("data size != width * height");
 }
 
+Image::Image(Dimensions d, const float *src, size_t pitch, Point start) : dims_(d)
+{
+	data_.reserve((size_t)d.x * d.y);
+	for (unsigned j = 0; j < d.y; ++j) {
+		const float *row = src + (size_t)(j + start.y) * pitch + start.x;
+		data_.insert(data_.end(), row, row + d.x);
+	}
+}
+
 void Image::zero() { std::fill(data_.begin(), data_.end(), 0.0); }
 
 double Image::total() const
@@ -604,8 +613,11 @@ profit_amd::Engine &cached_engine(const profit_amd::GalaxySpec &gs, int method, 
 
 void clear_cache()
 {
-	std::lock_guard<std::mutex> lock(g_cache_mu);
-	g_cache.clear();
+	{
+		std::lock_guard<std::mutex> lock(g_cache_mu);
+		g_cache.clear();
+	}
+	profit_amd::clear_convolution_plans();
 }
 
 std::map<std::string, std::shared_ptr<ProfileStats>> Model::get_stats() const
@@ -619,9 +631,12 @@ std::map<std::string, std::shared_ptr<ProfileStats>> Model::get_stats() const
 void Model::evaluate(Image &image, Point &offset_out)
 {
 	const Analysis a = analyze_inputs();
-	if (image.getDimensions() == a.drawing_dims) image.zero();
-	else image = Image(a.drawing_dims);
+	auto blank = [&] {
+		if (image.getDimensions() == a.drawing_dims) image.zero();
+		else image = Image(a.drawing_dims);
+	};
 	if (dry_run_) {
+		blank();
 		if (&offset_out != &NO_OFFSET) offset_out = Point{0, 0};
 		return;
 	}
@@ -659,6 +674,10 @@ void Model::evaluate(Image &image, Point &offset_out)
 	const bool literal = a.convolution_required && (ctype == NO_OP || (ctype == FFT && !crop_));
 	Point offset{0, 0};
 	RadialProfileStats times;
+	// the canvas's part that is returned, taken straight from it where no
+	// uncropped convolution can have enlarged the frame
+	const bool cropped = a.psf_padding && crop_ && !literal && !drawn.empty();
+	if (literal || drawn.empty()) blank();
 	if (!drawn.empty() || literal) {
 		profit_amd::GalaxySpec gs;
 		gs.W = (int)(requested_dimensions_.x * finesampling_);
@@ -681,7 +700,8 @@ void Model::evaluate(Image &image, Point &offset_out)
 			gs.ch = (int)draw_mask->getHeight();
 		}
 		const size_t nd = (size_t)a.drawing_dims.x * a.drawing_dims.y;
-		std::vector<float> canvas(nd, 0.f), direct(literal ? nd : 0, 0.f);
+		Image to_convolve;
+		if (literal) to_convolve = Image(a.drawing_dims);
 		if (!drawn.empty()) {
 			const int method = literal ? profit_amd::CK_VALU : kernel_method(ctype);
 			std::lock_guard<std::mutex> lock(g_cache_mu);
@@ -690,24 +710,36 @@ void Model::evaluate(Image &image, Point &offset_out)
 			if ((unsigned)g.DW != a.drawing_dims.x || (unsigned)g.DH != a.drawing_dims.y)
 				throw std::logic_error("engine drawing dimensions differ from the model analysis");
 			const auto t0 = std::chrono::steady_clock::now();
+			const float *canvas = nullptr, *direct = nullptr;
 			try {
-				eng.model_canvas(drawn.data(), canvas.data(), literal ? direct.data() : nullptr);
+				canvas = eng.model_canvas(drawn.data(), &direct, !literal);
 			} catch (const std::invalid_argument &e) {
 				throw invalid_parameter(e.what());
 			}
 			times.total = (nsecs_t)std::chrono::duration_cast<std::chrono::nanoseconds>(
 			                  std::chrono::steady_clock::now() - t0)
 			                  .count();
+			if (!literal) {
+				const Point start = cropped ? Point(a.psf_padding) : Point{0, 0};
+				const Dimensions d = a.drawing_dims - Dimensions(start) * 2;
+				image = Image(d, canvas, a.drawing_dims.x, start);
+				if (direct)
+					for (unsigned j = 0; j < d.y; ++j)
+						for (unsigned i = 0; i < d.x; ++i) {
+							// the sum of the two canvases in FP32, as the engine holds them
+							const size_t q = (size_t)(j + start.y) * a.drawing_dims.x + i + start.x;
+							image[i + (size_t)j * d.x] = canvas[q] + direct[q];
+						}
+			}
+			else {
+				for (size_t k = 0; k < nd; ++k) to_convolve[k] = canvas[k];
+				if (direct)
+					for (size_t k = 0; k < nd; ++k) image[k] += direct[k];
+			}
 		}
-		if (!literal) {
-			for (size_t k = 0; k < nd; ++k) image[k] += canvas[k];
-		}
-		else {
+		if (literal) {
 			// model.cpp:355-377: the unconvolved profiles on the canvas, then
 			// convolve, extend the canvas to the result's frame and add
-			for (size_t k = 0; k < nd; ++k) image[k] += direct[k];
-			Image to_convolve(a.drawing_dims);
-			for (size_t k = 0; k < nd; ++k) to_convolve[k] = canvas[k];
 			const Image conv = convolver->convolve(to_convolve, psf_, *draw_mask, crop_, offset);
 			if (conv.getDimensions() != a.drawing_dims) image = image.extend(conv.getDimensions(), offset);
 			for (size_t k = 0; k < image.size(); ++k) image[k] += conv[k];
@@ -715,7 +747,7 @@ void Model::evaluate(Image &image, Point &offset_out)
 	}
 	for (auto &p : profiles_) p->set_stats(times);
 
-	if (a.psf_padding) {
+	if (a.psf_padding && !cropped) {
 		// model.cpp:306-324
 		Point crop_offset = a.psf_padding;
 		Dimensions crop_dims = a.drawing_dims - a.psf_padding * 2;

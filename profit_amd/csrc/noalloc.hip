@@ -5,7 +5,7 @@
 // HIP graph capture, tight serving loops).
 //
 // The staging that the allocating entry point (convolve_image in engine.cpp)
-// allocates per call -- the FP32 copy of the source, the flipped FP32 kernel,
+// allocates -- the FP32 copy of the source, the flipped FP32 kernel,
 // the tile list, the galaxy and instance descriptors and the FP32 result --
 // lives here in one file-scope device array, `scratch`, of fixed size.  Every
 // GPU the library runs on holds its own copy until the process ends.  Host
@@ -166,7 +166,8 @@ void convolve_noalloc(int method, const double *src, int w, int h, const double 
 	hip_check(launch_conv(CONV_MODEL, kRows, g.n_atiles, kw, std::min(kh, 64),
 	                      reinterpret_cast<const GalaxyDev *>(base + kOffGal),
 	                      reinterpret_cast<const InstDev *>(base + kOffInst),
-	                      reinterpret_cast<const int *>(base + kOffTileOff), 1, nullptr, nullptr, st),
+	                      reinterpret_cast<const int *>(base + kOffTileOff), 1, nullptr, nullptr, st,
+	                      conv_split(kRows, g.n_atiles)),
 	          "convolution launch");
 	k_noalloc_out<<<grid_for(n), 256, 0, st>>>(reinterpret_cast<const float *>(base + kOffDst), out, n);
 	hip_check(hipGetLastError(), "output launch");

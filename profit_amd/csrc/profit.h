@@ -81,6 +81,8 @@ class Image {
 	Image(unsigned int w, unsigned int h) : dims_(w, h), data_((size_t)w * h, 0.0) {}
 	explicit Image(Dimensions d) : Image(d.x, d.y) {}
 	Image(const std::vector<double> &data, unsigned int w, unsigned int h);
+	// the rectangle d at `start` of an FP32 image of row length `pitch`
+	Image(Dimensions d, const float *src, size_t pitch, Point start);
 	unsigned int getWidth() const { return dims_.x; }
 	unsigned int getHeight() const { return dims_.y; }
 	Dimensions getDimensions() const { return dims_; }
