@@ -85,6 +85,16 @@ static int next_pow2(int v)
 // fold the bit reversal into their first and last three radix-2 stages)
 static int fft_frame(int v) { return std::max(8, next_pow2(v)); }
 
+// FFT frame of a galaxy's axis: canvas length d, kernel length k, padded by
+// k / 2 on both sides or not.  On a padded canvas only image pixels feed or read
+// the convolution, and they lie k / 2 from its edges: a circular convolution
+// over the canvas alone wraps nothing onto them, in either direction (the
+// padding itself, which is cropped from every image, would see the wrap).  An
+// unpadded canvas needs room for the kernel beside it.  A 237-pixel canvas with
+// 41 taps takes 256 points instead of 512 (256 likelihoods of 197x180: 1.23
+// times the speed).
+static int galaxy_frame(int d, int k, int pad) { return fft_frame(pad > 0 ? d : d + k); }
+
 // rows per thread of the brute-force convolution of a bare image (the
 // allocation-free entry point takes the same)
 static constexpr int kImageRows = 4;
@@ -233,7 +243,7 @@ Engine::TuneReport Engine::autotune(const ProfileParams *params, int reps, bool 
 			if (kind == CK_VALU) v = (double)(g.n_ctiles + g.n_atiles) * 256.0 * conv_rows_ * g.Kx * g.Ky;
 			else if (kind == CK_MFMA) v = (double)(g.n_mtl + g.n_mtc) * g.Ky * (g.mfma_kc + 2);
 			else {
-				const double n1 = fft_frame(g.DW + g.Kx), n2 = fft_frame(g.DH + g.Ky);
+				const double n1 = galaxy_frame(g.DW, g.Kx, g.padx), n2 = galaxy_frame(g.DH, g.Ky, g.pady);
 				v = n1 * n2 * std::log2(n1 * n2);
 			}
 			w[inst_galaxy_[i]] += v;
@@ -322,7 +332,7 @@ void Engine::ensure_fft_spectra()
 	int twn = 2;
 	for (const auto &g : gal_host_)
 		if (g.conv_kind == CK_FFT) {
-			const int n1 = fft_frame(g.DW + g.Kx), n2 = fft_frame(g.DH + g.Ky);
+			const int n1 = galaxy_frame(g.DW, g.Kx, g.padx), n2 = galaxy_frame(g.DH, g.Ky, g.pady);
 			twn = std::max(twn, std::max(n1, n2));
 		}
 	if (twn > 4096) throw std::invalid_argument("FFT frame above 4096 points per axis is not supported");
@@ -337,7 +347,7 @@ void Engine::ensure_fft_spectra()
 		GalaxyDev &g = gal_host_[gi];
 		GalaxyBuffers &b = gal_bufs_[gi];
 		if (g.conv_kind != CK_FFT || b.fft_spec.size()) continue;
-		const int n1 = fft_frame(g.DW + g.Kx), n2 = fft_frame(g.DH + g.Ky);
+		const int n1 = galaxy_frame(g.DW, g.Kx, g.padx), n2 = galaxy_frame(g.DH, g.Ky, g.pady);
 		g.fft_n1 = n1;
 		g.fft_n2 = n2;
 		g.fft_l1 = ilog2(n1);
