@@ -915,11 +915,13 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 	n_bt_blocks_ = bt_off_[n];
 	split_canvas_ = conv_split(conv_rows_, n_bt_blocks_);
 	// the renders give each thread about 32 canvas pixels of a component where
-	// that leaves 2,048 blocks (eight a CU), and fewer otherwise (a block's
-	// first pixel waits for a chain of loads, and the adjoint pays a reduction
-	// per component and block); below 1,024 tiles they split each tile over
+	// that leaves 8,192 blocks, and fewer otherwise (a block's first pixel waits
+	// for a chain of loads, and the adjoint pays a reduction per component and
+	// block; but 7,000 tiles of survey galaxies drawn in threes left the GPU
+	// waiting for its last blocks: renders 0.50 and 0.39 ms, adjoint
+	// renders 0.48 and 0.30); below 1,024 tiles they split each tile over
 	// several blocks, to two rows a thread at the least
-	adj_grp_ = std::min(std::max(1, 32 / conv_rows_), std::max(1, n_at_blocks_ / 2048));
+	adj_grp_ = std::min(std::max(1, 32 / conv_rows_), std::max(1, n_at_blocks_ / 8192));
 	tile_parts_ = 1;
 	while (n_at_blocks_ * tile_parts_ < 1024 && conv_rows_ / tile_parts_ > 2) tile_parts_ *= 2;
 	ag_off_.assign(n + 1, 0);
@@ -1132,6 +1134,7 @@ bool Engine::sync_aux_flags(bool enable)
 	bool any = false, changed = false;
 	unsigned types = 0, keys = 0;
 	int family[kFamilies] = {};
+	unsigned depth = 0;
 	for (int i = 0; i < ninst(); ++i) {
 		int aux = 0;
 		for (int k = 0; k < inst_ncomp_[i]; ++k) {
@@ -1139,6 +1142,7 @@ bool Engine::sync_aux_flags(bool enable)
 			if (is_radial(q.type)) {
 				types |= 1u << q.type;
 				++family[q.type];
+				depth = std::max(depth, q.max_recursions);
 				keys |= 1u << (2 * q.type + (wants_grad64(q) ? 1 : 0));
 				continue;
 			}
@@ -1153,6 +1157,13 @@ bool Engine::sync_aux_flags(bool enable)
 			changed = true;
 		}
 	}
+	// big trees do not fill the GPU with blocks of four wavefronts (see
+	// launch_subsample_fwd): up to 256 components of a family, or 1,024 whose
+	// ordinary pixels' trees are deep as well (512 components of two recursions:
+	// 0.17 ms with blocks of four, 0.20 with blocks of twelve; 500 of four: 0.69 and 0.47 ms)
+	const int few = depth > 2 ? 1024 : 256;
+	if (few != few_components_) invalidate_graphs(graph_exec_);
+	few_components_ = few;
 	if (any != any_nonradial_ || types != radial_types_ || keys != grad_keys_ ||
 	    std::memcmp(family, family_comps_, sizeof(family)) != 0) {
 		std::memcpy(family_comps_, family, sizeof(family));
@@ -1171,7 +1182,7 @@ void Engine::launch_walkers_fwd(int split, bool jac, hipStream_t st)
 	for (int t = 0; t < 6; ++t)
 		if ((radial_types_ >> t) & 1u)
 			hip_check(launch_subsample_fwd(t, subsample_blocks_, d_gals_.as<GalaxyDev>(), d_insts_.as<InstDev>(),
-			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, family_comps_[t], st),
+			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, family_comps_[t] <= few_components_, st),
 			          "subsample");
 }
 

@@ -32,10 +32,10 @@ int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *grp_of
 // (and per sum precision in the adjoint render: 1 = FP64 per-thread sums,
 // steep cores only).  jac: the forward walk also writes each entry's Jacobian
 // (wq.ljac, wq.hjac), which launch_adj_queue weighs by G(q).  mask: the trees
-// by the mask walk (after a tree overflowed the tree walk's stack).  ncomp: the
-// batch's components of the family.
+// by the mask walk (after a tree overflowed the tree walk's stack).  few: too few
+// big trees to fill the GPU with blocks of four wavefronts.
 int launch_subsample_fwd(int type, int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
-                         WorkQueue wq, int split, bool jac, bool mask, int ncomp, hipStream_t st);
+                         WorkQueue wq, int split, bool jac, bool mask, bool few, hipStream_t st);
 int launch_adj_queue(int type, int nblocks, const InstDev *insts, const Comp *comps, WorkQueue wq, double *grad_acc,
                      hipStream_t st);
 int launch_subsample_nodes(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
@@ -337,6 +337,7 @@ class Engine {
 	// keys present (bit 2t + prec), which decide the walker launches
 	unsigned radial_types_ = 0, grad_keys_ = 0;
 	int family_comps_[kFamilies] = {};  // components of each radial family
+	int few_components_ = 256;          // up to which its big trees are few
 	// trees by the mask walk: set while an evaluation runs again because a
 	// tree overflowed the tree walk's stack
 	bool mask_walk_ = false;

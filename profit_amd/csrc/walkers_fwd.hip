@@ -5,16 +5,14 @@
 
 namespace profit_amd {
 
-constexpr int kFewComponents = 512;
-
 // The root pass over the light entries, then the tree walk over the heavy list
 // and the entries the root pass left to it (mask: the mask walk instead, one
-// wavefront per tree).  `few`: at most kFewComponents components of the family:
-// their big trees (four centre pixels a component, or the like) do not fill the
-// GPU, so the tree walk takes blocks of twelve wavefronts, one a CU, and
-// otherwise blocks of four, three a CU.  Four and twelve, measured: 384 survey
-// galaxies (about 150 components a family), Sersic 336 and 188 us, King 740 and
-// 711, core-Sersic 1354 and 701; one bulge+disk image 53 and 30.
+// wavefront per tree).  `few`: the family's big trees (four centre pixels a
+// component, or the like) do not fill the GPU, so the tree walk takes blocks of
+// twelve wavefronts, one a CU, and otherwise blocks of four, three a CU.  Four and
+// twelve, measured: 384 survey galaxies (about 150 components a family), Sersic
+// 336 and 188 us, King 740 and 711, core-Sersic 1354 and 701; one bulge+disk
+// image 53 and 30.
 template <int TYPE, bool kJac>
 static int fwd_launch(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps, WorkQueue wq,
                       int split, bool mask, bool few, hipStream_t st)
@@ -27,10 +25,9 @@ static int fwd_launch(int nblocks, const GalaxyDev *gals, const InstDev *insts, 
 }
 
 int launch_subsample_fwd(int type, int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
-                         WorkQueue wq, int split, bool jac, bool mask, int ncomp, hipStream_t st)
+                         WorkQueue wq, int split, bool jac, bool mask, bool few, hipStream_t st)
 {
 	if (nblocks <= 0) return 0;
-	const bool few = ncomp <= kFewComponents;
 #define PA_FWD(T)                                                                                        \
 	case T:                                                                                              \
 		return jac ? fwd_launch<T, true>(nblocks, gals, insts, comps, wq, split, mask, few, st)               \
