@@ -893,16 +893,31 @@ __global__ __launch_bounds__(1024) void k_like_t(const GalaxyDev *__restrict__ g
 	if (g.likefunc != LIKE_T) return;
 	const long n = (long)g.W * g.H;
 	const double N = g.n_region;
+	// kAhead pixels' loads in flight at a time
+	constexpr int kAhead = 8;
+	auto each = [&](auto term) {
+		for (long o = threadIdx.x; o < n; o += (long)kAhead * blockDim.x) {
+			uint8_t in[kAhead];
+			float z[kAhead];
+#pragma unroll
+			for (int u = 0; u < kAhead; ++u) {
+				const long p = o + (long)u * blockDim.x;
+				in[u] = p < n ? g.region[p] : 0;
+				z[u] = I.w[p < n ? p : 0];
+			}
+#pragma unroll
+			for (int u = 0; u < kAhead; ++u)
+				if (in[u]) term((double)z[u]);
+		}
+	};
 	double a = 0;
-	for (long o = threadIdx.x; o < n; o += blockDim.x)
-		if (g.region[o]) a += (double)I.w[o];
+	each([&](double z) { a += z; });
 	const double mean = block_sum(a, sh) / N;
 	a = 0;
-	for (long o = threadIdx.x; o < n; o += blockDim.x)
-		if (g.region[o]) {
-			const double d = (double)I.w[o] - mean;
-			a += d * d;
-		}
+	each([&](double z) {
+		const double d = z - mean;
+		a += d * d;
+	});
 	const double var = block_sum(a, sh) / (N - 1);
 	double dof = 2 * var / (var - 1);
 	bool clamped = false;
@@ -913,15 +928,15 @@ __global__ __launch_bounds__(1024) void k_like_t(const GalaxyDev *__restrict__ g
 	}
 	const bool normal = sf::is_inf(dof);
 	double sl = 0, sc = 0;
-	for (long o = threadIdx.x; o < n; o += blockDim.x)
-		if (g.region[o]) {
-			const double z = (double)I.w[o];
-			if (normal) sl += z * z;
-			else {
-				sl += log1p(z * z / dof);
-				sc += z * z / (dof * (dof + z * z));
-			}
-		}
+	if (normal) {
+		each([&](double z) { sl += z * z; });
+	}
+	else {
+		each([&](double z) {
+			sl += log1p(z * z / dof);
+			if (grad) sc += z * z / (dof * (dof + z * z));
+		});
+	}
 	sl = block_sum(sl, sh);
 	sc = block_sum(sc, sh);
 	double L;
