@@ -130,8 +130,6 @@ __device__ __forceinline__ int tile_class(const Comp &c, const TileRect &r)
 	return 2;
 }
 
-// rows whose masks and G an adjoint render thread loads together
-constexpr int kAdjRows = 4;
 // components whose tile classes a block keeps as bit masks (the ones beyond
 // are taken as class 1)
 constexpr int kCullWords = 64;
@@ -150,14 +148,48 @@ __device__ __forceinline__ double sample_accumulate(const Comp &c, double xp, do
 	const T ca = (T)c.cos_ang, sa = (T)c.sin_ang;
 	const T sq = (T)c.sin_over, cq = (T)c.cos_over;
 	const T fx = o[1], fy = o[2];
-	gs[G_XCEN] += wgt * (double)(fx * -ca + fy * sq);
-	gs[G_YCEN] += wgt * (double)(fx * -sa + fy * -cq);
-	gs[G_ANG] += wgt * (double)((fx * (q * fyp) + fy * (-fxp * iq)) * (T(3.14159265358979323846) / T(180)));
-	gs[G_AXRAT] += wgt * (double)(fy * (-fyp * iq));
-	if (c.grad_box) gs[G_BOX] += wgt * (double)o[3];
+	gs[G_XCEN] = fma(wgt, (double)(fx * -ca + fy * sq), gs[G_XCEN]);
+	gs[G_YCEN] = fma(wgt, (double)(fx * -sa + fy * -cq), gs[G_YCEN]);
+	gs[G_ANG] = fma(wgt, (double)((fx * (q * fyp) + fy * (-fxp * iq)) * (T(3.14159265358979323846) / T(180))), gs[G_ANG]);
+	gs[G_AXRAT] = fma(wgt, (double)(fy * (-fyp * iq)), gs[G_AXRAT]);
+	if (c.grad_box) gs[G_BOX] = fma(wgt, (double)o[3], gs[G_BOX]);
 #pragma unroll
-	for (int s = 0; s < n_shape(TYPE); ++s) gs[G_S0 + s] += wgt * (double)o[4 + s];
+	for (int s = 0; s < n_shape(TYPE); ++s) gs[G_S0 + s] = fma(wgt, (double)o[4 + s], gs[G_S0 + s]);
 	return (double)o[0];
+}
+
+// The same for a Sersic sample without box: the FP32 derivatives from the
+// value's own logarithm and exponentials, with no powers or signs of the
+// general form (and two logarithms more where d / d box is wanted).  A 500-source
+// field's steep cores, every slot wanted: 2.27 -> 2.01 ms.
+__device__ __forceinline__ double sersic_accumulate(const Comp &c, double xp, double yp, double wgt, double *gs)
+{
+#pragma clang fp contract(fast)
+	const float x = (float)xp, y = (float)yp;
+	float base, l2, rf;
+	const float f = sersic_parts_f32(c, x, y, base, l2, rf);
+	if (!(base > 0.f)) return (double)f;  // the centre: every derivative is 0
+	const float bfr = c.f.bn * f * rf * c.f.inv_n;
+	const float k = -bfr * c.f.inv_re2 * __builtin_amdgcn_rcpf(base);
+	const float fx = k * x, fy = k * y;
+	const float q = c.f.axrat, iq = c.f.inv_axrat;
+	gs[G_XCEN] = fma(wgt, (double)(fx * -c.f.cos_ang + fy * c.f.sin_over), gs[G_XCEN]);
+	gs[G_YCEN] = fma(wgt, (double)(fx * -c.f.sin_ang + fy * -c.f.cos_over), gs[G_YCEN]);
+	gs[G_ANG] = fma(wgt, (double)((fx * (q * y) + fy * (-x * iq)) * (3.14159265358979323846f / 180.f)), gs[G_ANG]);
+	gs[G_AXRAT] = fma(wgt, (double)(fy * (-y * iq)), gs[G_AXRAT]);
+	if (c.grad_box) {
+		// d base / dB = pu ln u + pv ln v with u = |x| / re, pu = u^2, at B = 2;
+		// ln u = ln(u^2) / 2
+		const float pu = (x * x) * c.f.inv_re2, pv = (y * y) * c.f.inv_re2;
+		const float d2 = (pu > 0.f ? pu * log2_fast(pu) : 0.f) + (pv > 0.f ? pv * log2_fast(pv) : 0.f);
+		const float half_ln2 = 0.5f * float(kLn2);
+		// inv_nB (dbase_dB / base - ln(base) / B), inv_nB = inv_n / 2
+		const float t = 0.5f * half_ln2 * (d2 * __builtin_amdgcn_rcpf(base) - l2);
+		gs[G_BOX] = fma(wgt, (double)(-bfr * t), gs[G_BOX]);
+	}
+	gs[G_S0] = fma(wgt, (double)(bfr * c.f.inv_re), gs[G_S0]);
+	gs[G_S1] = fma(wgt, (double)(f * (-c.f.dbn * (rf - 1.f) + c.f.bn * rf * (l2 * float(kLn2)) * c.f.inv_n * c.f.inv_2n)), gs[G_S1]);
+	return (double)f;
 }
 
 // Where a King or Ferrer cell lies against its profile's cut-off (rt, rout),
@@ -600,12 +632,14 @@ __global__ __launch_bounds__(256, kJac && (TYPE == SERSIC || TYPE == MOFFAT || T
 // with a wavefront each.
 //
 // Bound by VALU issue on long lists and by latency on short ones, so the group
-// is as wide as the list leaves room for in kRootLanes lanes (four wavefronts
-// per SIMD): one lane per entry from 131,073 entries (no exchange, 0.63 ms for
-// the 1.3 M of a batch of 1024 bulge+disk images), a whole wavefront below
-// 4,097.  Entries are dealt out by index: asking a counter cost 11.6 ns per
-// wavefront (95 us for 8,192 of them, also with nothing to do).
-constexpr int kRootLanes = 1 << 18;
+// is as wide as the list leaves room for in kRootLanes lanes: one lane per entry
+// from 524,289 entries (no exchange, 0.53 ms for the 1.3 M of a batch of 1024
+// bulge+disk images), a whole wavefront up to 16,384.  At 2^18 lanes the families
+// of 384 survey galaxies took 172 to 752 us, at 2^20 91 to 521; at 2^21 the 300 k
+// entries of 256 likelihoods 127 us (110, 107).  Entries are dealt out by index:
+// asking a counter cost 11.6 ns per wavefront (95 us for 8,192 of them, also with
+// nothing to do).
+constexpr int kRootLanes = 1 << 20;
 constexpr int kBigTree = 8;
 
 template <int TYPE, bool kJac>
@@ -1004,6 +1038,7 @@ __global__ __launch_bounds__(256) void k_adj_render(const GalaxyDev *__restrict_
                                                     const int *__restrict__ grp_off, int ninst, int grp, int parts,
                                                     const Comp *__restrict__ comps, double *grad_acc)
 {
+	constexpr int kAdjRows = 4;  // rows whose masks and G a thread loads together
 	__shared__ double red[4][NGRAD];
 	__shared__ unsigned long long hit[kCullWords];
 	const int b = blockIdx.x / parts, part = blockIdx.x - b * parts;
@@ -1071,7 +1106,9 @@ __global__ __launch_bounds__(256) void k_adj_render(const GalaxyDev *__restrict_
 					const double xp = xr * c.cos_ang + yr * c.sin_ang;
 					const double yp = -xr * c.sin_over + yr * c.cos_over;
 					const double wq = (double)Gq * c.flux_scale;
-					vsum += wq * sample_accumulate<float, TYPE>(c, xp, yp, wq, gl);
+					const double v = TYPE == SERSIC && !c.boxy ? sersic_accumulate(c, xp, yp, wq, gl)
+					                                           : sample_accumulate<float, TYPE>(c, xp, yp, wq, gl);
+					vsum = fma(wq, v, vsum);
 				  }
 				}
 			}
