@@ -120,7 +120,8 @@ int profit_amd_output_dims(const profit_amd_model_desc *model, const profit_amd_
 
 /* Releases the device set-ups (buffers, tile lists, FFT spectra) that
  * repeated profit_amd_make_model calls with the same image geometry, PSF and
- * calc region reuse.  Replaces R_profit_clear_cache (src/r_profit.cpp:822-825),
+ * calc region reuse, and those that repeated profit_amd_convolve calls of one
+ * geometry reuse.  Replaces R_profit_clear_cache (src/r_profit.cpp:822-825),
  * which clears libprofit's OpenCL kernel cache. */
 int profit_amd_clear_cache(void);
 

@@ -329,13 +329,15 @@ Engine::TuneReport Engine::autotune(const ProfileParams *params, int reps, bool 
 // N1 x N2 frame and transformed with the same FFT kernels.
 void Engine::ensure_fft_spectra()
 {
-	int twn = 2;
+	int twn = 2, largest = 2;
 	for (const auto &g : gal_host_)
 		if (g.conv_kind == CK_FFT) {
 			const int n1 = galaxy_frame(g.DW, g.Kx, g.padx), n2 = galaxy_frame(g.DH, g.Ky, g.pady);
 			twn = std::max(twn, std::max(n1, n2));
+			// the limit holds for canvas and kernel together
+			largest = std::max({largest, fft_frame(g.DW + g.Kx), fft_frame(g.DH + g.Ky)});
 		}
-	if (twn > 4096) throw std::invalid_argument("FFT frame above 4096 points per axis is not supported");
+	if (largest > 4096) throw std::invalid_argument("FFT frame above 4096 points per axis is not supported");
 	if (twn != twn_) {
 		const std::vector<double2> tw = twiddles(twn);
 		d_tw_.alloc(tw.size() * sizeof(double2));
