@@ -89,7 +89,8 @@ PA_HD void default_params(int type, ProfileParams *p)
 }
 
 // Sersic r_factor specialisations (sersic.cpp:79-163)
-enum SersicKind : int32_t { K_HALF = 0, K_ONE, K_TWO, K_THREE, K_FOUR, K_EIGHT, K_SIXTEEN, K_GENERAL };
+// and, for a core-Sersic, whether its FP32 forms are those of a sharp transition (sharp_at)
+enum SersicKind : int32_t { K_HALF = 0, K_ONE, K_TWO, K_THREE, K_FOUR, K_EIGHT, K_SIXTEEN, K_GENERAL, K_SHARP };
 
 // Device descriptor of one component after initial_calculations.
 struct Comp {
@@ -118,7 +119,7 @@ struct Comp {
 	// enter FP32 arithmetic as scalar operands without conversions; aux per
 	// family: King 1/rc, 1/a, C = (1 + (rt/rc)^2)^(-1/a), log2(1 + (rt/rc)^2)
 	// and C / (1 + (rt/rc)^2); Moffat and Ferrer 1/rscale; core-Sersic
-	// log2 rb, rb^a, re^-a, 1/(n a) and log2 re
+	// log2 rb, rb^a, re^-a (sharp: 1/rb, 1/a), 1/(n a) and log2 re
 	struct F32 {
 		float cos_ang, sin_ang, cos_over, sin_over, axrat, inv_axrat;
 		float inv_re, inv_re2, inv_n, inv_nB, inv_2n, bn, dbn;
@@ -262,6 +263,15 @@ __device__ __forceinline__ float pow_acc(float x, float e)
 	const float l = log2_kl(x, &k);
 	const float p = e * k;
 	return exp2_hl(p, fmaf(e, l, fmaf(e, k, -p)));
+}
+// x^e y^g for x, y > 0, with one exponential and the rounding of the exponents' sum kept
+__device__ __forceinline__ float pow2_acc(float x, float e, float y, float g)
+{
+	float kx, ky;
+	const float lx = log2_kl(x, &kx), ly = log2_kl(y, &ky);
+	const float p = e * kx, q = g * ky, hi = p + q, t = hi - p;
+	const float lo = ((p - (hi - t)) + (q - t)) + (fmaf(e, kx, -p) + fmaf(g, ky, -q));
+	return exp2_hl(hi, fmaf(e, lx, fmaf(g, ly, lo)));
 }
 __device__ __forceinline__ float exp_acc(float x)
 {
@@ -468,12 +478,61 @@ PA_HDI T brokenexp_dlog(T r, T h1, T h2, T rb, T a, T *ds)
 	return -T(1) / h1 + expo * sig;
 }
 
+// The core-Sersic profile in FP32 where its powers r^a, rb^a, re^a or (r/rb)^-a leave
+// FP32's range (K_SHARP; a = 11 and r = rb / 4000: 3e39): from x = (min(r, rb) /
+// max(r, rb))^a <= 1 and M = max(r, rb),
+//   f = (r/rb)^-b [r < rb] (1 + x)^(b/a) exp(-bn (M/re)^(1/n) (1 + x)^(1/(n a))).
+// sharp_at is the value (a few ulps for any exponent, as pow_t gives them), sharp_f32
+// the same from one logarithm of r (plain forms) and, with ds non-null, d ln f / d
+// shape (ds[0..4]) and d ln f / dr in *dlog.  An ordinary transition keeps the direct
+// forms, which take fewer operations on the way to the derivatives.
+__device__ __forceinline__ float sharp_at(const Comp &c, float r)
+{
+	const Comp::F32 &k = c.f;
+	const float a = k.s[3], b = k.s[4], u = r / k.s[1];
+	const bool in = u < 1.f;
+	const float q = 1.f + pow_t<float>(u, in ? a : -a);
+	const float W = pow2_acc((in ? k.s[1] : r) / k.s[0], k.inv_n, q, k.aux[3]);
+	return (in ? pow_t<float>(u, -b) : 1.f) * pow_t<float>(q, b / a) * exp_t<float>(-k.bn * W);
+}
+
+__device__ __forceinline__ float sharp_f32(const Comp &c, float r, float *ds, float *dlog)
+{
+	const Comp::F32 &k = c.f;
+	const float re = k.s[0], rb = k.s[1], a = k.s[3], b = k.s[4], bn = k.bn;
+	const float lrb = k.aux[0], ia = k.aux[2], ina = k.aux[3], lre = k.aux[4];
+	const float lr = log2_fast(r), d = lr - lrb;
+	const bool in = d < 0.f;
+	const float x = exp2_fast(-a * fabsf(d)), q = 1.f + x, lq = log2_fast(q);
+	// log2 of 1 + (r/rb)^-a and of (r^a + rb^a) / re^a
+	const float lQ = in ? lq - a * d : lq, lS2 = a * ((in ? lrb : lr) - lre) + lq;
+	const float W = exp2_fast(k.inv_n * ((in ? lrb : lr) - lre) + ina * lq);
+	const float e1 = b == 0.f ? 0.f : (in ? -b * d : 0.f) + b * ia * lq;
+	const float f = exp2_fast(e1 - bn * W * float(kLog2e));
+	if (ds) {
+		const float ln2 = float(kLn2), inn = k.inv_n, lS = lS2 * ln2;
+		const float irb = k.aux[1], ir = __builtin_amdgcn_rcpf(r);
+		// the shares of rb^a and r^a in their sum
+		const float iq = __builtin_amdgcn_rcpf(q), xq = x * iq;
+		const float gb = in ? iq : xq, gr = in ? xq : iq;
+		ds[0] = bn * W * inn * k.inv_re;
+		ds[1] = (b * gb - bn * W * gb * inn) * irb;
+		ds[2] = -k.dbn * W + bn * W * lS * ina * inn;
+		const float dlnS_da = (gr * lr + gb * lrb) * ln2 - lre * ln2;
+		ds[3] = -(b * ia * ia) * lQ * ln2 - b * ia * gb * d * ln2 - bn * W * (dlnS_da * ina - lS * ina * ia);
+		ds[4] = lQ * ln2 * ia;
+		*dlog = (-b * gb - bn * W * gr * inn) * ir;
+	}
+	return f;
+}
+
 // The core-Sersic profile in FP32 from one logarithm of r:
 // t = (r/rb)^-a, Q = 1 + t, S = (r^a + rb^a) / re^a, W = S^(1/(n a)),
 // f = Q^(b/a) exp(-bn W).  With ds non-null it also gives d ln f / d shape
 // (ds[0..4]) and returns d ln f / dr in *dlog, as coresersic_dlog does.
 __device__ __forceinline__ float coresersic_f32(const Comp &c, float r, float *ds, float *dlog)
 {
+	if (c.kind == K_SHARP) return sharp_f32(c, r, ds, dlog);
 	const Comp::F32 &k = c.f;
 	const float re = k.s[0], rb = k.s[1], a = k.s[3], b = k.s[4], bn = k.bn;
 	const float lrb = k.aux[0], rba = k.aux[1], rea = k.aux[2], ina = k.aux[3], lre = k.aux[4];
@@ -570,7 +629,10 @@ PA_HDI T eval_at(const Comp &c, T x, T y)
 			const float u = r * f.aux[0];
 			return pow_t<float>(pow_t<float>(1.f + u * u, -f.aux[1]) - f.aux[2], f.s[2]);
 		}
-		case CORESERSIC: return coresersic_core<float>(c, boxy_r<float>(c, x, y));
+		case CORESERSIC: {
+			const float r = boxy_r<float>(c, x, y);
+			return c.kind == K_SHARP ? sharp_at(c, r) : coresersic_core<float>(c, r);
+		}
 		case BROKENEXP: return brokenexp_core<float>(boxy_r<float>(c, x, y), f.s[0], f.s[1], f.s[2], f.s[3]);
 		default: return 0.f;
 		}
@@ -1246,11 +1308,20 @@ PA_HD int setup_component(const ProfileParams &p, double magzero, double sx, dou
 	for (int i = 0; i < 5; ++i) f.s[i] = (float)c->s[i];
 	for (int i = 0; i < 5; ++i) f.aux[i] = 0.f;
 	if (p.type == CORESERSIC) {
+		// radii from 1e-8 (the FP32 positions' resolution) to the largest drawn
+		const double far = ::fmax(::fmax(s[0], s[1]), rmax > 0 ? c->rmax_r : 1e5);
+		if (s[3] * (27 + ::fmax(::log2(far), 0.)) > 126) c->kind = K_SHARP;
+		f.inv_re = (float)(1 / s[0]);
+		f.inv_n = (float)(1 / s[2]);
 		f.aux[0] = (float)::log2(s[1]);
 		f.aux[1] = (float)::pow(s[1], s[3]);
 		f.aux[2] = (float)::pow(s[0], -s[3]);
 		f.aux[3] = (float)(1 / (s[2] * s[3]));
 		f.aux[4] = (float)::log2(s[0]);
+		if (c->kind == K_SHARP) {
+			f.aux[1] = (float)(1 / s[1]);
+			f.aux[2] = (float)(1 / s[3]);
+		}
 	}
 	else if (p.type == KING) {
 		f.aux[0] = (float)(1 / s[0]);
