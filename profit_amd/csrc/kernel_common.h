@@ -215,27 +215,53 @@ __device__ __forceinline__ int cut_zone(const Comp &c, float x, float y, float a
 	return band_c || band_t ? 1 : -1;
 }
 
+// The component's accuracy, guard band and near radius (Comp::F32), read once per
+// tree or entry: where the test may not run, or behind a barrier, the component's
+// fields would be loaded again for every cell or round (root pass of 300,000 entries
+// 103 -> 117 us, tree walk 167 -> 182).
+struct RefineLimits {
+	float acc, band, rnear;
+};
+
+__device__ __forceinline__ RefineLimits refine_limits(const Comp &c) { return RefineLimits{c.f.acc, c.f.band, c.f.rnear}; }
+
+// What the refinement test of a node's cells needs besides a cell's value: the test
+// point's offset, the limits and the squared profile radius below which a cell is
+// undecided.
+struct RefineTest {
+	float dyp, acc, band, near2;
+};
+
+__device__ __forceinline__ RefineTest refine_test(const RefineLimits &l, float dyp, float xbin)
+{
+	const float near = fmaxf(0.05f * xbin, l.rnear);
+	return RefineTest{dyp, l.acc, l.band, near * near};
+}
+
 // libprofit's refinement test |test - val| > acc * val (radial.cpp:92-100),
 // evaluated in FP32 at FP32 cell positions: 1 refine, 0 leaf, 2 undecided.
-// The decision is taken only when the FP32 margin lies outside a guard band
-// of 2.5e-4 * val around the threshold; the FP32 evaluation errors (values and
-// positions: a few parts in 1e7 of val, and at worst, an exponent of 45 in the
-// core-Sersic, 3e-5) are far inside it, so a decision taken here equals the FP64
-// one.  A band of 1e-3 sent four times the cells to FP64, which was half the
-// root pass of a King family (1.64 -> 0.80 ms for 77 of them).  King and Ferrer cells beyond their cut-off are
-// leaves; those near it are undecided (cut_zone).  Undecided cells take
-// refine_cell64 at libprofit's own FP64 cell position.
+// The decision is taken only when the FP32 margin lies outside the component's guard
+// band, which covers the FP32 errors of values and positions (guard_band), so it equals
+// the FP64 one.  The positions err by 6e-8 of the node, which is more than the band
+// allows for next to the profile's centre: a cell within 5% of a cell of it is
+// undecided, as is one so close that a box's powers underflow (RefineTest::near2).  King and
+// Ferrer cells beyond their cut-off are leaves; those near it are undecided (cut_zone).
+// Undecided cells take refine_cell64 at libprofit's own FP64 cell position, and its
+// value if they are leaves.  Ordinary shapes have a band of 2.5e-4; one of 1e-3 for all
+// sent four times the cells to FP64, half the root pass of a King family (77 of them:
+// 1.64 ms, 0.80 now), with the same image errors against FP64 (the FP64 leaf values
+// within 1e-3 change them by less than 1%).
 template <int TYPE = -1>
-__device__ __forceinline__ int refine_cell32(const Comp &c, float xp, float yp, float dyp, float v32)
+__device__ __forceinline__ int refine_cell32(const Comp &c, float xp, float yp, const RefineTest &rt, float v32)
 {
-	const float ax = fabsf(xp), ay = fabsf(yp) + fabsf(dyp);
+	const float ax = fabsf(xp), ay = fabsf(yp) + fabsf(rt.dyp);
 	const int zone = cut_zone<TYPE>(c, xp, yp, ax, ay);
 	if (zone == 0) return 0;
 	if (zone == 1) return 2;
 	const float t32 = eval_fast<TYPE>(c, ax, ay);
-	const float margin = fabsf(t32 - v32) - c.f.acc * v32;
-	if (v32 > 1e-30f && isfinite(margin) && fabsf(margin) > 2.5e-4f * v32) return margin > 0.f ? 1 : 0;
-	return 2;
+	const float margin = fabsf(t32 - v32) - rt.acc * v32;
+	if (!(v32 > 1e-30f && isfinite(margin) && fabsf(margin) > rt.band * v32 && xp * xp + yp * yp >= rt.near2)) return 2;
+	return margin > 0.f ? 1 : 0;
 }
 
 // the FP64 refinement test; *v64 receives the FP64 value
@@ -320,15 +346,17 @@ __device__ __forceinline__ void sersic_jac_f32(const Comp &c, float xp, float yp
 }
 
 // A node of the recursion: its FP64 bounds (libprofit's), the resolution,
-// and the FP32 cell size, test offset and lower corner relative to the
+// and the FP32 cell size, refinement test and lower corner relative to the
 // component centre that the FP32 cell positions use.
 struct Node {
 	double x0, x1, y0, y1;
 	int res;
-	float inv_res, xbin, ybin, dyp, ox, oy;
+	float inv_res, xbin, ybin, ox, oy;
+	RefineTest test;
 };
 
-__device__ __forceinline__ Node make_node(const Comp &c, double x0, double x1, double y0, double y1, int res)
+__device__ __forceinline__ Node make_node(const Comp &c, const RefineLimits &lim, double x0, double x1, double y0,
+                                          double y1, int res)
 {
 	Node n;
 	n.x0 = x0;
@@ -339,7 +367,7 @@ __device__ __forceinline__ Node make_node(const Comp &c, double x0, double x1, d
 	n.inv_res = kInvRes[res];
 	n.xbin = (float)(x1 - x0) * n.inv_res;
 	n.ybin = (float)(y1 - y0) * n.inv_res;
-	n.dyp = -n.xbin * c.f.sin_over + n.ybin * c.f.cos_over;
+	n.test = refine_test(lim, -n.xbin * c.f.sin_over + n.ybin * c.f.cos_over, n.xbin);
 	n.ox = (float)(x0 - c.xc);
 	n.oy = (float)(y0 - c.yc);
 	return n;
@@ -372,7 +400,7 @@ __device__ __forceinline__ bool cell_step(const Comp &c, const Node &n, int cell
 	float v32, s_base = 0.f, s_l2 = 0.f, s_rf = 0.f;
 	if (fuse) v32 = sersic_parts_f32(c, xp, yp, s_base, s_l2, s_rf);
 	else v32 = eval_at<float, TYPE>(c, xp, yp);
-	int dec = recurse ? refine_cell32<TYPE>(c, xp, yp, n.dyp, v32) : 0;
+	int dec = recurse ? refine_cell32<TYPE>(c, xp, yp, n.test, v32) : 0;
 	double v64 = 0;
 	bool have64 = false;
 	if (dec == 2) {
@@ -423,9 +451,10 @@ __device__ __forceinline__ void walk_pixel(const Comp &c, WalkLevel *L, int lane
 	int level = 0;
 	double nx0 = x0, nx1 = x1, ny0 = y0, ny1 = y1;
 	double weight = inv_cells;
+	const RefineLimits lim = refine_limits(c);
 	for (;;) {
 		const bool recurse = res > 1 && level < maxrec;
-		const Node n = make_node(c, nx0, nx1, ny0, ny1, res);
+		const Node n = make_node(c, lim, nx0, nx1, ny0, ny1, res);
 		// the cells in chunks of 64 (one per lane); lane 0 stores each chunk's
 		// refine mask with the node, and `any` gathers them.  A node with no
 		// cell to refine is not stored: the search below starts under it.
@@ -683,7 +712,7 @@ __global__ __launch_bounds__(256) void k_subsample_root(const GalaxyDev *__restr
 				wide = ncell > 64;
 				const bool recurse = res > 1 && c.maxrec > 0;
 				const bool fuse = kJac && TYPE == SERSIC && !c.boxy && !c.grad_box;
-				const Node n = make_node(c, x - hx, x + hx, y - hy, y + hy, res);
+				const Node n = make_node(c, refine_limits(c), x - hx, x + hx, y - hy, y + hy, res);
 				const double weight = kInvCells[res];
 				const bool fp64 = g.render_fp64 != 0;
 				for (int cell = sub; cell < ncell; cell += grp)
@@ -770,6 +799,7 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack<W> &S, int ba
 	const bool fuse = kJac && TYPE == SERSIC && !c.boxy && !c.grad_box;
 	const int ncell = res * res, wv = tid >> 6, lane = tid & 63;
 	const double inv_cells = kInvCells[res];
+	const RefineLimits lim = refine_limits(c);
 	// the thread's node of a round and its first cell
 	const int per = ncell >= T ? 1 : T / ncell;
 	const int slot = ncell >= T ? 0 : tid / ncell;
@@ -802,7 +832,7 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack<W> &S, int ba
 		const int r = base + top - 1 - (on ? slot : 0);
 		const typename TreeStack<W>::Share &Q = S.q[r / kTreeShare];
 		const int k = r % kTreeShare;
-		const Node node = make_node(c, Q.x0[k], Q.x1[k], Q.y0[k], Q.y1[k], res);
+		const Node node = make_node(c, lim, Q.x0[k], Q.x1[k], Q.y0[k], Q.y1[k], res);
 		const double weight = Q.weight[k];
 		const int level = Q.level[k];
 		const bool recurse = res > 1 && level < maxrec;

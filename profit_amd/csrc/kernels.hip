@@ -551,7 +551,7 @@ __global__ __launch_bounds__(256) void k_subsample_nodes(const GalaxyDev *__rest
 					float xp, yp;
 					cell_pos32(c, (float)(nx0 - c.xc), (float)(ny0 - c.yc), (float)xbin, (float)ybin, ci, cj, &xp, &yp);
 					const float v32 = eval_at<float>(c, xp, yp);
-					int dec = refine_cell32(c, xp, yp, (float)dyp, v32);
+					int dec = refine_cell32(c, xp, yp, refine_test(refine_limits(c), (float)dyp, (float)xbin), v32);
 					if (dec == 2) {
 						double xp64, yp64, v64;
 						cell_pos64(c, nx0, ny0, chx, chy, ci, cj, &xp64, &yp64);

@@ -127,6 +127,8 @@ struct Comp {
 		float rmax2, rsw2;  // (rscale_max rscale)^2, (rscale_switch rscale)^2
 		float s[5];
 		float aux[5];
+		float band;   // guard band of the FP32 refinement test (guard_band)
+		float rnear;  // profile radius below which that test leaves a cell to FP64
 	} f;
 };
 
@@ -573,7 +575,7 @@ __device__ __forceinline__ bool near_cut_fp64(const Comp &c, float xp, float yp)
 
 // The profile in FP32 with the plain transcendental forms (2^(e log2 x),
 // errors of about |e log2 x| ulps): the refinement test's second value,
-// which only has to fall on the right side of a guard band of 2.5e-4.
+// which only has to fall on the right side of the guard band.
 template <int TYPE = -1>
 __device__ __forceinline__ float eval_fast(const Comp &c, float x, float y)
 {
@@ -1005,6 +1007,84 @@ PA_HD double lum_gradient(const Comp &c, int w, sf::QuadState *qs)
 	return -d / c.lumtot;
 }
 
+// The largest profile radius of a cell of the sub-sampled pixels (pixel centres
+// within rscale_switch) or of its test point.
+PA_HDI float guard_radius(const Comp &c, double sx, double sy)
+{
+	return (float)(c.rsw_r + (0.71 + 1.42 / c.res) * ::fmax(sx, sy) * c.inv_axrat);
+}
+
+// Guard band of the FP32 refinement test (refine_cell32), relative to the cell's
+// value: twice what the FP32 margin |test - val| - acc val can be off by near its
+// zero, over the cells up to profile radius R, and at least kMinBand.
+//
+// In units of 2^-23: the radius errs by `rho` (the rotation's coordinates cancel along
+// a thin ellipse; a box's powers), which counts times d ln f / d ln r; the powers and
+// exponentials of the value err by a few units times the exponents behind them, the
+// plain forms 2^(x log2 y) of the test's second value by |x log2 y| units; King's A - C
+// and Ferrer's 1 - t^(2-b) divide that by what their subtraction leaves at 0.97 of the
+// cut (0.99 where the test's value, beyond the cell's, can be as large), which cut_zone
+// bounds.  The decision asks for values above 1e-30, so an exponent counts up to 69.
+//
+// Over 60 million cells of random components, each result of the transcendental unit
+// off by up to one unit, the worst error is 0.94 of half the band (Ferrer; King 0.88,
+// Sersic 0.75).  A fixed band falls short: King at a = 9.7 errs by 5e-4, Ferrer at
+// b = 1.95 by 6e-3.  Ordinary shapes stay at kMinBand, ten times their error.
+constexpr float kMinBand = 2.5e-4f;
+PA_HDI float guard_band(const Comp &c, float R)
+{
+	const Comp::F32 &f = c.f;
+	const float e = 1.2e-7f, ln2 = float(kLn2);
+	auto ln = [&](float x) { return ::log2f(x) * ln2; };
+	auto power = [&](float x, float y) { return ::exp2f(y * ::log2f(x)); };
+	const float b2 = f.box + 2.f;
+	float rho = 3.f + f.inv_axrat;
+	if (c.boxy) rho = 1.5f * (b2 < 1.f ? power(rho * e, b2) / (b2 * e) : rho) + 6.f + 6.f / b2;
+	float err = 0.f;  // in units of e
+	switch (c.type) {
+	case SERSIC: {
+		const float rf = fminf(power(R * f.inv_re, f.inv_n), 69.f / f.bn + 1.f);
+		const float E = f.bn * rf;
+		err = E * (3.f + rho * f.inv_n + 2.f * fmaxf(ln(rf), 0.f)) + 3.f * f.bn + 3.f;
+		break;
+	}
+	case MOFFAT: {
+		const float t = R * f.aux[0], w = t * t / (1.f + t * t);
+		err = f.s[1] * (1.2f + 2.f * rho * w) + 2.f * fminf(69.f, f.s[1] * ln(1.f + t * t)) + 4.f;
+		break;
+	}
+	case FERRER: {
+		const float p = 2.f - f.s[2], a = f.s[1];
+		const float t = fminf(R * f.aux[0], a < 1.f ? .99f : .97f), tp = power(t, p);
+		const float g = fmaxf(1.f - tp, 0.f) + 1e-30f;
+		err = a * (8.f + 1.3f * p * rho) * tp / g + a / p + 2.f * fminf(69.f, -a * ln(g)) + 4.f;
+		break;
+	}
+	case KING: {
+		const float a = f.s[2], ia = f.aux[1], r = fminf(R, (a < 1.f ? .99f : .97f) * f.s[1]), u = r * f.aux[0];
+		const float lq = ln(1.f + u * u), A = ::exp2f(-ia * lq / ln2), D = fmaxf(A - f.aux[2], 0.f) + 1e-30f;
+		err = a * (A / D) * (4.f + 3.f * ia * lq + ia * (1.f + 2.f * rho * u * u / (1.f + u * u))) +
+		      2.f * fminf(69.f, -a * ln(D)) + 4.f;
+		break;
+	}
+	case CORESERSIC: {
+		const float re = f.s[0], rb = f.s[1], a = f.s[3], b = fabsf(f.s[4]), in = a * f.aux[3];
+		const float M = fmaxf(R, rb), W = power(M / re, in) * power(2.f, f.aux[3]);
+		const float E = f.bn * W, L = fabsf(ln(R)) + fabsf(ln(rb)) + fabsf(ln(re)) + 3.f;
+		err = b * (2.f * L + rho) + 4.f * b / a + E * (9.f * f.aux[3] + (rho + 2.f * L) * in + 3.f + 3.f * fabsf(ln(W)));
+		if (f.s[4] < 0.f) err *= 1.f + f.acc;  // the value may rise outwards
+		break;
+	}
+	case BROKENEXP: {
+		const float h1 = f.s[0], h2 = f.s[1], rb = f.s[2], a = f.s[3], d = fabsf(1.f / h1 - 1.f / h2);
+		err = R / h1 * (3.f + rho) + d * (R * (3.f + rho) + rb + 5.f / a);
+		break;
+	}
+	default: break;
+	}
+	return fmaxf(kMinBand, 2.f * e * err);
+}
+
 // grad_integrals = false leaves the slots of lum_gradient to a separate pass.
 // kWave (device code): a whole wavefront runs the set-up with the same
 // arguments, and the luminosity integrals spread their Kronrod points over
@@ -1334,6 +1414,8 @@ PA_HD int setup_component(const ProfileParams &p, double magzero, double sx, dou
 	else if (p.type == MOFFAT || p.type == FERRER) {
 		f.aux[0] = (float)(1 / c->rscale);
 	}
+	f.rnear = c->boxy ? ::exp2f(-100.f / (f.box + 2.f)) * (p.type == SERSIC ? fmaxf(1.f, (float)s[0]) : 1.f) : 0.f;
+	f.band = guard_band(*c, guard_radius(*c, sx, sy));
 	return SE_OK;
 }
 

@@ -44,7 +44,7 @@ template <int TYPE>
 static void recurse(const Comp &c, double x0, double x1, double y0, double y1, double w, int res, int maxrec, int level,
                     double &sum, float *gj, long &leaves)
 {
-	const Node n = make_node(c, x0, x1, y0, y1, res);
+	const Node n = make_node(c, refine_limits(c), x0, x1, y0, y1, res);
 	const bool fuse = TYPE == SERSIC && !c.boxy && !c.grad_box;
 	for (int cell = 0; cell < res * res; ++cell) {
 		if (!cell_step<TYPE, true>(c, n, cell, res > 1 && level < maxrec, false, fuse, w, sum, gj)) {
