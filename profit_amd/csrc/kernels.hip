@@ -53,7 +53,10 @@ __global__ __launch_bounds__(256, 2) void k_setup(const ProfileParams *__restric
 	Comp out;
 	int e = setup_component<true>(params[c], g.magzero, g.sx, g.sy, g.img_sx, g.img_sy, g.padx, g.pady, &qs, &out,
 	                              false);
-	if (e == SE_OK && params[c].type == POINTSRC && !g.psf_pt) e = SE_NO_PSF;
+	if (e == SE_OK && params[c].type == POINTSRC && !g.psf_pt) {
+		e = SE_NO_PSF;
+		undrawn_component(&out);
+	}
 	out.grad_box = g.grad_box;
 	out.instance = inst;
 	// every lane holds the same result; lane 0 stores it

@@ -1085,14 +1085,25 @@ PA_HDI float guard_band(const Comp &c, float R)
 	return fmaxf(kMinBand, 2.f * e * err);
 }
 
+// A component that draws nothing, whatever kernel meets it: no family's type, and
+// every pixel beyond its rscale_max.
+PA_HD void undrawn_component(Comp *c)
+{
+	*c = Comp{};
+	c->type = NULLPROF;
+	c->has_rmax = 1;
+	c->rmax_r = -1;
+	c->f.rmax2 = -1.f;
+}
+
 // grad_integrals = false leaves the slots of lum_gradient to a separate pass.
 // kWave (device code): a whole wavefront runs the set-up with the same
 // arguments, and the luminosity integrals spread their Kronrod points over
-// its lanes (sf::kronrod).
-template <bool kWave = false>
-PA_HD int setup_component(const ProfileParams &p, double magzero, double sx, double sy, double img_sx,
-                          double img_sy, unsigned offx, unsigned offy, sf::QuadState *qs, Comp *c,
-                          bool grad_integrals = true)
+// its lanes (sf::kronrod).  On an error *c is left unfinished (setup_component).
+template <bool kWave>
+PA_HD int form_component(const ProfileParams &p, double magzero, double sx, double sy, double img_sx,
+                         double img_sy, unsigned offx, unsigned offy, sf::QuadState *qs, Comp *c,
+                         bool grad_integrals)
 {
 	const int verr = validate_params(p);
 	if (verr != SE_OK) return verr;
@@ -1417,6 +1428,19 @@ PA_HD int setup_component(const ProfileParams &p, double magzero, double sx, dou
 	f.rnear = c->boxy ? ::exp2f(-100.f / (f.box + 2.f)) * (p.type == SERSIC ? fmaxf(1.f, (float)s[0]) : 1.f) : 0.f;
 	f.band = guard_band(*c, guard_radius(*c, sx, sy));
 	return SE_OK;
+}
+
+// form_component, and on an error a component that draws nothing: the evaluation's
+// kernels have been launched by the time the error is seen, and a resolution or
+// recursion depth beyond the limits would take the walks outside their tables.
+template <bool kWave = false>
+PA_HD int setup_component(const ProfileParams &p, double magzero, double sx, double sy, double img_sx,
+                          double img_sy, unsigned offx, unsigned offy, sf::QuadState *qs, Comp *c,
+                          bool grad_integrals = true)
+{
+	const int e = form_component<kWave>(p, magzero, sx, sy, img_sx, img_sy, offx, offy, qs, c, grad_integrals);
+	if (e != SE_OK) undrawn_component(c);
+	return e;
 }
 
 #undef PA_HD
