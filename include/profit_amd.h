@@ -298,6 +298,11 @@ int profit_amd_engine_stats(profit_amd_engine *engine, double *stage_ms, int64_t
  * stage (kernel_ms[3..5]), and the number of evaluations each was timed over
  * (calls[0..1]).  No counterpart in the reference (measurement). */
 int profit_amd_engine_fft_stats(profit_amd_engine *engine, double *kernel_ms, int64_t *calls);
+/* Sub-pixel trees of the last evaluation that overflowed the tree walk's stack
+ * (and were walked by masks instead), and the evaluations that had to run again
+ * because a work list or a tree did not fit.  No counterpart in the reference
+ * (measurement). */
+int profit_amd_engine_walk_stats(profit_amd_engine *engine, int32_t *overflowed, int64_t *repeats);
 int profit_amd_engine_reset_stats(profit_amd_engine *engine);
 
 #ifdef __cplusplus

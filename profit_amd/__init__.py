@@ -123,6 +123,7 @@ SYMBOLS = [
     ("profit_amd_engine_adjusted_settings", C.c_int, [C.c_void_p, _P(Profile), _P(C.c_int32), _P(C.c_int32),
                                                       _P(C.c_double), _P(C.c_double), _P(C.c_double)]),
     ("profit_amd_engine_fft_stats", C.c_int, [C.c_void_p, _P(C.c_double), _P(C.c_int64)]),
+    ("profit_amd_engine_walk_stats", C.c_int, [C.c_void_p, _P(C.c_int32), _P(C.c_int64)]),
     ("profit_amd_engine_reset_stats", C.c_int, [C.c_void_p]),
 ]
 STAGES = ("setup", "render", "subsample", "conv_like", "like_finalize", "adjoint_conv", "adjoint_render",
@@ -466,6 +467,14 @@ class Engine:
                                                          _d(rmax)))
         return dict(resolution=res[:nc], max_recursions=mr[:nc], acc=acc[:nc], rscale_switch=rsw[:nc],
                     rscale_max=rmax[:nc])
+
+    def walk_stats(self):
+        """Trees of the last evaluation that overflowed the tree walk's stack (and
+        were walked by masks), and how many evaluations had to run again because a
+        work list or a tree did not fit."""
+        n, r = C.c_int32(), C.c_int64()
+        _check(lib().profit_amd_engine_walk_stats(self._h, C.byref(n), C.byref(r)))
+        return {"overflowed": n.value, "repeats": r.value}
 
     def fft_stats(self):
         """Milliseconds per timed evaluation of each FFT kernel: forward rows,

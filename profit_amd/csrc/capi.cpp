@@ -468,6 +468,15 @@ int profit_amd_engine_fft_stats(profit_amd_engine *engine, double *kernel_ms, in
 	});
 }
 
+int profit_amd_engine_walk_stats(profit_amd_engine *engine, int32_t *overflowed, int64_t *repeats)
+{
+	return guarded([&] {
+		const profit_amd::EngineStats &s = engine->eng.stats();
+		if (overflowed) *overflowed = s.overflowed;
+		if (repeats) *repeats = s.repeats;
+	});
+}
+
 int profit_amd_engine_reset_stats(profit_amd_engine *engine)
 {
 	return guarded([&] { engine->eng.reset_stats(); });

@@ -131,14 +131,12 @@ struct WorkQueue {
 };
 constexpr int kJacStride = 12;
 // count[0]: trees that overflowed the tree walk's stack; count[1]: length of
-// the heavy list; then a (heavy, deep) pair of hand-out counters per mask walk
-// (one per profile family); the length of each family's light list, of its big
-// trees' list and of its other deep entries' list
-constexpr int kQueueCounters = 32;
-__host__ __device__ constexpr int fwd_counter(int type) { return 2 + 2 * type; }
-__host__ __device__ constexpr int light_count(int type) { return 14 + type; }
-__host__ __device__ constexpr int big_count(int type) { return 20 + type; }
-__host__ __device__ constexpr int deep_count(int type) { return 26 + type; }
+// the heavy list; then, per profile family, the length of its light list, of its
+// big trees' list and of its other deep entries' list
+__host__ __device__ constexpr int light_count(int type) { return 2 + type; }
+__host__ __device__ constexpr int big_count(int type) { return 8 + type; }
+__host__ __device__ constexpr int deep_count(int type) { return 14 + type; }
+constexpr int kQueueCounters = 20;
 
 // Where an evaluation's results go (pinned host memory); ll and grad nullable.
 struct HostReport {

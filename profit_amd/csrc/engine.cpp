@@ -763,8 +763,8 @@ WorkQueue Engine::work_queue()
 	return q;
 }
 
-// whether the last evaluation's trees fitted the tree walk's stack
-bool Engine::trees_ok() const { return h_qcount_.as<int>()[0] == 0; }
+// whether all of the last evaluation's trees were walked
+bool Engine::trees_ok() const { return mask_walk_ || h_qcount_.as<int>()[0] == 0; }
 
 // whether the last evaluation's work lists and trees fitted
 bool Engine::queue_ok() const
@@ -776,10 +776,17 @@ bool Engine::queue_ok() const
 	return q[1] <= hcap_;
 }
 
-// prepares a second run of an evaluation whose work lists or trees did not fit
-void Engine::retry_evaluation()
+// Prepares another run of an evaluation whose work lists or trees did not fit (its
+// `attempt`, from 0).  The mask walk stays on until the next batch, so that the
+// evaluations of a fit whose trees overflow run once each, from their graph.
+void Engine::retry_evaluation(int attempt)
 {
-	if (!trees_ok()) mask_walk_ = true;
+	if (attempt >= 3) throw std::runtime_error("sub-pixel work queue kept overflowing");
+	stats_.repeats += 1;
+	if (!trees_ok()) {
+		mask_walk_ = true;
+		invalidate_graphs(graph_exec_);
+	}
 	grow_queue();
 }
 
@@ -800,6 +807,7 @@ void Engine::set_batch(const std::vector<int> &inst_galaxy, const std::vector<in
 	if (inst_galaxy.size() != inst_ncomp.size()) throw std::invalid_argument("instance arrays differ in length");
 	hip_check(hipSetDevice(device_), "hipSetDevice");
 	invalidate_graphs(graph_exec_);
+	mask_walk_ = false;
 	bool any_fft = false;
 	kind_override_.resize(gal_host_.size(), -1);
 	for (size_t gi = 0; gi < gal_host_.size(); ++gi) {
@@ -1192,10 +1200,9 @@ void Engine::run(bool grad, bool use_graph)
 {
 	hip_check(hipSetDevice(device_), "hipSetDevice");
 	if (timing_) use_graph = false;  // events between kernels need the eager sequence
-	mask_walk_ = false;
-	for (int attempt = 0; attempt < 4; ++attempt) {
+	for (int attempt = 0;; ++attempt) {
 		const int gi = grad ? 1 : 0;
-		if (use_graph && !mask_walk_) {
+		if (use_graph) {
 			if (!graph_exec_[gi]) {
 				// first call runs eagerly (sets kernel attributes), later calls replay a graph
 				record(grad);
@@ -1223,6 +1230,7 @@ void Engine::run(bool grad, bool use_graph)
 			int total = q[1];
 			for (int f = 0; f < kFamilies; ++f) total += q[light_count(f)];
 			stats_.queue_count = total;
+			stats_.overflowed = q[0];
 		}
 		if (queue_ok()) {
 			if (timing_) {
@@ -1247,9 +1255,8 @@ void Engine::run(bool grad, bool use_graph)
 			stats_.evaluations += 1;
 			return;
 		}
-		retry_evaluation();
+		retry_evaluation(attempt);
 	}
-	throw std::runtime_error("sub-pixel work queue kept overflowing");
 }
 
 void Engine::evaluate(const ProfileParams *params, double *ll, double *grad, bool use_graph)
@@ -1276,7 +1283,7 @@ void Engine::diagnostics(const ProfileParams *params, int *cls, int *nodes)
 	hipStream_t st = stream_;
 	const GalaxyDev *gals = d_gals_.as<GalaxyDev>();
 	const InstDev *insts = d_insts_.as<InstDev>();
-	for (int attempt = 0; attempt < 4; ++attempt) {
+	for (int attempt = 0;; ++attempt) {
 		hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
 		                       d_err_.as<int>(), nc, d_qcount_.as<int>(), nullptr, st),
 		          "setup");
@@ -1289,7 +1296,7 @@ void Engine::diagnostics(const ProfileParams *params, int *cls, int *nodes)
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
 		if (queue_ok()) break;
-		grow_queue();
+		retry_evaluation(attempt);
 	}
 	hip_check(hipMemcpy(cls, dcls.as<int>(), plane * nc * sizeof(int), hipMemcpyDeviceToHost), "cls");
 	hip_check(hipMemcpy(nodes, dnodes.as<int>(), plane * nc * sizeof(int), hipMemcpyDeviceToHost), "nodes");
@@ -1330,8 +1337,7 @@ void Engine::model_images(const ProfileParams *params, float *out)
 	hipStream_t st = stream_;
 	const GalaxyDev *gals = d_gals_.as<GalaxyDev>();
 	const InstDev *insts = d_insts_.as<InstDev>();
-	mask_walk_ = false;
-	for (int attempt = 0; attempt < 4; ++attempt) {
+	for (int attempt = 0;; ++attempt) {
 		hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
 		                       d_err_.as<int>(), nc, d_qcount_.as<int>(), nullptr, st),
 		          "setup");
@@ -1341,8 +1347,9 @@ void Engine::model_images(const ProfileParams *params, float *out)
 		report(false, false, st);
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
+		stats_.overflowed = h_qcount_.as<int>()[0];
 		if (queue_ok()) break;
-		retry_evaluation();
+		retry_evaluation(attempt);
 	}
 	// the images leave the canvases in groups, through the two halves of a
 	// pinned buffer: while the host copies one group out, a kernel crops the
@@ -1403,8 +1410,7 @@ const float *Engine::model_canvas(const ProfileParams *params, const float **dir
 	const size_t nd = (size_t)g.DW * g.DH;
 	if (h_images_.size() < 2 * nd * sizeof(float)) h_images_.alloc(2 * nd * sizeof(float));
 	float *canvas = h_images_.as<float>(), *aux = canvas + nd;
-	mask_walk_ = false;
-	for (int attempt = 0; attempt < 4; ++attempt) {
+	for (int attempt = 0;; ++attempt) {
 		hip_check(launch_setup(h_params_.as<ProfileParams>(), d_setup_order_.as<int>(), d_comp_inst_.as<int>(), insts, gals, d_comps_.as<Comp>(),
 		                       d_err_.as<int>(), nc, d_qcount_.as<int>(), nullptr, st),
 		          "setup");
@@ -1419,8 +1425,9 @@ const float *Engine::model_canvas(const ProfileParams *params, const float **dir
 		report(false, false, st);
 		hip_check(hipStreamSynchronize(st), "sync");
 		check_setup_errors();
+		stats_.overflowed = h_qcount_.as<int>()[0];
 		if (queue_ok()) break;
-		retry_evaluation();
+		retry_evaluation(attempt);
 	}
 	*direct = beside ? aux : nullptr;
 	return canvas;

@@ -31,8 +31,8 @@ int launch_render(const GalaxyDev *gals, const InstDev *insts, const int *grp_of
 // the forward walker and the adjoint render, one launch per radial family
 // (and per sum precision in the adjoint render: 1 = FP64 per-thread sums,
 // steep cores only).  jac: the forward walk also writes each entry's Jacobian
-// (wq.ljac, wq.hjac), which launch_adj_queue weighs by G(q).  mask: the trees
-// by the mask walk (after a tree overflowed the tree walk's stack).  few: too few
+// (wq.ljac, wq.hjac), which launch_adj_queue weighs by G(q).  mask: with the mask
+// walk of the trees that overflow the tree walk's stack.  few: too few
 // big trees to fill the GPU with blocks of four wavefronts.
 int launch_subsample_fwd(int type, int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps,
                          WorkQueue wq, int split, bool jac, bool mask, bool few, hipStream_t st);
@@ -190,6 +190,10 @@ struct EngineStats {
 	long calls[ST_COUNT] = {0};
 	int queue_count = 0;
 	long evaluations = 0;
+	// trees that overflowed the tree walk's stack in the last evaluation, and the
+	// evaluations that ran again (a work list or a tree that did not fit)
+	int overflowed = 0;
+	long repeats = 0;
 	// the FFT stages kernel by kernel: [forward, adjoint][rows forward,
 	// columns, rows inverse], over the evaluations that ran FFT galaxies
 	double fft_ms[2][3] = {{0}};
@@ -338,11 +342,11 @@ class Engine {
 	unsigned radial_types_ = 0, grad_keys_ = 0;
 	int family_comps_[kFamilies] = {};  // components of each radial family
 	int few_components_ = 256;          // up to which its big trees are few
-	// trees by the mask walk: set while an evaluation runs again because a
-	// tree overflowed the tree walk's stack
+	// the mask walk follows the tree walk: from the first tree that overflowed the
+	// tree walk's stack until the next batch
 	bool mask_walk_ = false;
 	bool trees_ok() const;
-	void retry_evaluation();
+	void retry_evaluation(int attempt);
 	void launch_walkers_fwd(int split, bool jac, hipStream_t st);
 	bool sync_aux_flags(bool enable);
 	std::vector<int> ct_off_, ag_off_;

@@ -519,19 +519,16 @@ __device__ __forceinline__ void walk_pixel(const Comp &c, WalkLevel *L, int lane
 	}
 }
 
-// One wavefront per queued pixel of a TYPE component (the walk of last resort,
-// for evaluations with a tree that overflows k_subsample_tree's stack: its
-// memory is one mask per level): adds flux_scale * value to the canvas (or the
-// aux canvas, or the FP64 canvas) and, with kJac, writes the entry's Jacobian
-// and value to wq.ljac / hjac for k_adj_queue.
-// `counter`: the pair of hand-out counters of this launch (heavy, light).
+// The trees that k_subsample_tree marked because they overflow its stack, one
+// wavefront each, by the mask walk, whose memory is one mask per level: adds
+// flux_scale * value to the canvas (or the aux canvas, or the FP64 canvas) and,
+// with kJac, writes the entry's Jacobian and value to wq.ljac / hjac for
+// k_adj_queue.  Entries are dealt out by index, as there, and the marks taken back.
 // Held to the registers of four waves per SIMD (three for the Sersic, Moffat
 // and broken-exponential walks with kJac, whose code needs more).
 template <int TYPE, bool kJac>
-__global__ __launch_bounds__(256, kJac && (TYPE == SERSIC || TYPE == MOFFAT || TYPE == BROKENEXP) ? 3 : 4) void k_subsample(const GalaxyDev *__restrict__ gals,
-                                                                 const InstDev *__restrict__ insts,
-                                                                 const Comp *__restrict__ comps, WorkQueue wq,
-                                                                 int counter, int split)
+__global__ __launch_bounds__(256, kJac && (TYPE == SERSIC || TYPE == MOFFAT || TYPE == BROKENEXP) ? 3 : 4) void k_subsample_mask(
+    const GalaxyDev *__restrict__ gals, const InstDev *__restrict__ insts, const Comp *__restrict__ comps, WorkQueue wq, int split)
 {
 	__shared__ WalkLevel levels[4][kMaxLevels];
 	// the Jacobian's slots of a pixel (with kJac) and its value: per
@@ -546,39 +543,31 @@ __global__ __launch_bounds__(256, kJac && (TYPE == SERSIC || TYPE == MOFFAT || T
 	WalkLevel *L = levels[wv];
 	static_assert(TYPE >= 0 && TYPE < kFamilies, "one walker launch per profile family");
 	static_assert(kSlots < kJacStride && kSlots + 1 <= 16, "Jacobian slots and the value");
-	const int lb = wq.lbase[TYPE];
-	// the light entries the root pass left to this walker (its deep list)
-	const int nl = min(wq.count[deep_count(TYPE)], wq.lbase[TYPE + 1] - lb), nh = min(wq.count[1], wq.hcap);
+	const int lb = wq.lbase[TYPE], cap = wq.lbase[TYPE + 1] - lb;
+	const int nd = min(wq.count[deep_count(TYPE)], cap), nb = min(wq.count[big_count(TYPE)], cap);
+	const int nh = TYPE == SERSIC ? min(wq.count[1], wq.hcap) : 0;
 	// per-lane Jacobian sums
 	float gj[NGRAD];
 #pragma unroll
 	for (int s = 0; s < NGRAD; ++s) gj[s] = 0.f;
-	// dynamic hand-out, one entry at a time: the centre-pixel trees first,
-	// then the light entries the root pass left (each a tree of several
-	// nodes), so that no wavefront is left with a long tail
-	bool heavy_left = nh > 0;
-	for (;;) {
-		bool heavy = false;
-		int h = nh;
-		if (heavy_left) {
-			if (lane == 0) h = atomicAdd(&wq.count[counter], 1);
-			h = __builtin_amdgcn_readfirstlane(h);
-		}
-		int e;  // the entry's index in its list (heavy, or the family's light list)
-		if (h < nh) {
-			e = h;
-			heavy = true;
+	for (int t = blockIdx.x * 4 + wv; t < nh + nb + nd; t += gridDim.x * 4) {
+		const bool heavy = t < nh;
+		int e = t;  // the entry's index in its list (heavy, or the family's light list)
+		QEntry q;
+		if (heavy) {
+			q = wq.heavy[e];
+			if (q.pix >= 0) continue;
+			q.pix = ~q.pix;
+			__builtin_amdgcn_wave_barrier();  // every lane has read the mark
+			if (lane == 0) wq.heavy[e].pix = q.pix;
 		}
 		else {
-			heavy_left = false;
-			int l = 0;
-			if (lane == 0) l = atomicAdd(&wq.count[counter + 1], 1);
-			l = __builtin_amdgcn_readfirstlane(l);
-			if (l >= nl) break;
-			e = wq.deep[lb + l];
+			e = wq.deep[lb + (t < nh + nb ? cap - 1 - (t - nh) : t - nh - nb)];
+			if (e >= 0) continue;
+			e = ~e;
+			q = wq.light[lb + e];
 		}
 		{
-			const QEntry q = heavy ? wq.heavy[e] : wq.light[lb + e];
 			const Comp &c = comps[q.comp];
 			if (c.type != TYPE) continue;
 			const InstDev &I = insts[c.instance];
@@ -656,8 +645,8 @@ __global__ __launch_bounds__(256, kJac && (TYPE == SERSIC || TYPE == MOFFAT || T
 // is to be refined (most pixels: 98% on a 400x400 bulge+disk) the group adds
 // the value to the canvas and, with kJac, writes the entry's Jacobian and
 // value.  An entry with a cell to refine goes to the family's deep list: to its
-// front, or, with `split_big` and from kBigTree refined cells or 64 cells a node
-// on, to its back; k_subsample_tree walks those trees from the root, the front's
+// front, or, from kBigTree refined cells or 64 cells a node on, to its back;
+// k_subsample_tree walks those trees from the root, the front's
 // with a wavefront each.
 //
 // Bound by VALU issue on long lists and by latency on short ones, so the group
@@ -674,8 +663,7 @@ constexpr int kBigTree = 8;
 template <int TYPE, bool kJac>
 __global__ __launch_bounds__(256) void k_subsample_root(const GalaxyDev *__restrict__ gals,
                                                          const InstDev *__restrict__ insts,
-                                                         const Comp *__restrict__ comps, WorkQueue wq, int split,
-                                                         int split_big)
+                                                         const Comp *__restrict__ comps, WorkQueue wq, int split)
 {
 	constexpr int kSlots = G_S0 + n_shape(TYPE);
 	const int lane = threadIdx.x & 63;
@@ -747,7 +735,7 @@ __global__ __launch_bounds__(256) void k_subsample_root(const GalaxyDev *__restr
 			}
 		}
 		// the deep entries appended, one atomic per wavefront and list
-		const bool big = lead && split_big && nref > 0 && (wide || nref >= kBigTree), deep = lead && nref > 0 && !big;
+		const bool big = lead && nref > 0 && (wide || nref >= kBigTree), deep = lead && nref > 0 && !big;
 #pragma unroll
 		for (int k = 0; k < 2; ++k) {
 			const unsigned long long m = __ballot(k ? big : deep);
@@ -876,8 +864,9 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack<W> &S, int ba
 // (the back of the deep list), a block each; then the other deep entries, a wavefront each.  Adds flux_scale
 // * value to the canvas (or the aux canvas, or the FP64 canvas) and, with kJac,
 // writes the entry's Jacobian and value.  Entries are dealt out by index; an
-// overflowing tree is counted in count[0] and the evaluation runs again with
-// the mask walk (k_subsample), whose memory does not depend on the tree.
+// overflowing tree is counted in count[0] and, with `mark`, its entry is marked for
+// the mask walk that follows (k_subsample_mask): the pixel of a heavy entry, the index
+// of a deep one, bitwise inverted.  Without it the evaluation has to be run again.
 //
 // A centre tree (res 8, depth 10: 160 nodes, 16 a level) is a chain of levels:
 // one wavefront walking its nodes in turn took 220 to 300 us, whatever the
@@ -888,7 +877,8 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack<W> &S, int ba
 template <int TYPE, bool kJac, int W>
 __global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *__restrict__ gals,
                                                            const InstDev *__restrict__ insts,
-                                                           const Comp *__restrict__ comps, WorkQueue wq, int split)
+                                                           const Comp *__restrict__ comps, WorkQueue wq, int split,
+                                                           int mark)
 {
 	constexpr int kSlots = G_S0 + n_shape(TYPE), kJacPitch = 68;
 	__shared__ __align__(16) TreeStack<W> S;
@@ -968,6 +958,8 @@ __global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *_
 		}
 		else if (threadIdx.x == 0) {
 			atomicAdd(&wq.count[0], 1);
+			if (mark && heavy) wq.heavy[e].pix = ~q.pix;
+			else if (mark) wq.deep[lb + cap - 1 - (t - nh)] = ~e;
 		}
 		__syncthreads();
 		if (ok && wv == 0) {
@@ -991,8 +983,10 @@ __global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *_
 		if (walk_tree<TYPE, kJac, 64>(c, S, wv * kTreeShare, lane, x - hx, x + hx, y - hy, y + hy, c.res, c.maxrec,
 		                              g.render_fp64 != 0, sum, gj))
 			finish(q, c, I, g, false, e, wave_totals());
-		else if (lane == 0)
+		else if (lane == 0) {
 			atomicAdd(&wq.count[0], 1);
+			if (mark) wq.deep[lb + t] = ~e;
+		}
 	}
 }
 

@@ -1,13 +1,13 @@
 // Forward recursion walk (libprofit's subsample_pixel, radial.cpp:54-134): a
-// root pass, the tree walk and the mask walk, one kernel each per radial
-// profile family; see kernel_common.h.
+// root pass, the tree walk and (for trees that overflow it) the mask walk, one
+// kernel each per radial profile family; see kernel_common.h.
 #include "kernel_common.h"
 
 namespace profit_amd {
 
 // The root pass over the light entries, then the tree walk over the heavy list
-// and the entries the root pass left to it (mask: the mask walk instead, one
-// wavefront per tree).  `few`: the family's big trees (four centre pixels a
+// and the entries the root pass left to it (mask: then the mask walk over the
+// trees that overflowed it).  `few`: the family's big trees (four centre pixels a
 // component, or the like) do not fill the GPU, so the tree walk takes blocks of
 // twelve wavefronts, one a CU, and otherwise blocks of four, three a CU.  Four and
 // twelve, measured: 384 survey galaxies (about 150 components a family), Sersic
@@ -17,10 +17,10 @@ template <int TYPE, bool kJac>
 static int fwd_launch(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps, WorkQueue wq,
                       int split, bool mask, bool few, hipStream_t st)
 {
-	k_subsample_root<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, split, mask ? 0 : 1);
-	if (mask) k_subsample<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, fwd_counter(TYPE), split);
-	else if (few) k_subsample_tree<TYPE, kJac, 12><<<(nblocks + 7) / 8, 768, 0, st>>>(gals, insts, comps, wq, split);
-	else k_subsample_tree<TYPE, kJac, 4><<<(nblocks * 3 + 7) / 8, 256, 0, st>>>(gals, insts, comps, wq, split);
+	k_subsample_root<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, split);
+	if (few) k_subsample_tree<TYPE, kJac, 12><<<(nblocks + 7) / 8, 768, 0, st>>>(gals, insts, comps, wq, split, mask);
+	else k_subsample_tree<TYPE, kJac, 4><<<(nblocks * 3 + 7) / 8, 256, 0, st>>>(gals, insts, comps, wq, split, mask);
+	if (mask) k_subsample_mask<TYPE, kJac><<<nblocks, 256, 0, st>>>(gals, insts, comps, wq, split);
 	return (int)hipGetLastError();
 }
 
