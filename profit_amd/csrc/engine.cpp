@@ -1144,7 +1144,7 @@ bool Engine::sync_aux_flags(bool enable)
 	bool any = false, changed = false;
 	unsigned types = 0, keys = 0;
 	int family[kFamilies] = {};
-	unsigned depth = 0;
+	unsigned depth[kFamilies] = {};
 	for (int i = 0; i < ninst(); ++i) {
 		int aux = 0;
 		for (int k = 0; k < inst_ncomp_[i]; ++k) {
@@ -1152,7 +1152,7 @@ bool Engine::sync_aux_flags(bool enable)
 			if (is_radial(q.type)) {
 				types |= 1u << q.type;
 				++family[q.type];
-				depth = std::max(depth, q.max_recursions);
+				depth[q.type] = std::max(depth[q.type], q.max_recursions);
 				keys |= 1u << (2 * q.type + (wants_grad64(q) ? 1 : 0));
 				continue;
 			}
@@ -1167,16 +1167,20 @@ bool Engine::sync_aux_flags(bool enable)
 			changed = true;
 		}
 	}
-	// big trees do not fill the GPU with blocks of four wavefronts (see
-	// launch_subsample_fwd): up to 256 components of a family, or 1,024 whose
-	// ordinary pixels' trees are deep as well (512 components of two recursions:
-	// 0.17 ms with blocks of four, 0.20 with blocks of twelve; 500 of four: 0.69 and 0.47 ms)
-	const int few = depth > 2 ? 1024 : 256;
-	if (few != few_components_) invalidate_graphs(graph_exec_);
-	few_components_ = few;
-	if (any != any_nonradial_ || types != radial_types_ || keys != grad_keys_ ||
-	    std::memcmp(family, family_comps_, sizeof(family)) != 0) {
-		std::memcpy(family_comps_, family, sizeof(family));
+	// Up to how many components a family's big trees do not fill the GPU with blocks of
+	// four wavefronts (see launch_subsample_fwd).  Time of the sub-sample stage with
+	// blocks of four over that with twelve, 64 / 256 / 1,024 / 2,048 components of 100x100
+	// images: King 1.9 / 1.1 / 1.1 / 1.1, core-Sersic 1.8 / 1.4 / 1.2 / 1.1, Moffat
+	// - / 1.3 / 1.05 / 1.03 (0.95 at 4,096), Ferrer 1.0, broken exponential 1.1 at 128 and
+	// 0.9 / 0.8 / 0.85 from 256, whatever the recursion depth; Sersic 1.5 / 1.1 / 0.93 /
+	// 0.88, 1.03 to 1.07 at 512, where 256 bulges and disks take 0.83 and 500 sources of
+	// four recursions 1.47.
+	const int limit[kFamilies] = {depth[SERSIC] > 2 ? 512 : 256, 2048, 2048, 2048, 2048, 128};
+	unsigned few = 0;
+	for (int t = 0; t < kFamilies; ++t)
+		if (family[t] <= limit[t]) few |= 1u << t;
+	if (any != any_nonradial_ || types != radial_types_ || keys != grad_keys_ || few != few_trees_) {
+		few_trees_ = few;
 		any_nonradial_ = any;
 		radial_types_ = types;
 		grad_keys_ = keys;
@@ -1192,7 +1196,7 @@ void Engine::launch_walkers_fwd(int split, bool jac, hipStream_t st)
 	for (int t = 0; t < 6; ++t)
 		if ((radial_types_ >> t) & 1u)
 			hip_check(launch_subsample_fwd(t, subsample_blocks_, d_gals_.as<GalaxyDev>(), d_insts_.as<InstDev>(),
-			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, family_comps_[t] <= few_components_, st),
+			                               d_comps_.as<Comp>(), work_queue(), split, jac, mask_walk_, (few_trees_ >> t) & 1u, st),
 			          "subsample");
 }
 

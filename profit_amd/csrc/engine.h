@@ -340,8 +340,7 @@ class Engine {
 	// radial families present (bit t) and the adjoint's (family, precision)
 	// keys present (bit 2t + prec), which decide the walker launches
 	unsigned radial_types_ = 0, grad_keys_ = 0;
-	int family_comps_[kFamilies] = {};  // components of each radial family
-	int few_components_ = 256;          // up to which its big trees are few
+	unsigned few_trees_ = 0;  // families with few big trees (bit t), see sync_aux_flags
 	// the mask walk follows the tree walk: from the first tree that overflowed the
 	// tree walk's stack until the next batch
 	bool mask_walk_ = false;
