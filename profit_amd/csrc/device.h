@@ -132,11 +132,13 @@ struct WorkQueue {
 constexpr int kJacStride = 12;
 // count[0]: trees that overflowed the tree walk's stack; count[1]: length of
 // the heavy list; then, per profile family, the length of its light list, of its
-// big trees' list and of its other deep entries' list
+// big trees' list and of its other deep entries' list, and the hand-out counter of
+// its big trees
 __host__ __device__ constexpr int light_count(int type) { return 2 + type; }
 __host__ __device__ constexpr int big_count(int type) { return 8 + type; }
 __host__ __device__ constexpr int deep_count(int type) { return 14 + type; }
-constexpr int kQueueCounters = 20;
+__host__ __device__ constexpr int tree_count(int type) { return 20 + type; }
+constexpr int kQueueCounters = 26;
 
 // Where an evaluation's results go (pinned host memory); ll and grad nullable.
 struct HostReport {

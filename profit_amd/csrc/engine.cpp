@@ -1169,13 +1169,14 @@ bool Engine::sync_aux_flags(bool enable)
 	}
 	// Up to how many components a family's big trees do not fill the GPU with blocks of
 	// four wavefronts (see launch_subsample_fwd).  Time of the sub-sample stage with
-	// blocks of four over that with twelve, 64 / 256 / 1,024 / 2,048 components of 100x100
-	// images: King 1.9 / 1.1 / 1.1 / 1.1, core-Sersic 1.8 / 1.4 / 1.2 / 1.1, Moffat
-	// - / 1.3 / 1.05 / 1.03 (0.95 at 4,096), Ferrer 1.0, broken exponential 1.1 at 128 and
-	// 0.9 / 0.8 / 0.85 from 256, whatever the recursion depth; Sersic 1.5 / 1.1 / 0.93 /
-	// 0.88, 1.03 to 1.07 at 512, where 256 bulges and disks take 0.83 and 500 sources of
-	// four recursions 1.47.
-	const int limit[kFamilies] = {depth[SERSIC] > 2 ? 512 : 256, 2048, 2048, 2048, 2048, 128};
+	// blocks of four over that with twelve, 64 / 256 / 1,024 / 2,048 / 4,096 components of
+	// every size on 100x100 images: King 1.5 / 1.2 / 0.91 / 0.86 / 0.81 (1.5 at 512), core-
+	// Sersic 1.9 / 1.5 / 1.3 / 1.1 / 1.0, Moffat 1.1 / 1.0 / 1.3 / 1.1 / 1.0, Ferrer 1.0,
+	// broken exponential 1.2 / 1.0 / 0.8 / 0.74 / 0.71.  Sersic 1.4 / 1.5 / 1.2 / 1.1 / 0.94
+	// and the same with four recursions, but the chains of one galaxy, whose trees are
+	// alike, lose: 256 bulges and disks 0.97, 512 disks 0.98, 1,024 bulges and disks 0.97;
+	// 48 bulges and disks 1.09, 500 field sources of four recursions 1.04 (whole calls).
+	const int limit[kFamilies] = {depth[SERSIC] > 2 ? 512 : 256, 2048, 2048, 512, 2048, 256};
 	unsigned few = 0;
 	for (int t = 0; t < kFamilies; ++t)
 		if (family[t] <= limit[t]) few |= 1u << t;

@@ -1,10 +1,10 @@
 // Device code shared by the kernel translation units: block ownership,
 // wave reductions, libprofit's cell positions and refinement test, and the
-// templates of the recursion walker and of the adjoint render.
-// walkers_fwd.hip compiles the forward walker once per profile family and
-// walkers_adj.hip the adjoint walker once per family and the adjoint render
+// templates of the sub-pixel walks and of the adjoint kernels.
+// walkers_fwd.hip compiles the forward walks once per profile family and
+// walkers_adj.hip the sub-pixel adjoint once per family and the adjoint render
 // once per family and sum precision: a kernel's register allocation is the
-// maximum over the code it holds, so one family per kernel lifts the walkers
+// maximum over the code it holds, so one family per kernel lifts the walks
 // from two to three or four waves per SIMD and the adjoint render from two
 // to seven or eight.
 #pragma once
@@ -863,8 +863,10 @@ __device__ __forceinline__ bool walk_tree(const Comp &c, TreeStack<W> &S, int ba
 // entries with kBigTree or more refined root cells or more than 64 cells a node
 // (the back of the deep list), a block each; then the other deep entries, a wavefront each.  Adds flux_scale
 // * value to the canvas (or the aux canvas, or the FP64 canvas) and, with kJac,
-// writes the entry's Jacobian and value.  Entries are dealt out by index; an
-// overflowing tree is counted in count[0] and, with `mark`, its entry is marked for
+// writes the entry's Jacobian and value.  A block takes its first big tree by index and
+// the next ones from a counter, asked for while it walks (the trees differ by a factor
+// of hundreds: King trees of 4,096 survey galaxies 5.7 ms by index, 4.4 so, core-Sersic
+// 3.1 and 2.0); small trees are dealt out by index.  An overflowing tree is counted in count[0] and, with `mark`, its entry is marked for
 // the mask walk that follows (k_subsample_mask): the pixel of a heavy entry, the index
 // of a deep one, bitwise inverted.  Without it the evaluation has to be run again.
 //
@@ -883,6 +885,7 @@ __global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *_
 	constexpr int kSlots = G_S0 + n_shape(TYPE), kJacPitch = 68;
 	__shared__ __align__(16) TreeStack<W> S;
 	__shared__ double red[W][16];
+	__shared__ int next;
 	static_assert(kSlots < kJacStride && kSlots + 1 <= 16, "Jacobian slots and the value");
 	static_assert(sizeof(float) * kSlots * kJacPitch <= sizeof(typename TreeStack<W>::Share), "a wavefront's rows fit its share");
 	static_assert(sizeof(typename TreeStack<W>::Share) % 16 == 0, "a wavefront's rows are 16-byte aligned");
@@ -937,12 +940,12 @@ __global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *_
 #pragma unroll
 		for (int s = 0; s < NGRAD; ++s) gj[s] = 0.f;
 	};
-	for (int t = blockIdx.x; t < nh + nb; t += gridDim.x) {
+	for (int t = blockIdx.x; t < nh + nb;) {
+		if (threadIdx.x == 0) next = gridDim.x + atomicAdd(&wq.count[tree_count(TYPE)], 1);
 		const bool heavy = t < nh;
 		const int e = heavy ? t : wq.deep[lb + cap - 1 - (t - nh)];
 		const QEntry q = heavy ? wq.heavy[e] : wq.light[lb + e];
 		const Comp &c = comps[q.comp];
-		if (c.type != TYPE) continue;
 		const InstDev &I = insts[c.instance];
 		const GalaxyDev &g = gals[I.galaxy];
 		const int i = q.pix % g.DW, j = q.pix / g.DW;
@@ -962,6 +965,7 @@ __global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *_
 			else if (mark) wq.deep[lb + cap - 1 - (t - nh)] = ~e;
 		}
 		__syncthreads();
+		const int then = next;
 		if (ok && wv == 0) {
 			double v = 0;
 #pragma unroll
@@ -969,6 +973,7 @@ __global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *_
 			finish(q, c, I, g, heavy, e, v);
 		}
 		__syncthreads();
+		t = then;
 	}
 	for (int t = blockIdx.x * W + wv; t < nd; t += gridDim.x * W) {
 		const int e = wq.deep[lb + t];
@@ -991,7 +996,7 @@ __global__ __launch_bounds__(64 * W, 3) void k_subsample_tree(const GalaxyDev *_
 }
 
 // The adjoint of the sub-sampled pixels from their Jacobians (written by the
-// forward walk, k_subsample<TYPE, true>): per entry (component c,
+// forward walk's three kernels with kJac): per entry (component c,
 // pixel q), G(q) fs (J_s + dlnfs_s V) for every slot s.  Lanes take
 // consecutive entries of the family's lists (the heavy list first, Sersic
 // only); the lanes of one component are summed across the wave, one
