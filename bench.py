@@ -433,7 +433,7 @@ def main():
 
     # per-kernel rooflines (one launch = the whole batch); algorithmic work per
     # unit of each kernel family:
-    #   rendering (k_render, the recursion walkers, the adjoint render): 5 B per
+    #   rendering (k_render, the sub-pixel walks, the adjoint render): 5 B per
     #     canvas pixel (4 B FP32 write + 1 B mask read), reported against HBM;
     #     their limit is the VALU / transcendental rate, so profile
     #     evaluations per second are given beside it
@@ -445,8 +445,9 @@ def main():
     geom = eng.geometry(g)
     dw, dh, _, _ = geom
     K = wl["psf"].shape[0]
-    n1 = max(8, 1 << int(np.ceil(np.log2(dw + K))))
-    n2 = max(8, 1 << int(np.ceil(np.log2(dh + K))))
+    # the frame of a padded canvas leaves no room for the kernel beside it
+    n1 = max(8, 1 << int(np.ceil(np.log2(dw if dw > 400 else dw + K))))
+    n2 = max(8, 1 << int(np.ceil(np.log2(dh if dh > 400 else dh + K))))
     render_bytes = B * dw * dh * 5.0
     direct, cells, queued = sample_counts(eng1, gpu_params(P, [wl["components"]]), geom, wl["components"])
     traffic = {}
@@ -474,8 +475,9 @@ def main():
                 "direct_pixels_per_instance": direct})
     # the forward walk of a gradient evaluation: cell values, refinement tests
     # and each cell's derivatives into the pixel's Jacobian
-    add_kernel("subsample", "k_subsample_root<0, true> + k_subsample<0, true>", stage_ms["subsample"], "hbm",
-               render_bytes, PEAK_HBM_GBS,
+    # (blocks of twelve wavefronts up to 256 components, of four beyond)
+    add_kernel("subsample", f"k_subsample_root<0, true> + k_subsample_tree<0, true, {12 if 2 * B <= 256 else 4}>",
+               stage_ms["subsample"], "hbm", render_bytes, PEAK_HBM_GBS,
                "GB/s", {"cell_value_and_derivative_evals_per_s": round(B * cells / (stage_ms["subsample"] * 1e-3), 0),
                         "cells_per_instance": cells})
     add_kernel("adjoint_render", "k_adj_render<0, *>", stage_ms["adjoint_render"], "hbm", render_bytes, PEAK_HBM_GBS,

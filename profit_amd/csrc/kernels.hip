@@ -4,10 +4,13 @@
 //   k_render         pixel classification (FP64, bit-exact with libprofit) and
 //                    direct FP32 evaluation (radial.cpp:291-344); pixels that need
 //                    sub-pixel integration are appended to a work queue
-//   k_subsample      one wavefront per queued pixel walks libprofit's adaptive
-//                    recursion (radial.cpp:54-134) depth-first, FP32 cell positions
-//                    and tests with FP64 re-tests in a guard band; the walk keeps
-//                    one node and a 256-bit "cells to refine" mask per level
+//   k_subsample_root / k_subsample_tree / k_subsample_mask
+//                    libprofit's adaptive recursion (radial.cpp:54-134) of the queued
+//                    pixels, FP32 cell positions and tests with FP64 re-tests in a
+//                    guard band: the root cells by groups of lanes, then each tree by a
+//                    block or a wavefront with its pending nodes on an LDS stack, and
+//                    the trees that overflow it by a wavefront with a 256-bit mask of
+//                    cells per level (kernel_common.h, walkers_fwd.hip)
 //   k_conv           LDS-tiled brute-force convolution (convolve.cpp:158-231) with
 //                    three epilogues: fused masked likelihood, model image, and
 //                    the adjoint correlation

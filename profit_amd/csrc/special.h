@@ -107,9 +107,9 @@ PA_HD double qgamma_upper(double x, double a, double lga)
 
 // Quantile of the unit-scale gamma distribution: Halley steps kept inside a
 // bracket.  The steps converge cubically, so a step below 1e-6 x leaves an
-// error below the rounding of x and is the last: two or three evaluations of P
-// or Q (one for the median of a >= 3), where iterating until the step itself
-// vanished took seven to thirty.  They are what bounds a Sersic component's
+// error below the rounding of x and is the last: one or two evaluations of P or Q for
+// the median of a >= 1, two or three for the set-up's other quantiles (three to eight
+// where a < 1), where iterating until the step itself vanished took seven to thirty.  They are what bounds a Sersic component's
 // set-up (2048 of them: 131 -> 64 us; one image's: 45 -> 38 us).
 PA_HD double qgamma(double p, double a)
 {
