@@ -9,10 +9,9 @@ namespace profit_amd {
 // and the entries the root pass left to it (mask: then the mask walk over the
 // trees that overflowed it).  `few`: the family's big trees (four centre pixels a
 // component, or the like) do not fill the GPU, so the tree walk takes blocks of
-// twelve wavefronts, one a CU, and otherwise blocks of four, three a CU.  Four and
-// twelve, measured: 384 survey galaxies (about 150 components a family), Sersic
-// 336 and 188 us, King 740 and 711, core-Sersic 1354 and 701; one bulge+disk
-// image 53 and 30.
+// twelve wavefronts, one a CU, and otherwise blocks of four, three a CU (one
+// bulge+disk image: 53 us with four, 30 with twelve; both shapes by family and
+// count: Engine::sync_aux_flags).
 template <int TYPE, bool kJac>
 static int fwd_launch(int nblocks, const GalaxyDev *gals, const InstDev *insts, const Comp *comps, WorkQueue wq,
                       int split, bool mask, bool few, hipStream_t st)
